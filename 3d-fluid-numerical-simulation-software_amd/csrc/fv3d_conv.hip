@@ -75,7 +75,7 @@ __device__ inline void stream_face(const BlockDev &B, const Gas &g, int d, int i
     const long xd = d == 0 ? cidx(B, i, j + 1, k + 1) : d == 1 ? cidx(B, i + 1, j, k + 1) : cidx(B, i + 1, j + 1, k);
     double fcx = 0.0, fcy = 0.0;
     if (B.w_rot != 0.0) { fcx = B.fc[d][xf]; fcy = B.fc[d][box + xf]; }
-    face_core(g, st, wF, wB, B.fS[d][xf], B.fS[d][box + xf], B.fS[d][2 * box + xf], B.fs[d][xf], fcx, fcy, B.w_rot,
+    face_core<MODE>(g, st, wF, wB, B.fS[d][xf], B.fS[d][box + xf], B.fS[d][2 * box + xf], B.fs[d][xf], fcx, fcy, B.w_rot,
               B.node[xd] - B.node[xf], B.node[box + xd] - B.node[box + xf], B.node[2 * box + xd] - B.node[2 * box + xf],
               out);
 }

@@ -1644,11 +1644,16 @@ static int launch_restriction_timestep(fv3d_ctx *c)
 
 static int launch_convective(fv3d_ctx *c)
 {
+    // the reconstruction's variables (any code other than 100 and 200 is
+    // characteristic, source/UserInput.cpp:117-130)
+    const int mode = c->cfg.recon_var == 200 ? 0 : c->cfg.recon_var == 100 ? 1 : 2;
     if (!c->store_faces && c->tile_sel[0] == kConvFaces) {
         if (!c->d_fstart) return fail(c, FV3D_ESTATE, "face-parallel convective form not built");
         const int nb = (int)c->blocks.size();
-        hipLaunchKernelGGL(k_conv_faces, dim3((unsigned)((c->nfaces + 255) / 256)), dim3(256), 0, c->stream, c->d_blocks,
-                           c->d_fstart, 3 * nb, c->gas);
+        const dim3 gf((unsigned)((c->nfaces + 255) / 256));
+        if (mode == 0) hipLaunchKernelGGL(k_conv_faces<0>, gf, dim3(256), 0, c->stream, c->d_blocks, c->d_fstart, 3 * nb, c->gas);
+        else if (mode == 1) hipLaunchKernelGGL(k_conv_faces<1>, gf, dim3(256), 0, c->stream, c->d_blocks, c->d_fstart, 3 * nb, c->gas);
+        else hipLaunchKernelGGL(k_conv_faces<2>, gf, dim3(256), 0, c->stream, c->d_blocks, c->d_fstart, 3 * nb, c->gas);
         hipLaunchKernelGGL(k_conv_sum, dim3((unsigned)((c->ncell + 255) / 256)), dim3(256), 0, c->stream, c->d_blocks,
                            c->d_cstart, nb);
         HIPCK(c, hipGetLastError());
@@ -1659,7 +1664,6 @@ static int launch_convective(fv3d_ctx *c)
         int rc = ensure_stream_tiles(c, q);
         if (rc) return rc;
         const int nt = c->nstiles[q], ci = kStreamShape[q][2];
-        const int mode = c->cfg.recon_var == 200 ? 0 : c->cfg.recon_var == 100 ? 1 : 2;
         const dim3 g((unsigned)(8 * ((nt + 7) / 8)));
         switch (q < 2 || q == 4 ? 0 : 1) {
 #define FV3D_STREAM(S, TJ, TK)                                                                                     \
@@ -1683,14 +1687,16 @@ static int launch_convective(fv3d_ctx *c)
     const int q = c->tile_sel[0] < kNumTiles ? c->tile_sel[0] : 0;
     if (!c->d_tiles_s[q]) return fail(c, FV3D_ESTATE, "convective tiles of shape %d not built", q);
     const dim3 g((unsigned)c->ntiles_s[q]), b(256);
-    switch (q) {
-#define FV3D_CONV(S, A, B, C)                                                                                    \
-    case S:                                                                                                       \
-        hipLaunchKernelGGL((k_convective<A, B, C>), g, b, 0, c->stream, c->d_blocks, c->d_tiles_s[q], c->gas,       \
+    switch (3 * q + mode) {
+#define FV3D_CONV_M(S, M, A, B, C)                                                                               \
+    case 3 * S + M:                                                                                               \
+        hipLaunchKernelGGL((k_convective<A, B, C, M>), g, b, 0, c->stream, c->d_blocks, c->d_tiles_s[q], c->gas,    \
                            c->store_faces, c->d_faces[0], c->d_faces[1], c->d_faces[2]);                         \
         break;
+#define FV3D_CONV(S, A, B, C) FV3D_CONV_M(S, 0, A, B, C) FV3D_CONV_M(S, 1, A, B, C) FV3D_CONV_M(S, 2, A, B, C)
         FV3D_FOR_TILES(FV3D_CONV)
 #undef FV3D_CONV
+#undef FV3D_CONV_M
     }
     HIPCK(c, hipGetLastError());
     return FV3D_OK;

@@ -428,6 +428,10 @@ __device__ inline void sw_half(double Gamma, const double Q[5], double que, doub
 // face vector S, its area s, the node diagonal r and the grid velocity of the
 // face centroid (fcx, fcy) times w_rot, the Roe or Steger-Warming flux, and
 // the flux rotated back and times the area.
+// MODE is the reconstruction's variables (0 primitive, 1 conservative, 2
+// characteristic), a compile-time choice so that a kernel carries one
+// reconstruction's registers; scheme and flux are run-time (wave-uniform) ones.
+template <int MODE>
 __device__ inline void face_core(const Gas &g, const double st[4][5], const double wF[6], const double wB[6],
                                  double Sx, double Sy, double Sz, double s_, double fcx, double fcy, double w_rot,
                                  double rx, double ry, double rz, double out[5])
@@ -435,13 +439,13 @@ __device__ inline void face_core(const Gas &g, const double st[4][5], const doub
     const double Gamma = g.gamma;
     const double lim_zero = F32C(1E-20);
     double L[5], R[5], cvL[5], cvR[5];
-    if (g.recon_var != 100 && g.recon_var != 200) {
+    if constexpr (MODE == 2) {
         recon_char(g.recon_scheme, Gamma, g.rgas, wF, wB, st, cvL, cvR);
         double pL = (Gamma - F32C(1.0)) * (cvL[4] - F32C(0.5) * (cvL[1] * cvL[1] + cvL[2] * cvL[2] + cvL[3] * cvL[3]) / cvL[0]);
         double pR = (Gamma - F32C(1.0)) * (cvR[4] - F32C(0.5) * (cvR[1] * cvR[1] + cvR[2] * cvR[2] + cvR[3] * cvR[3]) / cvR[0]);
         if (cvL[0] <= lim_zero || pL <= lim_zero) for (int c = 0; c < 5; ++c) cvL[c] = st[1][c];
         if (cvR[0] <= lim_zero || pR <= lim_zero) for (int c = 0; c < 5; ++c) cvR[c] = st[2][c];
-    } else if (g.recon_var == 200) {
+    } else if constexpr (MODE == 0) {
         for (int c = 0; c < 5; ++c) recon1_prim(g.recon_scheme, st[0][c], st[1][c], st[2][c], st[3][c], L[c], R[c]);
         if (L[0] <= lim_zero || L[4] <= lim_zero) for (int c = 0; c < 5; ++c) L[c] = st[1][c];
         if (R[0] <= lim_zero || R[4] <= lim_zero) for (int c = 0; c < 5; ++c) R[c] = st[2][c];

@@ -103,10 +103,12 @@ __global__ void k_exchange(const BlockDev *blocks, const ExchDev *el, long n, co
 // the CFL number of each block's instance: BlockDev::cfl
 __global__ void k_spectral_dt(const BlockDev *blocks, const long *cstart, int nblock, Gas g);
 __global__ void k_dt_flag_decrement(const BlockDev *blocks, int nblock);
-template <int TI, int TJ, int TK>
+// MODE: the reconstruction's variables, 0 primitive, 1 conservative, 2 characteristic
+template <int TI, int TJ, int TK, int MODE>
 __global__ void k_convective(const BlockDev *blocks, const int4 *tiles, Gas g, int store_faces, double *fI, double *fJ,
                              double *fK);
 // fstart: running face counts per (block, direction), 3 * nblock entries + 1
+template <int MODE>
 __global__ void k_conv_faces(const BlockDev *blocks, const long *fstart, int nlist, Gas g);
 __global__ void k_conv_sum(const BlockDev *blocks, const long *cstart, int nblock);
 template <bool FORWARD>

@@ -377,6 +377,7 @@ __global__ void k_dt_flag_decrement(const BlockDev *__restrict__ blocks, int nbl
 // =================================================== convective residual
 // Face flux of CSpaceDiscr::Upwind_Convective (source/Upwind_Convective.cpp:5-360)
 // with the WallFlux override (source/WallFlux.cpp:70-175).
+template <int MODE>
 __device__ static void face_flux(const BlockDev &B, const Gas &g, int d, int i, int j, int k, double out[5])
 {
     const long box = B.box;
@@ -400,7 +401,7 @@ __device__ static void face_flux(const BlockDev &B, const Gas &g, int d, int i, 
     // layers.  Characteristic reconstruction (any variable code other than
     // 100 and 200, source/UserInput.cpp:117-130) takes the conservative
     // stencil and the primitive variables of F and B.
-    const bool prim = g.recon_var == 200, chr = g.recon_var != 100 && g.recon_var != 200;
+    constexpr bool prim = MODE == 0, chr = MODE == 2;
     double st[4][5], wFB[2][6];
     const long dstride = d == 0 ? B.si : d == 1 ? B.sj : 1;
     const double *src = prim ? B.W : B.Q;
@@ -425,7 +426,7 @@ __device__ static void face_flux(const BlockDev &B, const Gas &g, int d, int i, 
     // a non-rotating block skips the face centroid (its grid velocity is zero)
     double fcx = 0.0, fcy = 0.0;
     if (B.w_rot != 0.0) { fcx = B.fc[d][xf]; fcy = B.fc[d][box + xf]; }
-    face_core(g, st, wFB[0], wFB[1], B.fS[d][xf], B.fS[d][box + xf], B.fS[d][2 * box + xf], B.fs[d][xf], fcx, fcy,
+    face_core<MODE>(g, st, wFB[0], wFB[1], B.fS[d][xf], B.fS[d][box + xf], B.fS[d][2 * box + xf], B.fs[d][xf], fcx, fcy,
               B.w_rot, B.node[xd] - B.node[xf], B.node[box + xd] - B.node[box + xf],
               B.node[2 * box + xd] - B.node[2 * box + xf], out);
 }
@@ -434,12 +435,25 @@ __device__ static void face_flux(const BlockDev &B, const Gas &g, int d, int i, 
 // once into LDS, then each cell sums its six faces and subtracts the rotation
 // source (source/ComputeAllBlockVars.cpp:85-118, 237-254).  Optionally stores
 // the face fluxes for inspection.
-// Three waves per SIMD: the register budget (168) holds the face code with a
-// few spills, and the third wave hides more latency than the spills cost.
-template <int TI, int TJ, int TK>
-__global__ void __launch_bounds__(TI *TJ *TK) __attribute__((amdgpu_waves_per_eu(3))) k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles,
-                                                           Gas g, int store_faces, double *fI0, double *fJ0, double *fK0)
+//
+// The face code is bound by FP64 issue, so what counts is how many times a wave
+// runs it.  The tile's faces (about 3.5 per cell) are handed out 64 at a time,
+// each group of one direction (so the direction and every array it selects is
+// wave-uniform): 15 or 16 groups for every shape, at most four per wave.  With
+// the faces handed out by cell (each thread its three low faces, the threads on
+// the tile's upper edges the high ones) a wave ran the code six times, the last
+// three with an eighth to a half of its lanes: 651 -> 494 us on a 2.54M-cell
+// passage (4x4x16), 260 -> 201 us on a 1.05M-cell channel.  With one
+// reconstruction per kernel the face code fits 128 registers and four waves per
+// SIMD: 494 -> 467 us, 201 -> 188 us (the characteristic one needs 166 and
+// keeps three).
+template <int TI, int TJ, int TK, int MODE>
+__global__ void __launch_bounds__(TI *TJ *TK) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 3 : 4)))
+k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles, Gas g, int store_faces, double *fI0,
+             double *fJ0, double *fK0)
 {
+    constexpr int NFI = (TI + 1) * TJ * TK, NFJ = TI * (TJ + 1) * TK, NFK = TI * TJ * (TK + 1);
+    constexpr int GI = (NFI + 63) / 64, GJ = (NFJ + 63) / 64, GK = (NFK + 63) / 64;   // groups per direction
     __shared__ double sI[5][TI + 1][TJ][TK];
     __shared__ double sJ[5][TI][TJ + 1][TK];
     __shared__ double sK[5][TI][TJ][TK + 1];
@@ -447,32 +461,30 @@ __global__ void __launch_bounds__(TI *TJ *TK) __attribute__((amdgpu_waves_per_eu
     if (tl.x < 0) return;   // padding of the XCD-ordered tile list
     const BlockDev &B = blocks[tl.x];
     const int t = threadIdx.x;
-    const int tk = t % TK, tj = (t / TK) % TJ, ti = t / (TK * TJ);
-    const int i = tl.y + ti + 1, j = tl.z + tj + 1, k = tl.w + tk + 1;
-    const bool valid = i <= B.ni && j <= B.nj && k <= B.nk;
-    double f[5];
-    if (valid) {
-        // the cell's three low faces, then the high faces on the tile's upper
-        // edges, all through one copy of the face code: the loop stays rolled
-        // because six inlined copies of it (every scheme and reconstruction)
-        // would not fit the instruction cache
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+    // one copy of the face code in a rolled loop: a copy per direction (every
+    // scheme and both fluxes) would crowd the instruction cache
 #pragma nounroll
-        for (int e = 0; e < 6; ++e) {
-            const int d = e < 3 ? e : e - 3, hi = e < 3 ? 0 : 1;
-            if (hi && !(d == 0 ? (ti == TI - 1 || i == B.ni) : d == 1 ? (tj == TJ - 1 || j == B.nj)
-                                                                    : (tk == TK - 1 || k == B.nk)))
-                continue;
-            face_flux(B, g, d, i + (d == 0 ? hi : 0), j + (d == 1 ? hi : 0), k + (d == 2 ? hi : 0), f);
-            if (d == 0)
-                for (int c = 0; c < 5; ++c) sI[c][ti + hi][tj][tk] = f[c];
-            else if (d == 1)
-                for (int c = 0; c < 5; ++c) sJ[c][ti][tj + hi][tk] = f[c];
-            else
-                for (int c = 0; c < 5; ++c) sK[c][ti][tj][tk + hi] = f[c];
-        }
+    for (int q = wave; q < GI + GJ + GK; q += TI * TJ * TK / 64) {
+        const int d = q < GI ? 0 : q < GI + GJ ? 1 : 2;
+        const int f = (q - (d == 0 ? 0 : d == 1 ? GI : GI + GJ)) * 64 + lane;   // face number within its direction
+        // place in the tile; the divisors are constants in each branch
+        int a, b, c;
+        if (d == 0) { c = f % TK; b = f / TK % TJ; a = f / (TK * TJ); }
+        else if (d == 1) { c = f % TK; b = f / TK % (TJ + 1); a = f / (TK * (TJ + 1)); }
+        else { c = f % (TK + 1); b = f / (TK + 1) % TJ; a = f / ((TK + 1) * TJ); }
+        const int i = tl.y + a + 1, j = tl.z + b + 1, k = tl.w + c + 1;   // the face's higher cell
+        if (a >= TI + (d == 0) || i > B.ni + (d == 0) || j > B.nj + (d == 1) || k > B.nk + (d == 2)) continue;
+        double out[5];
+        face_flux<MODE>(B, g, d, i, j, k, out);
+        double *dst = (d == 0 ? &sI[0][0][0][0] : d == 1 ? &sJ[0][0][0][0] : &sK[0][0][0][0]) + f;
+        const int n = d == 0 ? NFI : d == 1 ? NFJ : NFK;
+        for (int e = 0; e < 5; ++e) dst[e * n] = out[e];
     }
     __syncthreads();
-    if (!valid) return;
+    const int tk = t % TK, tj = (t / TK) % TJ, ti = t / (TK * TJ);
+    const int i = tl.y + ti + 1, j = tl.z + tj + 1, k = tl.w + tk + 1;
+    if (i > B.ni || j > B.nj || k > B.nk) return;
     const long box = B.box, x = cidx(B, i, j, k);
     const double w_rot = B.w_rot;
     const double vol = B.vol[x];
@@ -500,15 +512,18 @@ __global__ void __launch_bounds__(TI *TJ *TK) __attribute__((amdgpu_waves_per_eu
     }
 }
 
-#define FV3D_CONV(S, A, B, C) \
-    template __global__ void k_convective<A, B, C>(const BlockDev *, const int4 *, Gas, int, double *, double *, double *);
+#define FV3D_CONV_M(M, A, B, C) \
+    template __global__ void k_convective<A, B, C, M>(const BlockDev *, const int4 *, Gas, int, double *, double *, double *);
+#define FV3D_CONV(S, A, B, C) FV3D_CONV_M(0, A, B, C) FV3D_CONV_M(1, A, B, C) FV3D_CONV_M(2, A, B, C)
 FV3D_FOR_TILES(FV3D_CONV)
 #undef FV3D_CONV
+#undef FV3D_CONV_M
 
 // Face-parallel form of the same residual: every face of every block once, one
 // thread per face (faces of a block and direction i-slowest, k fastest), into
 // B.fcv; k_conv_sum then forms each cell's residual from its six faces and the
 // rotation source in k_convective's order, so the two forms agree bit for bit.
+template <int MODE>
 __global__ void __launch_bounds__(256) k_conv_faces(const BlockDev *__restrict__ blocks, const long *__restrict__ fstart,
                                                     int nlist, Gas g)
 {
@@ -521,10 +536,14 @@ __global__ void __launch_bounds__(256) k_conv_faces(const BlockDev *__restrict__
     const int nj = B.nj + (d == 1 ? 1 : 0), nk = B.nk + (d == 2 ? 1 : 0);
     const int i = (int)(r / ((long)nj * nk)) + 1, j = (int)(r / nk % nj) + 1, k = (int)(r % nk) + 1;
     double f[5];
-    face_flux(B, g, d, i, j, k, f);
+    face_flux<MODE>(B, g, d, i, j, k, f);
     const long x = cidx(B, i, j, k);
     for (int c = 0; c < 5; ++c) B.fcv[(long)(d * 5 + c) * B.box + x] = f[c];
 }
+
+template __global__ void k_conv_faces<0>(const BlockDev *, const long *, int, Gas);
+template __global__ void k_conv_faces<1>(const BlockDev *, const long *, int, Gas);
+template __global__ void k_conv_faces<2>(const BlockDev *, const long *, int, Gas);
 
 __global__ void __launch_bounds__(256) k_conv_sum(const BlockDev *__restrict__ blocks, const long *__restrict__ cstart,
                                                   int nblock)
