@@ -26,7 +26,7 @@ namespace fv3d {
 // MODE 0: primitive rho u v w p (W); 1: conservative (Q); 2: characteristic
 // reconstruction, Q (c < 5) then the primitive rho u v w p (c >= 5).
 template <int MODE>
-__device__ inline double stencil_val(const BlockDev &B, int i, int j, int k, int c)
+__device__ inline double stencil_val(BlockRef B, int i, int j, int k, int c)
 {
     const bool fromW = MODE == 0 || (MODE == 2 && c >= 5);
     const int cc = (MODE == 2 && c >= 5) ? c - 5 : c;
@@ -48,7 +48,7 @@ __device__ inline double stencil_val(const BlockDev &B, int i, int j, int k, int
 // Face (i, j, k) of direction d from its stencil (NV variables of the four
 // cells), with the wall override on wall faces of the block boundary.
 template <int MODE, int NV>
-__device__ inline void stream_face(const BlockDev &B, const Gas &g, int d, int i, int j, int k, const double v0[NV],
+__device__ inline void stream_face(BlockRef B, const Gas &g, int d, int i, int j, int k, const double v0[NV],
                                    const double v1[NV], const double v2[NV], const double v3[NV], double out[5])
 {
     const long box = B.box;
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(TJ *TK) k_conv_stream(const BlockDev *__restri
     const int tix = (int)(blockIdx.x & 7) * nper + (int)(blockIdx.x >> 3);
     if (tix >= ntiles) return;
     const int4 tl = tiles[tix];
-    const BlockDev &B = blocks[tl.x];
+    BlockRef B = block_at(blocks, tl.x);
     const int t = threadIdx.x, tk = t % TK, tj = t / TK;
     const int j = tl.z + tj + 1, k = tl.w + tk + 1;
     const bool own = j <= B.nj && k <= B.nk;

@@ -15,7 +15,7 @@ namespace fv3d {
 // and centrifugal outlet (source/BndCondOutlet.cpp:116-305), no-slip wall
 // (source/BndCondWall.cpp:20-284).  Writes ghost cells of Q/W and the two
 // Dummy layers of the patch side.
-__device__ static void set_dummies(const BlockDev &B, int s, int a, int b, const double cv[5], const double pv[6])
+__device__ static void set_dummies(BlockRef B, int s, int a, int b, const double cv[5], const double pv[6])
 {
     for (int l = 1; l <= kND; ++l) {
         for (int c = 0; c < 5; ++c) *dummy_ptr(B, s, l, c, a, b) = cv[c];
@@ -45,7 +45,7 @@ __global__ void k_bc(const BlockDev *__restrict__ blocks, const PatchDev *__rest
     if (t >= pstart[npatch]) return;
     const int q = find_range(pstart, npatch, t);
     const PatchDev P = patches[q];
-    const BlockDev &B = blocks[P.block];
+    BlockRef B = block_at(blocks, P.block);
     long r = t - pstart[q];
     int a = P.a0 + (int)(r / P.nb), b = P.b0 + (int)(r % P.nb);   // tangential cell indices
     const int d = P.dir, hi = P.hi;
@@ -173,7 +173,7 @@ __global__ void __launch_bounds__(256) k_bc_axial(const BlockDev *__restrict__ b
     __shared__ double cu[kAxialMaxI];
     const PatchDev P = patches[list[blockIdx.x]];
     if (P.dir != 2 || !P.hi) return;   // K+ faces only (source/BndCondOutlet.cpp:33-41)
-    const BlockDev &B = blocks[P.block];
+    BlockRef B = block_at(blocks, P.block);
     const int IM = B.IM, JM = B.JM, KM = B.KM, k = KM - 1;
     const long box = B.box;
     const double *fc = B.fc[2], *fs = B.fs[2];
@@ -246,7 +246,7 @@ __global__ void __launch_bounds__(256) k_dt_block_min(const BlockDev *__restrict
     __syncthreads();
     int n, i, j, k;
     if (cell_item(blocks, cstart, nblock, t, n, i, j, k)) {
-        const BlockDev &B = blocks[n];
+        BlockRef B = block_at(blocks, n);
         const unsigned long long v = (unsigned long long)__double_as_longlong(B.dt[cidx(B, i, j, k)]);
         if (n - n0 < kSlots) atomicMin(&smin[n - n0], v);
         else atomicMin(dtmin + n, v);
@@ -262,7 +262,7 @@ __global__ void __launch_bounds__(256) k_dt_global(const BlockDev *__restrict__ 
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(blocks, cstart, nblock, t, n, i, j, k)) return;
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     const long box = B.box, x = cidx(B, i, j, k);
     const double dt = __longlong_as_double((long long)dtmin[n]);
     B.dt[x] = dt;
@@ -291,7 +291,7 @@ __global__ void k_exchange(const BlockDev *__restrict__ blocks, const ExchDev *_
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     const ExchDev e = el[t];
-    const BlockDev &A = blocks[e.src_block], &B = blocks[e.dst_block];
+    BlockRef A = block_at(blocks, e.src_block), B = block_at(blocks, e.dst_block);
     double q[5], w[6];
     for (int c = 0; c < 5; ++c) q[c] = A.Q[c * A.box + e.src];
     for (int c = 0; c < 6; ++c) w[c] = A.W[c * A.box + e.src];
@@ -321,7 +321,7 @@ __global__ void k_exchange(const BlockDev *__restrict__ blocks, const ExchDev *_
 __global__ void k_spectral_dt(const BlockDev *__restrict__ blocks, const long *__restrict__ cstart, int nblock, Gas g)
 {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    for_cell_item(blocks, cstart, nblock, t, [&](const BlockDev &B, int, int i, int j, int k) {
+    for_cell_item(blocks, cstart, nblock, t, [&](BlockRef B, int, int i, int j, int k) {
         const long box = B.box, x = cidx(B, i, j, k);
         const double Gamma = g.gamma, Rgas = g.rgas;
         double uvelr = B.W[box + x] + B.w_rot * B.cc[box + x];
@@ -378,7 +378,7 @@ __global__ void k_dt_flag_decrement(const BlockDev *__restrict__ blocks, int nbl
 // Face flux of CSpaceDiscr::Upwind_Convective (source/Upwind_Convective.cpp:5-360)
 // with the WallFlux override (source/WallFlux.cpp:70-175).
 template <int MODE>
-__device__ static void face_flux(const BlockDev &B, const Gas &g, int d, int i, int j, int k, double out[5])
+__device__ static void face_flux(BlockRef B, const Gas &g, int d, int i, int j, int k, double out[5])
 {
     const long box = B.box;
     const int N = d == 0 ? B.IM : d == 1 ? B.JM : B.KM;
@@ -459,7 +459,7 @@ k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles
     __shared__ double sK[5][TI][TJ][TK + 1];
     const int4 tl = tiles[blockIdx.x];
     if (tl.x < 0) return;   // padding of the XCD-ordered tile list
-    const BlockDev &B = blocks[tl.x];
+    BlockRef B = block_at(blocks, tl.x);
     const int t = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
     // one copy of the face code in a rolled loop: a copy per direction (every
@@ -531,7 +531,7 @@ __global__ void __launch_bounds__(256) k_conv_faces(const BlockDev *__restrict__
     if (t >= fstart[nlist]) return;
     const int q = find_range(fstart, nlist, t);
     const int d = q % 3;
-    const BlockDev &B = blocks[q / 3];
+    BlockRef B = block_at(blocks, q / 3);
     const long r = t - fstart[q];
     const int nj = B.nj + (d == 1 ? 1 : 0), nk = B.nk + (d == 2 ? 1 : 0);
     const int i = (int)(r / ((long)nj * nk)) + 1, j = (int)(r / nk % nj) + 1, k = (int)(r % nk) + 1;
@@ -551,7 +551,7 @@ __global__ void __launch_bounds__(256) k_conv_sum(const BlockDev *__restrict__ b
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(blocks, cstart, nblock, t, n, i, j, k)) return;
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     const long box = B.box, x = cidx(B, i, j, k);
     const double w_rot = B.w_rot;
     const double vol = B.vol[x];
@@ -573,7 +573,7 @@ __global__ void __launch_bounds__(256) k_conv_sum(const BlockDev *__restrict__ b
 // Flux difference of CTimeDiscr::delt_Fn_up / delt_Fn_down
 // (source/LU_SGS_Marching.cpp:293-419) at neighbour cell nb whose faces along
 // d are nb (lower) and nb + stride (upper).
-__device__ static void delt_fn(const BlockDev &B, double Gamma, int d, long nb, double df[5])
+__device__ static void delt_fn(BlockRef B, double Gamma, int d, long nb, double df[5])
 {
     const long box = B.box;
     const long st = d == 0 ? B.si : d == 1 ? B.sj : 1;
@@ -609,7 +609,7 @@ __global__ void k_lusgs_plane(const BlockDev *__restrict__ blocks, const long *_
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= pstart[nblock]) return;
     const int n = find_range(pstart, nblock, t);
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     const long r = t - pstart[n];
     const int i = (int)(r / B.nj) + 1, j = (int)(r % B.nj) + 1;
     const int last = B.IM + B.JM + B.KM - 3;
@@ -714,7 +714,7 @@ __device__ inline bool mbox_empty(float x) { return __builtin_bit_cast(unsigned 
 // the mailbox set of a sweep direction, in words of T (both sets share one
 // allocation whose second half starts at mbox[1])
 template <class T>
-__device__ inline T *mbox_base(const BlockDev &B, bool fwd)
+__device__ inline T *mbox_base(BlockRef B, bool fwd)
 {
     return (T *)B.mbox[0] + (fwd ? 0 : (B.mbox[1] - B.mbox[0]));
 }
@@ -732,7 +732,7 @@ template <class T>
 __global__ void __launch_bounds__(256) k_sweep_fill(const BlockDev *__restrict__ blocks, int block, long nrows, int what)
 {
     constexpr int TJ = kKbaTJ, TK = kKbaTK;
-    const BlockDev &B = blocks[block];
+    BlockRef B = block_at(blocks, block);
     const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= nrows) return;
     const int lane = threadIdx.x & 63, tj = lane / TK, tk = lane % TK;
@@ -774,7 +774,7 @@ __device__ inline long xcd_item(long b, long n)
 // chunks of i, then j tiles, so consecutive items are neighbours along k (they
 // share the cell-box lines at their k edges) and items ntk apart neighbours
 // along i (they share the partly written rows at their chunk edges)
-__device__ inline void pack_item(const BlockDev &B, long wg, int nchunk, int &slot, int &i0)
+__device__ inline void pack_item(BlockRef B, long wg, int nchunk, int &slot, int &i0)
 {
     const int K = (int)(wg % B.ntk);
     const long rest = wg / B.ntk;
@@ -799,7 +799,7 @@ __global__ void __launch_bounds__(256) k_sweep_pack(const BlockDev *__restrict__
     const long item = xcd_item(blockIdx.x, gridDim.x);
     const int qg = (int)(item % qsplit);
     const int block = find_range(gstart, nblock, item / qsplit);
-    const BlockDev &B = blocks[block];
+    BlockRef B = block_at(blocks, block);
     const long wg = item / qsplit - gstart[block];
     const int nchunk = (B.ni + kPackChunk - 1) / kPackChunk;
     int slot, i0;
@@ -850,7 +850,7 @@ __global__ void __launch_bounds__(256) k_sweep_unpack(const BlockDev *__restrict
     const long item = xcd_item(blockIdx.x, gridDim.x);
     const int cg = (int)(item % csplit);
     const int block = find_range(gstart, nblock, item / csplit);
-    const BlockDev &B = blocks[block];
+    BlockRef B = block_at(blocks, block);
     const long wg = item / csplit - gstart[block];
     const int nchunk = (B.ni + kPackChunk - 1) / kPackChunk;
     int slot, i0;
@@ -939,7 +939,7 @@ __global__ void __launch_bounds__(256) k_lusgs_sl(const BlockDev *__restrict__ b
         __syncthreads();
         if (q >= ntiles) return;
         const KbaTile tl = tiles[q];
-        const BlockDev &B = blocks[tl.block];
+        BlockRef B = block_at(blocks, tl.block);
         const int ni = B.ni, nj = B.nj, nk = B.nk, nr = B.nr, ntk = B.ntk;
         const int slot = (tl.j0 / TJ) * ntk + tl.k0 / TK;
         const gcT<T> rows = (gcT<T>)((const T *)B.srow + (long)slot * nr * RQ);
@@ -1287,7 +1287,7 @@ __global__ void __launch_bounds__(256) k_update(const BlockDev *__restrict__ blo
     __shared__ double red[5][256];
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     double rm[5] = {0, 0, 0, 0, 0};
-    for_cell_item(blocks, cstart, nblock, t, [&](const BlockDev &B, int n, int i, int j, int k) {
+    for_cell_item(blocks, cstart, nblock, t, [&](BlockRef B, int n, int i, int j, int k) {
         const long box = B.box, x = cidx(B, i, j, k);
         double q[5];
         const double vol = B.vol[x];
@@ -1325,7 +1325,7 @@ __global__ void __launch_bounds__(256) k_update(const BlockDev *__restrict__ blo
 // Limit_Vars (source/Limit_FlowVars.cpp:8-119) in the reference's serial order:
 // cells are repaired one after the other, so later repairs see earlier ones.
 // Runs as one thread and returns at once unless k_update flagged a bad cell.
-__device__ static bool bad_cell(const BlockDev &B, long x)
+__device__ static bool bad_cell(BlockRef B, long x)
 {
     const long box = B.box;
     const double dmin = F32C(1.0E-6), dmax = F32C(1000.0), vmax = F32C(1000.0);
@@ -1350,7 +1350,7 @@ __global__ void k_limiter_serial(const BlockDev *__restrict__ blocks, int nblock
     for (int n = 0; n < nblock; ++n) {
         if (!bad_flag[n]) continue;
         bad_flag[n] = 0;
-        const BlockDev &B = blocks[n];
+        BlockRef B = block_at(blocks, n);
         const long box = B.box;
         int nneg = 0;
         for (int i = 1; i <= B.ni; ++i)
@@ -1419,7 +1419,7 @@ __global__ void __launch_bounds__(256) k_sections(const BlockDev *__restrict__ b
     __shared__ double red[3][256];
     const int sec = blockIdx.x / kSecParts, part = blockIdx.x % kSecParts;
     const int2 sc = secs[sec];
-    const BlockDev &B = blocks[sc.x];
+    BlockRef B = block_at(blocks, sc.x);
     const int K = sc.y;
     const long box = B.box;
     const double Gamma = g.gamma, Rgas = g.rgas;
@@ -1540,7 +1540,7 @@ struct MixAvg {
     double d, u, v, w, p, c, ev;
 };
 
-__device__ static void mix_terms(const BlockDev &B, int i, int j, int kf, int kc, int sa, double *t)
+__device__ static void mix_terms(BlockRef B, int i, int j, int kf, int kc, int sa, double *t)
 {
     const long xf = cidx(B, i, j, kf), xc = cidx(B, i, j, kc), box = B.box;
     const double s = B.fs[2][xf];
@@ -1591,7 +1591,7 @@ __device__ static MixAvg mix_reduce(const double (*t)[10], int nj, const Gas &g,
     return a;
 }
 
-__device__ static void mix_ghost(const BlockDev &B, int s, int i, int j, int kg, double d, double u, double v,
+__device__ static void mix_ghost(BlockRef B, int s, int i, int j, int kg, double d, double u, double v,
                                  double w, double p, double ev, const Gas &g, int sa)
 {
     const double Gamma = g.gamma, Rgas = g.rgas;
@@ -1614,7 +1614,7 @@ __global__ void __launch_bounds__(256) k_mixing_plane(const BlockDev *__restrict
     while (q + 1 < nmix && mix[q + 1].line0 <= (int)blockIdx.x) ++q;
     const MixDev M = mix[q];
     const int i = M.i0 + ((int)blockIdx.x - M.line0);
-    const BlockDev &U = blocks[M.b1], &D = blocks[M.b2];
+    BlockRef U = block_at(blocks, M.b1), D = block_at(blocks, M.b2);
     const int KM = U.KM;
     for (int side = 0; side < 2; ++side) {
         const int nj = side ? M.nj2 : M.nj1, j0 = side ? M.j2 : M.j1;

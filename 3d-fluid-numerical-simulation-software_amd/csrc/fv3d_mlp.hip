@@ -219,7 +219,7 @@ __device__ inline bf16x8 input_operand(const float *sx, int q, int lane)
 // Omega = sqrt(2 W_ij W_ij), d the wall distance.  The differences of the
 // state are taken in FP64 (they cancel), the rest in FP32: the features feed
 // a BF16 network.
-__device__ inline void cell_features(const BlockDev &B, const Gas &g, int i, int j, int k, float f[kMlpIn])
+__device__ inline void cell_features(BlockRef B, const Gas &g, int i, int j, int k, float f[kMlpIn])
 {
     const long box = B.box, x = cidx(B, i, j, k);
     const long st[3] = {B.si, B.sj, 1};
@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(256) k_mlp_features(const BlockDev *__restrict
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(blocks, cstart, nblock, t, n, i, j, k)) return;
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     float f[kMlpIn];
     cell_features(B, g, i, j, k, f);
     const long r = fstart[n] + ((long)(i - 1) * B.nj + (j - 1)) * B.nk + (k - 1);
@@ -282,7 +282,7 @@ __global__ void __launch_bounds__(256) k_mlp_targets(const BlockDev *__restrict_
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(blocks, cstart, nblock, t, n, i, j, k)) return;
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     const long x = cidx(B, i, j, k);
     const double mue_lam = sutherland(g, B.W[5 * B.box + x]);
     out[fstart[n] + ((long)(i - 1) * B.nj + (j - 1)) * B.nk + (k - 1)] = (float)log1p(B.mut[x] / mue_lam);
@@ -330,7 +330,7 @@ __global__ void __launch_bounds__(256) k_mlp_cell_features(const BlockDev *__res
     if (t >= ncell) return;
     float f[kMlpIn] = {0, 0, 0, 0, 0, 0};
     bool ok = false;
-    for_cell_item(blocks, cstart, nblock, t, [&](const BlockDev &B, int, int i, int j, int k) {
+    for_cell_item(blocks, cstart, nblock, t, [&](BlockRef B, int, int i, int j, int k) {
         cell_features(B, g, i, j, k, f);
         ok = true;
         for (int q = 0; q < kMlpIn; ++q) {
@@ -348,7 +348,7 @@ __global__ void __launch_bounds__(256) k_mlp_cell_features(const BlockDev *__res
 // above the largest trained value, the Spalart-Allmaras value of its frozen
 // nu~ (fv1 rho nu~ / Re, clipped as SA_Model clips it); true when the
 // fallback was taken.
-__device__ static bool mut_cell(const BlockDev &B, int i, int j, int k, const Gas &g, const float *__restrict__ bounds,
+__device__ static bool mut_cell(BlockRef B, int i, int j, int k, const Gas &g, const float *__restrict__ bounds,
                                 float yhat, bool ok, double relax)
 {
     const long box = B.box, x = cidx(B, i, j, k);
@@ -429,7 +429,7 @@ __global__ void __launch_bounds__(256) k_mlp_mut(const BlockDev *__restrict__ bl
     // not depend on, so the wave waits on memory once for them and the block
     const float2 v = ((const float2 *)(xc + 8 * (c < cstart[nblock] ? c : 0)))[3];
     bool trip = false;
-    for_cell_item(blocks, cstart, nblock, c, [&](const BlockDev &B, int, int i, int j, int k) {
+    for_cell_item(blocks, cstart, nblock, c, [&](BlockRef B, int, int i, int j, int k) {
         trip = mut_cell(B, i, j, k, g, bounds, v.y, v.x != 0.0f, relax);
     });
     // one atomic per wave for the fallback count (every lane reaches this

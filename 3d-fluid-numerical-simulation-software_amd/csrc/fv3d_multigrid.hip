@@ -13,7 +13,7 @@ namespace fv3d {
 // W from Q for one interior cell (CFluidProps::PrimitiveVars,
 // source/PrimitiveVars.cpp:7-29) and the limiter's bad-cell test
 // (source/Limit_FlowVars.cpp:26-28)
-__device__ static inline void prim_vars(const BlockDev &B, long x, const double q[5], const Gas &g, int *bad)
+__device__ static inline void prim_vars(BlockRef B, long x, const double q[5], const Gas &g, int *bad)
 {
     const long box = B.box;
     const double Gamma = g.gamma, Rgas = g.rgas;
@@ -34,7 +34,7 @@ __global__ void __launch_bounds__(256) k_prim_all(const BlockDev *__restrict__ b
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(blocks, cstart, nblock, t, n, i, j, k)) return;
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     const long x = cidx(B, i, j, k);
     double q[5];
     for (int c = 0; c < 5; ++c) q[c] = B.Q[c * B.box + x];
@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(256) k_mg_restrict(const BlockDev *__restrict_
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(coarse, cstart, nblock, t, n, i, j, k)) return;
-    const BlockDev &F = fine[n], &B = coarse[n];
+    BlockRef F = block_at(fine, n), B = block_at(coarse, n);
     double sq[5], sr[5];
     bool first = true;
     for (int a = 0; a < 2; ++a)
@@ -92,7 +92,7 @@ __global__ void __launch_bounds__(256) k_mg_restrict(const BlockDev *__restrict_
 // ever averages zeros: its ghost cells are never written.)
 __global__ void __launch_bounds__(256) k_mg_corner(const BlockDev *__restrict__ coarse)
 {
-    const BlockDev &B = coarse[blockIdx.x];
+    BlockRef B = block_at(coarse, blockIdx.x);
     const int IM = B.IM, JM = B.JM, KM = B.KM;
     const long box = B.box;
     const int ne = 4 * (IM - 1) + 4 * (JM - 1) + 4 * (KM - 1);
@@ -157,7 +157,7 @@ __global__ void __launch_bounds__(256) k_mg_prolong(const BlockDev *__restrict__
     __shared__ double sd[5][NH];
     const int4 tl = tiles[blockIdx.x];
     const int n = tl.x, I0 = tl.y, J0 = tl.z, K0 = tl.w;
-    const BlockDev &F = fine[n], &B = coarse[n];
+    BlockRef F = block_at(fine, n), B = block_at(coarse, n);
     const long cbox = B.box;
     for (int e = threadIdx.x; e < NH; e += blockDim.x) {
         const int c3 = e % HK, b3 = (e / HK) % HJ, a3 = e / (HK * HJ);
@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(256) k_fas(const BlockDev *__restrict__ blocks
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(blocks, cstart, nblock, t, n, i, j, k)) return;
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     const long x = cidx(B, i, j, k), box = B.box;
     for (int c = 0; c < 5; ++c) {
         const long y = c * box + x;

@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(256) k_wall_distance(const BlockDev *__restric
     long x = 0;
     int f0 = 0, f1 = 0;   // this cell's wall faces
     if (valid) {
-        const BlockDev &B = blocks[n];
+        BlockRef B = block_at(blocks, n);
         x = cidx(B, i, j, k);
         cx = B.cc[x]; cy = B.cc[B.box + x]; cz = B.cc[2 * B.box + x];
         f0 = B.wf0;
@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
     __shared__ double sf[3 * TL::NF];   // convective, viscous, plain gradient flux
     const int4 tl = tiles[blockIdx.x];
     if (tl.x < 0) return;   // padding of the XCD-ordered tile list
-    const BlockDev &B = blocks[tl.x];
+    BlockRef B = block_at(blocks, tl.x);
     const long box = B.box;
     const int t = threadIdx.x;
     const SaConst K;
@@ -246,7 +246,7 @@ __global__ void __launch_bounds__(256) k_sa_mut(const BlockDev *__restrict__ blo
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(blocks, cstart, nblock, t, n, i, j, k)) return;
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     const long box = B.box, x = cidx(B, i, j, k);
     const SaConst K;
     const double Re = g.re_ref;
@@ -276,7 +276,7 @@ __global__ void __launch_bounds__(256) k_sa_ghost(const BlockDev *__restrict__ b
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= gstart[nblock]) return;
     const int n = find_range(gstart, nblock, t);
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     long r = t - gstart[n];
     const long nf[3] = {(long)B.nj * B.nk, (long)B.ni * B.nk, (long)B.ni * B.nj};
     int side = 0;
@@ -315,7 +315,7 @@ __global__ void k_sa_plane(const BlockDev *__restrict__ blocks, const long *__re
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= pstart[nblock]) return;
     const int n = find_range(pstart, nblock, t);
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     const long r = t - pstart[n];
     const int i = (int)(r / B.nj) + 1, j = (int)(r % B.nj) + 1;
     const int last = B.IM + B.JM + B.KM - 3;
@@ -372,7 +372,7 @@ __global__ void k_sa_limit_serial(const BlockDev *__restrict__ blocks, int nbloc
     for (int n = 0; n < nblock; ++n) {
         if (!hi_flag[n]) continue;
         hi_flag[n] = 0;
-        const BlockDev &B = blocks[n];
+        BlockRef B = block_at(blocks, n);
         const int IM = B.IM, JM = B.JM, KM = B.KM;
         for (int i = 1; i <= B.ni; ++i)
             for (int j = 1; j <= B.nj; ++j)
@@ -410,7 +410,7 @@ __global__ void __launch_bounds__(256) k_sa_res(const BlockDev *__restrict__ blo
     double v = 0.0;
     int n, i, j, k;
     if (cell_item(blocks, cstart, nblock, t, n, i, j, k)) {
-        const BlockDev &B = blocks[n];
+        BlockRef B = block_at(blocks, n);
         const long x = cidx(B, i, j, k);
         double e = B.ev[x];
         if (clamp && e < F32C(1.0E-8)) {

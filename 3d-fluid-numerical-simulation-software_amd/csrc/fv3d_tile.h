@@ -27,7 +27,7 @@ struct VTile {
 // the other three averaged; at the J face j == JM, k == 1 the reference also
 // scales the lower three-cell sum by 0.25 (line 331).
 template <int D, class TL, int NV = 4>
-__device__ inline void face_dv(const double *sw, int l, int i, int j, int k, const BlockDev &B, double dv[3][NV])
+__device__ inline void face_dv(const double *sw, int l, int i, int j, int k, BlockRef B, double dv[3][NV])
 {
     constexpr int NH = TL::NH;
     const int st[3] = {TL::HJ * TL::HK, TL::HK, 1};

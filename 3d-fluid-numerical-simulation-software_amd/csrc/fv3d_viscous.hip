@@ -43,7 +43,7 @@ __device__ static void metric9(const double e1[3], const double e2[3], const dou
 __global__ void k_metrics(const BlockDev *__restrict__ blocks, int block, double *fg0, double *fg1, double *fg2,
                           double *cg)
 {
-    const BlockDev &B = blocks[block];
+    BlockRef B = block_at(blocks, block);
     const long box = B.box;
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= 4 * box) return;
@@ -106,7 +106,7 @@ __global__ void k_metrics(const BlockDev *__restrict__ blocks, int block, double
 // Viscous flux of one face (source/ViscousFlux.cpp:34-108); without a
 // turbulence model mue_tur = cond_tur = 0 (lines 68-72).
 template <int D, class TL>
-__device__ static void face_fv(const double *sw, int l, int i, int j, int k, const BlockDev &B, const Gas &g,
+__device__ static void face_fv(const double *sw, int l, int i, int j, int k, BlockRef B, const Gas &g,
                                double out[5], double *gstore)
 {
     constexpr int NH = TL::NH;
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_viscous(const BlockDev *__restri
     __shared__ double sf[4 * TL::NF];
     const int4 tl = tiles[blockIdx.x];
     if (tl.x < 0) return;   // padding of the XCD-ordered tile list
-    const BlockDev &B = blocks[tl.x];
+    BlockRef B = block_at(blocks, tl.x);
     const long box = B.box;
     const int t = threadIdx.x;
     // u v w T of the tile's cells and halo, clamped into the cell box
@@ -250,7 +250,7 @@ FV3D_FOR_TILES(FV3D_VISC)
 __global__ void k_curl(const BlockDev *__restrict__ blocks, const long *__restrict__ cstart, int nblock)
 {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    for_cell_item(blocks, cstart, nblock, t, [&](const BlockDev &B, int, int i, int j, int k) {
+    for_cell_item(blocks, cstart, nblock, t, [&](BlockRef B, int, int i, int j, int k) {
         const long box = B.box, x = cidx(B, i, j, k);
         const long st[3] = {B.si, B.sj, 1};
         double d[3][3];   // d/dkesi, d/dyita, d/dzita of u v w
@@ -305,7 +305,7 @@ __global__ void __launch_bounds__(kBlLines *G) k_bl_lines(const BlockDev *__rest
     int w = 0;
     while (w < nwalls && t >= walls[w].y) { t -= walls[w].y; ++w; }
     const PatchDev P = patches[walls[min(w, nwalls - 1)].x];
-    const BlockDev &B = blocks[P.block];
+    BlockRef B = block_at(blocks, P.block);
     const long line = t + lane;
     const bool active = w < nwalls && line < (long)P.na * P.nb;
     const int a = P.a0 + (int)(active ? line / P.nb : 0), cc = P.b0 + (int)(active ? line % P.nb : 0);
@@ -424,7 +424,7 @@ __global__ void __launch_bounds__(256) k_bl_merge(const BlockDev *__restrict__ b
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(blocks, cstart, nblock, t, n, i, j, k)) return;
-    const BlockDev &B = blocks[n];
+    BlockRef B = block_at(blocks, n);
     const long x = cidx(B, i, j, k);
     const unsigned long long v = B.blmin[x];
     if (v != kBlUnvisited) {
