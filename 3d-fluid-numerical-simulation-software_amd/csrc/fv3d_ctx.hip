@@ -1874,7 +1874,7 @@ static int launch_sweeps_kba(fv3d_ctx *c)
         auto sweep = [&](bool fwd) {
             int *tk = fwd ? tf : tb;
             const KbaTile *tl = c->d_kba[fwd ? 0 : 1];
-            dim3 g((unsigned)c->kba_grid), b(256);
+            dim3 g((unsigned)c->kba_grid), b(kSlThreads);
 #define FV3D_SL_LAUNCH(F, V, S, T) \
     hipLaunchKernelGGL((k_lusgs_sl<F, kKbaTJ, kKbaTK, V, S, T>), g, b, 0, c->stream, c->d_blocks, tl, c->nkba, tk, err, \
                        c->gas.relax, c->gas)

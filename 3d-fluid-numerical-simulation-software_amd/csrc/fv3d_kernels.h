@@ -129,6 +129,9 @@ constexpr int kSQ_Q = 0, kSQ_P = 5, kSQ_LAM = 6, kSQ_SWG = 9, kSQ_R = 24, kSQ_A 
 constexpr int kSweepD = 6;
 // what k_sweep_fill writes: the state quantities and/or the static metrics
 constexpr int kGatherState = 1, kGatherMetrics = 2;
+// threads per workgroup of k_lusgs_sl: three direction waves, the mailbox wave,
+// three combine waves
+constexpr int kSlThreads = 448;
 // T: double (plain FP64) or float (the FP32 operator of defect correction)
 // SA: the nu~ equation in the same sweep (Navier-Stokes only)
 template <bool FWD, int TJ, int TK, bool VISC, bool SA, class T>

@@ -669,45 +669,36 @@ using gT = T __attribute__((address_space(1))) *;
 #define TC(x) ((T)(x##f))
 
 namespace {
-// row-layout sweep: per step, the neighbour's static data with the terms of
-// the flux difference that do not depend on dQ, the upstream dQ, and (wave 0)
-// the cell's right-hand side and diagonal
+// row-layout sweep, direction waves: per step the neighbour's static data and the
+// terms of the flux difference that do not depend on dQ
 template <class T>
 struct RowPf {
-    T q[5], m[5], of[5], vn_old, cl;   // state, metrics, old-state flux terms
-    T p, l, lv;
-    T x[kSweepD];                      // upstream tile's dQ (and dnu~)
-    T r[5], a;
-    T ev, rev, a2;                     // Spalart-Allmaras: neighbour's nu~; own nu~ right-hand side and diagonal
+    T q[5], m[5], p, l, lv, ev;        // state, metrics, pressure, lambda_c, lambda_v, nu~
+    T of[5], vn_old, cl;               // old-state flux terms
 };
-template <int D>
-struct Dir {
-    static constexpr int value = D;
+template <int N>
+struct Int {
+    static constexpr int value = N;
 };
-// A direction wave issues the static loads of a step (the neighbour's state and
-// metrics, its own right-hand side) kStaticAhead steps before the step and
-// forms their early terms one step before it, so a load has kStaticAhead - 1
-// steps to arrive; it cycles through kRing row buffers.
-#ifndef FV3D_STATIC_AHEAD
-#define FV3D_STATIC_AHEAD 3
-#endif
-constexpr int kStaticAhead = FV3D_STATIC_AHEAD;
+// The static loads of a step are issued kStaticAhead steps before it and its
+// early terms formed one step before it, so a load has kStaticAhead - 1 steps to
+// arrive; a wave cycles through kRing row buffers.  Four steps: with three the
+// FP64 sweep of a 1.05M-cell channel takes 424 us instead of 326, with five or more
+// the idle steps at a tile's ends cost more than the loads still gain.
+constexpr int kStaticAhead = 4;
 constexpr int kRing = kStaticAhead + 1;
-// The upstream tile's dQ for a step is read kCrossAhead steps before the step
-// (the word may still be empty then; the step re-reads it until it is not).
-// Reading it earlier than one step ahead finds it empty more often than it
-// hides latency: measured on the 2.54M-cell vane passage, two steps ahead
-// gained 3-7 % on the fine FP32 sweeps and lost as much on FP64 and coarse ones.
-#ifndef FV3D_CROSS_AHEAD
-#define FV3D_CROSS_AHEAD 1
-#endif
-constexpr int kCrossAhead = FV3D_CROSS_AHEAD;
-static_assert(kCrossAhead >= 1 && kCrossAhead <= kStaticAhead, "the cross read lands in a free row buffer");
 constexpr int kRowS0 = -kStaticAhead;   // first (idle) step of the row-layout sweep loops
+// Keeps a value computed where it stands: the compiler may not move it past a
+// later barrier.  No instruction.
+__device__ inline void pin(double &x) { asm volatile("" : "+v"(x)); }
+__device__ inline void pin(float &x) { asm volatile("" : "+v"(x)); }
 // 1/x for the FP32 operator: the hardware reciprocal (within 1 ulp), one
 // instruction where a correctly rounded division takes about ten; the FP32
 // operator only preconditions the FP64 residual, whose fixed point it keeps
 __device__ inline float rcp_op(float x) { return __builtin_amdgcn_rcpf(x); }
+// the reciprocal a combine wave divides with: DivBy's (FP64), rcp_op's (FP32)
+__device__ inline double recip(double x) { return DivBy(x).r; }
+__device__ inline float recip(float x) { return rcp_op(x); }
 // whether a mailbox word still holds the empty pattern
 __device__ inline bool mbox_empty(double x) { return __builtin_bit_cast(unsigned long long, x) == kMboxEmpty; }
 __device__ inline bool mbox_empty(float x) { return __builtin_bit_cast(unsigned int, x) == kMboxEmpty32; }
@@ -885,25 +876,35 @@ template __global__ void k_sweep_unpack<double>(const BlockDev *, const long *, 
 template __global__ void k_sweep_unpack<float>(const BlockDev *, const long *, int, int, int);
 
 // The persistent wavefront form of the sweeps, on the tile-skewed layout.  The
-// (j,k) cross-section is cut into 4 x 16 tiles, one workgroup of four waves
-// per tile; tiles are handed out by a ticket counter in topological order, so
-// a tile waits only on tiles already running.  Waves 0, 1, 2 each own one
-// neighbour direction (i, j, k): a step ahead they load the neighbour's
-// state and metrics, then form the flux difference and off-diagonal terms of
-// the step's 64 cells in LDS; wave 3 combines them into dQ, keeps dQ in LDS for
-// the next step and stores it.  Every load is issued unconditionally with
-// clamped indices, so the compiler's memory-counter waits are exact.  The
-// per-hyperplane kernel k_lusgs_plane above is the reference's own schedule
-// and gives the same bits.  A step touches one row of its tile: the three
-// direction waves read their neighbours' state and metrics from the previous
-// row (a lane shift) or, on the tile's upstream edge, from the upstream tile's
-// row, so every load is a contiguous run of one row.  dQ goes to the tile's
-// dQ rows.
+// (j,k) cross-section is cut into 4 x 16 tiles, one workgroup per tile; tiles
+// are handed out by a ticket counter in topological order, so a tile waits only
+// on tiles already running.  A step (one row of the tile, 64 cells) needs the
+// dQ of the step before, so the sweep takes about ni + nj + nk steps in a chain
+// and its time is the latency of one step.  Everything that does not depend on
+// that dQ is therefore taken off the chain, by giving each wave one role:
+//   waves 0, 1, 2 (one neighbour direction each): the flux difference and the
+//     off-diagonal terms of the step's 64 cells into LDS; while the combine
+//     waves work, the loads of the step kStaticAhead on and the terms of the next
+//     step that use the old state only (kept there by an empty asm: left alone,
+//     the compiler moves them past the barrier, onto the chain);
+//   wave 3 (mailbox): reads the dQ that crosses the tile's two upstream edges,
+//     ahead of its step, waits for it (bounded) and leaves it in LDS
+//     beside the in-tile dQ, so a direction wave reads both alike;
+//   waves 4, 5, 6 (combine): each sums two of the components into dQ, keeps dQ in
+//     LDS for the next step and stores it; the right-hand side, the diagonal
+//     and its reciprocal are ready before the terms are.
+// Two barriers a step: the terms are in LDS, dQ is in LDS.  With three direction
+// waves and one combine wave, each doing its own loads and waits, a step took
+// 1.03 us (FP64) and 0.58 us (FP32); it takes 0.58 and 0.40 us.  Forward sweep: 96x32x32
+// channel 188 -> 115 us (FP64), 127 -> 83 us (FP32); 1.05M-cell channel 511 -> 323 and
+// 348 -> 248 us; 2.54M-cell five-block passage with nu~ 735 -> 435 and 398 -> 275 us.
+// Every load is issued unconditionally with clamped indices, so the compiler's
+// memory-counter waits are exact.  The per-hyperplane kernel k_lusgs_plane above is the reference's own
+// schedule and gives the same bits.
 //
 // Across a tile edge dQ travels through the upstream tile's mailbox: its
-// combine wave stores the dQ of its edge lanes there as soon as it has them,
-// and the consumer reads the words a step ahead and, before using them, waits
-// (bounded) while any word it needs still holds the empty pattern.  Tiles
+// combine waves store the dQ of its edge lanes there as soon as they have them;
+// a word that still holds the empty pattern has not been written.  Tiles
 // start in ticket order, so every upstream tile is already running.
 //
 // With SA the nu~ equation of Spalart-Allmaras rides along as a sixth
@@ -913,20 +914,32 @@ template __global__ void k_sweep_unpack<float>(const BlockDev *, const long *, i
 // updates both per cell from the same neighbour increments, so this is its
 // order.
 template <bool FWD, int TJ, int TK, bool VISC, bool SA, class T>
-__global__ void __launch_bounds__(256) k_lusgs_sl(const BlockDev *__restrict__ blocks, const KbaTile *__restrict__ tiles,
-                                                  int ntiles, int *__restrict__ ticket, int *__restrict__ err,
-                                                  double relax, Gas g)
+__global__ void __launch_bounds__(kSlThreads) k_lusgs_sl(const BlockDev *__restrict__ blocks, const KbaTile *__restrict__ tiles,
+                                                         int ntiles, int *__restrict__ ticket, int *__restrict__ err,
+                                                         double relax, Gas g)
 {
     static_assert(TJ * TK == 64, "64 cells per tile");
     static_assert(!SA || VISC, "Spalart-Allmaras runs with the viscous terms");
     // The FP32 operator forms the flux difference without cancellation; the
     // FP64 one follows the reference's expression order.
     constexpr bool kDeltaForm = sizeof(T) == 4;
-    constexpr int NC = SA ? 6 : 5;   // increments carried per cell
-    __shared__ T sdq[2][NC][64];
-    __shared__ T sA[3][NC][64];
-    __shared__ T sV[3][NC][64];
-    __shared__ T sR[SA ? 8 : 6][64];   // R, alpha; with SA the nu~ right-hand side and alpha2
+    constexpr int NC = SA ? 6 : 5;        // increments carried per cell
+    constexpr int kE = 64 + TK + TJ;      // dQ per component: the tile's cells, then the j-edge and k-edge words
+    // LDS words are laid out so that a lane moves 16 bytes at a time.
+    // dQ of a step, two buffers: FP32 (0..3) of a lane together, FP64 (0,1) and
+    // (2,3) in a plane each; then 4 (and nu~).
+    constexpr int NR = NC - 4;
+    constexpr bool kWide = sizeof(T) == 4;
+    __shared__ __align__(16) T sdq[2][kE * 4 + kE * NR];
+    auto dqi = [](int c, int l) {
+        return c >= 4 ? kE * 4 + l * NR + c - 4 : kWide ? l * 4 + c : (c >> 1) * kE * 2 + l * 2 + (c & 1);
+    };
+    // off-diagonal terms A and V of components (2p, 2p+1), per direction
+    typedef T Pair __attribute__((ext_vector_type(2)));
+    typedef T Quad __attribute__((ext_vector_type(4)));
+    __shared__ Pair sA[kWide && VISC ? 1 : 3][3][64];
+    __shared__ Pair sV[!kWide && VISC ? 3 : 1][3][64];
+    __shared__ Quad sAV[kWide && VISC ? 3 : 1][3][64];
     __shared__ int s_q;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int tj = lane / TK, tk = lane % TK;
@@ -947,17 +960,12 @@ __global__ void __launch_bounds__(256) k_lusgs_sl(const BlockDev *__restrict__ b
         const int lj = FWD ? tj : TJ - 1 - tj, lk = FWD ? tk : TK - 1 - tk;
         const int j = tl.j0 + tj + 1, k = tl.k0 + tk + 1;
         const bool col = j <= nj && k <= nk;
-        const int nsteps = nr;
         // steps run: [kRowS0, send), a whole number of kRing-step unrollings
-        const int send = (nsteps - kRowS0 + kRing - 1) / kRing * kRing + kRowS0;
+        const int send = (nr - kRowS0 + kRing - 1) / kRing * kRing + kRowS0;
         auto clampr = [&](int r) { return min(max(r, 0), nr - 1); };
-        // own row of a step, and whether this lane's cell is in the block
+        // own row of a step.  At step s a lane's cell has l2 = s - lj - lk cells
+        // of its column done before it, and exists when 0 <= l2 < ni.
         auto row_of = [&](int step) { return FWD ? step : nr - 1 - step; };
-        auto cell_at = [&](int step, int &i) -> bool {
-            const int l2 = step - lj - lk;
-            i = FWD ? l2 + 1 : ni - l2;
-            return col && l2 >= 0 && l2 < ni;
-        };
         auto bar = []() {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
             __builtin_amdgcn_s_barrier();
@@ -968,73 +976,29 @@ __global__ void __launch_bounds__(256) k_lusgs_sl(const BlockDev *__restrict__ b
             constexpr int TE = d == 1 ? TJ : TK;   // tile extent along d
             const int dep = d == 1 ? tl.dep_j : d == 2 ? tl.dep_k : -1;
             const bool edge = d == 1 ? tj == (FWD ? 0 : TJ - 1) : d == 2 ? tk == (FWD ? 0 : TK - 1) : false;
-            // upstream tile's rows (this tile's own when there is none: the
-            // values are then never used)
-            const int uslot = dep < 0 ? slot : d == 1 ? slot + (FWD ? -ntk : ntk) : slot + (FWD ? -1 : 1);
-            const gcT<T> urows = (gcT<T>)((const T *)B.srow + (long)uslot * nr * RQ);
-            const gcT<T> udrows = (gcT<T>)((const T *)B.sdq + (long)uslot * nr * RD);
-            // the upstream lane facing this lane across the tile edge
-            const int ulane = d == 1 ? (FWD ? (TJ - 1) * TK : 0) + tk : tj * TK + (FWD ? TK - 1 : 0);
-            // in-tile neighbour lane (lanes on the edge read the upstream row instead)
-            const int nlane = (d == 0 || edge) ? lane : d == 1 ? lane + (FWD ? -TK : TK) : lane + (FWD ? -1 : 1);
             const bool from_up = d != 0 && edge && dep >= 0;
-            // the upstream tile's mailbox words this lane reads (the other lanes
-            // read the same words as the edge lanes)
-            const gT<T> umbox = (gT<T>)(mbox_base<T>(B, FWD) + (long)uslot * nr * kMboxRow);
-            const int mword = d == 1 ? tk : kMboxJ + tj;
-            const int mstride = d == 1 ? TK : TJ;
-            // upstream dQ of a step, read one step ahead without waiting
-            auto issue_cross = [&](RowPf<T> &bn, int step) {
-                if (d == 0) return;
-                const int urow = clampr(FWD ? row_of(step) + TE - 1 : row_of(step) - (TE - 1));
-                for (int c = 0; c < NC; ++c)
-                    bn.x[c] = __hip_atomic_load(umbox + urow * kMboxRow + mword + c * mstride, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-            };
-            // before using the upstream dQ of step s: re-read while a word the
-            // step needs is still empty (bounded; a run-out sets the error word)
-            auto settle_cross = [&](RowPf<T> &b, int s, bool need) {
-                if (d == 0) return;
-                auto empty = [&](const T *x) {
-                    bool e = false;
-                    for (int c = 0; c < NC; ++c) e = e || (mbox_empty(x[c]));
-                    return e;
-                };
-                if (!__builtin_amdgcn_ballot_w64(need && empty(b.x))) return;
-                const int urow = clampr(FWD ? row_of(s) + TE - 1 : row_of(s) - (TE - 1));
-                long spins = 0;
-                while (__builtin_amdgcn_ballot_w64(need && empty(b.x))) {
-                    __builtin_amdgcn_s_sleep(1);
-                    for (int c = 0; c < NC; ++c)
-                        b.x[c] = __hip_atomic_load(umbox + urow * kMboxRow + mword + c * mstride, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-                    if (++spins > (1L << 22)) { atomicExch(err, 1); break; }
-                }
-            };
-            // the neighbour's state and metrics of a step (static during the
-            // sweep, so no wait), and for wave 0 the cell's right-hand side
+            // upstream tile, and its lane facing this lane across the tile edge
+            const int uslot = d == 1 ? slot + (FWD ? -ntk : ntk) : slot + (FWD ? -1 : 1);
+            const int ulane = d == 1 ? (FWD ? (TJ - 1) * TK : 0) + tk : tj * TK + (FWD ? TK - 1 : 0);
+            // in-tile neighbour lane
+            const int nlane = (d == 0 || edge) ? lane : d == 1 ? lane + (FWD ? -TK : TK) : lane + (FWD ? -1 : 1);
+            // where the neighbour's dQ lies in sdq, and its static row: the lane's
+            // column in the row before, or (edge lanes) the upstream tile's row
+            const int qlane = (d == 0 || !edge) ? nlane : d == 1 ? 64 + tk : 64 + TK + tj;
+            const gcT<T> src0 = from_up ? (gcT<T>)((const T *)B.srow + (long)uslot * nr * RQ) + ulane : rows + nlane;
+            const int radd = from_up ? (FWD ? TE - 1 : 1 - TE) : (FWD ? -1 : 1);
+            // the lane's neighbour takes part in steps 0 <= s - first < count
+            const bool okd = col && (d == 1 ? j != (FWD ? 1 : nj) : d == 2 ? k != (FWD ? 1 : nk) : true);
+            const int first = lj + lk + (d == 0 ? 1 : 0), count = okd ? ni - (d == 0 ? 1 : 0) : 0;
+            // the neighbour's state and metrics of a step (static during the sweep)
             auto issue_static = [&](RowPf<T> &bn, int step) {
-                const int rt = row_of(step);
-                const int urow = clampr(FWD ? rt + TE - 1 : rt - (TE - 1));
-                const int nrow = clampr(FWD ? rt - 1 : rt + 1);
-                const gcT<T> src = (from_up ? urows + urow * RQ + ulane : rows + nrow * RQ + nlane);
+                const gcT<T> src = src0 + (long)clampr(row_of(step) + radd) * RQ;
                 for (int c = 0; c < 5; ++c) bn.q[c] = src[(kSQ_Q + c) * 64];
                 bn.p = src[kSQ_P * 64];
                 bn.l = src[(kSQ_LAM + d) * 64];
                 if (VISC) bn.lv = src[(kSQ_LV + d) * 64];
                 for (int c = 0; c < 5; ++c) bn.m[c] = src[(kSQ_SWG + d * 5 + c) * 64];
                 if constexpr (SA) bn.ev = src[kSQ_EV * 64];
-                if (d == 0) {
-                    const int ro = clampr(rt);
-                    for (int c = 0; c < 5; ++c)
-                        bn.r[c] = FWD ? rows[ro * RQ + (kSQ_R + c) * 64 + lane] : ((gcT<T>)drows)[ro * RD + c * 64 + lane];
-                    bn.a = rows[ro * RQ + kSQ_A * 64 + lane];
-                    if constexpr (SA) {
-                        // forward: Res_ev; backward: the forward dnu~
-                        bn.rev = FWD ? rows[ro * RQ + kSQ_REV * 64 + lane] : ((gcT<T>)drows)[ro * RD + 5 * 64 + lane];
-                        bn.a2 = rows[ro * RQ + kSQ_A2 * 64 + lane];
-                    }
-                }
             };
             // the terms of the flux difference that use only the old state
             // (source/LU_SGS_Marching.cpp:293-419; same operations, evaluated early)
@@ -1052,30 +1016,36 @@ __global__ void __launch_bounds__(256) k_lusgs_sl(const BlockDev *__restrict__ b
                     b.of[2] = o[3] * r0;
                     b.of[3] = o[4] + press_old;
                     b.vn_old = b.of[0] * nx + b.of[1] * ny + b.of[2] * nz;
+                    pin(b.of[0]); pin(b.of[1]); pin(b.of[2]); pin(b.of[3]);
                 } else {
-                    const T Vn_old = o[1] / o[0] * nx + o[2] / o[0] * ny + o[3] / o[0] * nz;
+                    const DivBy by(o[0]);
+                    const T Vn_old = by.of(o[1]) * nx + by.of(o[2]) * ny + by.of(o[3]) * nz;
                     b.vn_old = Vn_old;
                     b.of[0] = o[0] * (Vn_old - Vn_e);
                     b.of[1] = o[1] * (Vn_old - Vn_e) + press_old * nx;
                     b.of[2] = o[2] * (Vn_old - Vn_e) + press_old * ny;
                     b.of[3] = o[3] * (Vn_old - Vn_e) + press_old * nz;
                     b.of[4] = (o[4] + press_old) * (Vn_old - Vn_e) + press_old * Vn_e;
+                    for (int c = 0; c < 5; ++c) pin(b.of[c]);
                 }
                 b.cl = (T)relax * b.l;
+                pin(b.cl);
+                pin(b.vn_old);
             };
-            // step s: the dQ-dependent part of the flux difference (critical
-            // path), then, while the combine wave works, the loads and early
-            // terms of the next steps
-            auto work = [&](RowPf<T> &b, RowPf<T> &b1, RowPf<T> &bc, RowPf<T> &bn, int s) {
-                int i;
-                const bool valid = cell_at(s, i);
-                const int p = d == 0 ? i : d == 1 ? j : k, lim = d == 0 ? ni : d == 1 ? nj : nk;
-                const bool use = valid && (FWD ? p != 1 : p != lim);
-                settle_cross(b, s, use && from_up);
+            // step s: the dQ-dependent part of the flux difference, the step's terms
+            auto chain = [&](const RowPf<T> &b, int s) {
+                const bool use = (unsigned)(s - first) < (unsigned)count;
                 T dqn[NC];
-                for (int c = 0; c < NC; ++c) {
-                    const T in_tile = sdq[(s - 1) & 1][c][nlane];
-                    dqn[c] = (d != 0 && edge) ? b.x[c] : in_tile;
+                {
+                    const T *from = sdq[(s - 1) & 1];
+                    if constexpr (kWide) {
+                        const Quad v = *(const Quad *)(from + dqi(0, qlane));
+                        for (int c = 0; c < 4; ++c) dqn[c] = v[c];
+                    } else {
+                        const Pair v = *(const Pair *)(from + dqi(0, qlane)), w = *(const Pair *)(from + dqi(2, qlane));
+                        dqn[0] = v[0]; dqn[1] = v[1]; dqn[2] = w[0]; dqn[3] = w[1];
+                    }
+                    for (int c = 4; c < NC; ++c) dqn[c] = from[dqi(c, qlane)];
                 }
                 const T nx = b.m[0], ny = b.m[1], nz = b.m[2], sd = b.m[3], Vn_e = b.m[4];
                 T df[5];
@@ -1107,7 +1077,8 @@ __global__ void __launch_bounds__(256) k_lusgs_sl(const BlockDev *__restrict__ b
                 } else {
                     T nw[5];
                     for (int c = 0; c < 5; ++c) nw[c] = b.q[c] + dqn[c];
-                    T dens = nw[0], uvel = nw[1] / nw[0], vvel = nw[2] / nw[0], wvel = nw[3] / nw[0], E = nw[4] / nw[0];
+                    const DivBy by(nw[0]);
+                    T dens = nw[0], uvel = by.of(nw[1]), vvel = by.of(nw[2]), wvel = by.of(nw[3]), E = by.of(nw[4]);
                     T press_new = (Gamma - TC(1.0)) * dens * (E - TC(0.5) * (uvel * uvel + vvel * vvel + wvel * wvel));
                     T Vn_new = uvel * nx + vvel * ny + wvel * nz;
                     vn_new = Vn_new;
@@ -1117,14 +1088,11 @@ __global__ void __launch_bounds__(256) k_lusgs_sl(const BlockDev *__restrict__ b
                     df[3] = (nw[3] * (Vn_new - Vn_e) + press_new * nz) - b.of[3];
                     df[4] = ((nw[4] + press_new) * (Vn_new - Vn_e) + press_new * Vn_e) - b.of[4];
                 }
-                T A[5], V[5];
+                T A[6] = {}, V[6] = {};
                 for (int c = 0; c < 5; ++c) {
-                    const T a = FWD ? (df[c] * sd + dqn[c] * b.cl) * TC(0.5) : (df[c] * sd - dqn[c] * b.cl) * TC(0.5);
-                    const T v = dqn[c] * (VISC ? b.lv : T(0));   // lamv * dQ, lamv = 0 on the inviscid path
-                    A[c] = use ? a : T(0);
-                    V[c] = use ? v : T(0);
+                    A[c] = FWD ? (df[c] * sd + dqn[c] * b.cl) * TC(0.5) : (df[c] * sd - dqn[c] * b.cl) * TC(0.5);
+                    if (VISC) V[c] = dqn[c] * b.lv;   // lamv * dQ
                 }
-                for (int c = 0; c < 5; ++c) { sA[d][c][lane] = A[c]; sV[d][c][lane] = V[c]; }
                 if constexpr (SA) {
                     // (nu~ + dnu~) Vn_new - nu~ Vn_old (source/LU_SGS_Marching.cpp:351-353); the
                     // FP32 operator writes it as nu~ dVn + dnu~ Vn_new
@@ -1137,105 +1105,188 @@ __global__ void __launch_bounds__(256) k_lusgs_sl(const BlockDev *__restrict__ b
                         const T ev_new = b.ev + dev;
                         dfe = ev_new * vn_new - b.ev * b.vn_old;
                     }
-                    const T a = FWD ? (dfe * sd + b.cl * dev) * TC(0.5) : (dfe * sd - b.cl * dev) * TC(0.5);
-                    sA[d][5][lane] = use ? a : T(0);
-                    sV[d][5][lane] = use ? b.lv * dev : T(0);
+                    A[5] = FWD ? (dfe * sd + b.cl * dev) * TC(0.5) : (dfe * sd - b.cl * dev) * TC(0.5);
+                    V[5] = b.lv * dev;
                 }
-                if (d == 0) {
-                    for (int c = 0; c < 5; ++c) sR[c][lane] = b.r[c];
-                    sR[5][lane] = b.a;
-                    if constexpr (SA) {
-                        sR[6][lane] = b.rev;
-                        sR[7][lane] = b.a2;
+                // a lane without this neighbour contributes zero (few steps have any)
+                if (__builtin_amdgcn_ballot_w64(!use))
+                    for (int c = 0; c < NC; ++c) {
+                        A[c] = use ? A[c] : T(0);
+                        if (VISC) V[c] = use ? V[c] : T(0);
                     }
+                for (int p = 0; p < 3; ++p) {
+                    if constexpr (kWide && VISC) sAV[d][p][lane] = Quad{A[2 * p], A[2 * p + 1], V[2 * p], V[2 * p + 1]};
+                    else sA[d][p][lane] = Pair{A[2 * p], A[2 * p + 1]};
+                    if constexpr (!kWide && VISC) sV[d][p][lane] = Pair{V[2 * p], V[2 * p + 1]};
                 }
-                bar();   // terms of step s are in LDS
-                issue_cross(bc, s + kCrossAhead);
-                issue_static(bn, s + kStaticAhead);
-                precompute(b1);
-                bar();   // dQ of step s is in LDS
             };
-            // b[u] serves step s0+u: static data issued kStaticAhead steps
-            // ahead (into the buffer the previous step has finished with), the
-            // upstream dQ kCrossAhead steps ahead.  The loop starts kStaticAhead idle
-            // steps early (every lane invalid) so that no load precedes it and
-            // every step runs the same code; nothing is in flight on entry.
+            // The loop starts kStaticAhead idle steps early (every lane idle) so
+            // that no load precedes it and every step runs the same code;
+            // nothing is in flight on entry.
+            // b[u] serves step s0 + u: its static data are issued kStaticAhead steps
+            // ahead, into the buffer the previous step has finished with
             RowPf<T> b[kRing] = {};
             __builtin_amdgcn_s_waitcnt(0);
             for (int s0 = kRowS0; s0 < send; s0 += kRing) {
 #pragma unroll
-                for (int u = 0; u < kRing; ++u)
-                    work(b[u], b[(u + 1) % kRing], b[(u + kCrossAhead) % kRing], b[(u + kStaticAhead) % kRing], s0 + u);
+                for (int u = 0; u < kRing; ++u) {
+                    chain(b[u], s0 + u);
+                    bar();   // terms of the step are in LDS
+                    issue_static(b[(u + kStaticAhead) % kRing], s0 + u + kStaticAhead);
+                    precompute(b[(u + 1) % kRing]);
+                    bar();   // dQ of the step is in LDS
+                }
             }
         };
-        if (wave == 0) {
-            dir_loop(Dir<0>());
-        } else if (wave == 1) {
-            dir_loop(Dir<1>());
-        } else if (wave == 2) {
-            dir_loop(Dir<2>());
-        } else {
-            // ---- combine wave (source/LU_SGS_Marching.cpp:155, 255)
+        // ---- mailbox wave: the upstream dQ of step s + 1 into the buffer that
+        // holds the dQ of step s
+        auto mail_loop = [&]() {
+            constexpr int NJ = TK * NC, NW = (TK + TJ) * NC;   // words: the j edge's, then the k edge's
+            gT<T> src[2];
+            int radd[2], first[2], count[2], dst[2];
+            for (int h = 0; h < 2; ++h) {
+                const int w = lane + 64 * h;
+                const bool onj = w < NJ;
+                const int v = onj ? w : w - NJ, c = onj ? v / TK : v / TJ, e = onj ? v % TK : v % TJ;
+                // the edge cell that needs the word
+                const int ej = onj ? (FWD ? 0 : TJ - 1) : e, ek = onj ? e : (FWD ? 0 : TK - 1);
+                const bool ok = w < NW && (onj ? tl.dep_j : tl.dep_k) >= 0 && tl.j0 + ej < nj && tl.k0 + ek < nk;
+                const int uslot = !ok ? slot : onj ? slot + (FWD ? -ntk : ntk) : slot + (FWD ? -1 : 1);
+                src[h] = (gT<T>)(mbox_base<T>(B, FWD) + (long)uslot * nr * kMboxRow) + (!ok ? 0 : onj ? v : kMboxJ + v);
+                radd[h] = FWD ? (onj ? TJ : TK) - 1 : 1 - (onj ? TJ : TK);
+                first[h] = (FWD ? ej : TJ - 1 - ej) + (FWD ? ek : TK - 1 - ek);
+                count[h] = ok ? ni : 0;
+                dst[h] = w < NW ? dqi(c, 64 + (onj ? e : TK + e)) : -1;
+            }
+            auto poll = [&](T x[2], int s) {
+                for (int h = 0; h < 2; ++h)
+                    x[h] = __hip_atomic_load(src[h] + (long)clampr(row_of(s) + radd[h]) * kMboxRow, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+            };
+            auto missing = [&](const T x[2], int s) {
+                bool m = false;
+                for (int h = 0; h < 2; ++h) m = m || ((unsigned)(s - first[h]) < (unsigned)count[h] && mbox_empty(x[h]));
+                return __builtin_amdgcn_ballot_w64(m) != 0;
+            };
+            // Row s + 1 is read as step s - 1 starts and goes to LDS as step s
+            // starts.  A read takes about as long as a step and its rest overlaps
+            // the direction waves; reading a step earlier keeps the tile a step
+            // further behind its neighbour, over some thirty tiles in a row, and
+            // reading later (between the barriers) holds up every step.
+            // Measured, forward sweep, FP64 / FP32: 1.05M-cell channel 321 / 248 us
+            // as here, 335 / 220 a step earlier, 410 / 305 later; 96x32x32 channel
+            // 111 / 82, 120 / 86, 112 / 87.
+            T x[2] = {};
+            __builtin_amdgcn_s_waitcnt(0);
+            for (int s = kRowS0; s < send; ++s) {
+                // bounded wait: a run-out sets the error word
+                long spins = 0;
+                while (missing(x, s + 1)) {
+                    poll(x, s + 1);
+                    if (++spins > (1L << 22)) { if (lane == 0) atomicExch(err, 1); break; }
+                }
+                T *to = sdq[s & 1];
+                for (int h = 0; h < 2; ++h)
+                    if (dst[h] >= 0) to[dst[h]] = x[h];
+                poll(x, s + 2);
+                bar();
+                bar();
+            }
+        };
+        // ---- combine waves (source/LU_SGS_Marching.cpp:155, 255): wave p takes the
+        // components 2p and 2p + 1
+        auto combine_loop = [&](auto pc) {
+            constexpr int p = decltype(pc)::value, C0 = 2 * p, N = NC - C0 < 2 ? NC - C0 : 2;
+            constexpr bool kNu = C0 + N > 5;   // with the nu~ one
             const gT<T> mbox = (gT<T>)(mbox_base<T>(B, FWD) + (long)slot * nr * kMboxRow);
             // downstream edges of this tile: the j edge (lanes tj = jl, word tk)
             // and the k edge (lanes tk = kl, word tj)
             const bool jedge = tj == (FWD ? TJ - 1 : 0), kedge = tk == (FWD ? TK - 1 : 0);
-            for (int s = kRowS0; s < send; ++s) {
-                int i;
-                const bool valid = cell_at(s, i);
-                const int ro = clampr(row_of(s));
-                T outv[NC];
-                bar();
-                if (valid) {
-                    const T alpha = sR[5][lane];
-                    T ra = T(0);
-                    if constexpr (kDeltaForm) ra = rcp_op(alpha);
-                    for (int c = 0; c < 5; ++c) {
-                        T v;
-                        if (FWD) {
-                            v = sR[c][lane] * TC(-1.0) + sA[0][c][lane];
-                            v = v + sA[1][c][lane]; v = v + sA[2][c][lane];
-                        } else {
-                            v = sR[c][lane] * alpha - sA[0][c][lane];
-                            v = v - sA[1][c][lane]; v = v - sA[2][c][lane];
-                        }
-                        v = v + sV[0][c][lane]; v = v + sV[1][c][lane]; v = v + sV[2][c][lane];
-                        if constexpr (kDeltaForm) outv[c] = v * ra;
-                        else outv[c] = v / alpha;
-                        sdq[s & 1][c][lane] = outv[c];
-                    }
-                    if constexpr (SA) {
-                        // source/LU_SGS_Marching.cpp:156-157, 256-257
-                        const T alpha2 = sR[7][lane];
-                        T v;
-                        if (FWD) {
-                            v = sR[6][lane] * TC(-1.0) + sA[0][5][lane];
-                            v = v + sA[1][5][lane]; v = v + sA[2][5][lane];
-                        } else {
-                            v = sR[6][lane] * alpha2 - sA[0][5][lane];
-                            v = v - sA[1][5][lane]; v = v - sA[2][5][lane];
-                        }
-                        v = v + sV[0][5][lane]; v = v + sV[1][5][lane]; v = v + sV[2][5][lane];
-                        if constexpr (kDeltaForm) outv[5] = v * rcp_op(alpha2);
-                        else outv[5] = v / alpha2;
-                        sdq[s & 1][5][lane] = outv[5];
-                    }
+            const int count = col ? ni : 0;
+            struct Rhs {
+                T r[2], a[2];   // right-hand side (backward: the forward dQ) and diagonal per component
+                T ra[2];        // reciprocals of the diagonals
+            };
+            auto issue = [&](Rhs &b, int step) {
+                const int ro = clampr(row_of(step));
+                const gcT<T> row = rows + (long)ro * RQ + lane, drow = (gcT<T>)drows + (long)ro * RD + lane;
+                for (int c = 0; c < N; ++c)
+                    b.r[c] = !FWD ? drow[(C0 + c) * 64] : C0 + c < 5 ? row[(kSQ_R + C0 + c) * 64] : row[kSQ_REV * 64];
+                b.a[0] = row[kSQ_A * 64];
+                if (kNu) b.a[1] = row[kSQ_A2 * 64];
+            };
+            // what does not depend on the step's terms
+            auto prepare = [&](Rhs &b) {
+                if (!kNu) b.a[1] = b.a[0];
+                b.ra[0] = recip(b.a[0]);
+                pin(b.ra[0]);
+                b.ra[1] = b.ra[0];
+                if (kNu) { b.ra[1] = recip(b.a[1]); pin(b.ra[1]); }
+                for (int c = 0; c < N; ++c) {
+                    b.r[c] = FWD ? b.r[c] * TC(-1.0) : b.r[c] * b.a[c];
+                    pin(b.r[c]);
                 }
-                bar();
-                if (valid) {
-                    // hand the edge values to the downstream tiles, then keep dQ
-                    if (jedge)
-                        for (int c = 0; c < NC; ++c)
-                            __hip_atomic_store(mbox + ro * kMboxRow + tk + c * TK, outv[c], __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                    if (kedge)
-                        for (int c = 0; c < NC; ++c)
-                            __hip_atomic_store(mbox + ro * kMboxRow + kMboxJ + tj + c * TJ, outv[c], __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                    for (int c = 0; c < NC; ++c) drows[ro * RD + c * 64 + lane] = outv[c];
+            };
+            Rhs b[kRing] = {};
+            __builtin_amdgcn_s_waitcnt(0);
+            for (int s0 = kRowS0; s0 < send; s0 += kRing) {
+#pragma unroll
+                for (int u = 0; u < kRing; ++u) {
+                    const int s = s0 + u;
+                    issue(b[(u + kStaticAhead) % kRing], s + kStaticAhead);
+                    prepare(b[u]);
+                    const bool valid = (unsigned)(s - lj - lk) < (unsigned)count;
+                    bar();
+                    Pair A[3], V[3];
+                    for (int d = 0; d < 3; ++d) {
+                        if constexpr (kWide && VISC) {
+                            const Quad v = sAV[d][p][lane];
+                            A[d] = Pair{v[0], v[1]};
+                            V[d] = Pair{v[2], v[3]};
+                        } else {
+                            A[d] = sA[d][p][lane];
+                            if constexpr (VISC) V[d] = sV[d][p][lane];
+                        }
+                    }
+                    T out[2];
+                    for (int c = 0; c < N; ++c) {
+                        T v = FWD ? b[u].r[c] + A[0][c] : b[u].r[c] - A[0][c];
+                        v = FWD ? v + A[1][c] : v - A[1][c];
+                        v = FWD ? v + A[2][c] : v - A[2][c];
+                        if constexpr (VISC) { v = v + V[0][c]; v = v + V[1][c]; v = v + V[2][c]; }
+                        if constexpr (kDeltaForm) out[c] = v * b[u].ra[c];
+                        else out[c] = DivBy(b[u].a[c], b[u].ra[c]).of(v);
+                    }
+                    if (valid) {
+                        T *to = sdq[s & 1] + dqi(C0, lane);
+                        if constexpr (N == 2) *(Pair *)to = Pair{out[0], out[1]};
+                        else *to = out[0];
+                    }
+                    bar();
+                    if (valid) {
+                        // hand the edge values to the downstream tiles, then keep dQ
+                        const int ro = row_of(s);
+                        const gT<T> mb = mbox + (long)ro * kMboxRow;
+                        if (jedge)
+                            for (int c = 0; c < N; ++c)
+                                __hip_atomic_store(mb + tk + (C0 + c) * TK, out[c], __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+                        if (kedge)
+                            for (int c = 0; c < N; ++c)
+                                __hip_atomic_store(mb + kMboxJ + tj + (C0 + c) * TJ, out[c], __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+                        for (int c = 0; c < N; ++c) drows[(long)ro * RD + (C0 + c) * 64 + lane] = out[c];
+                    }
                 }
             }
-        }
+        };
+        if (wave == 0) dir_loop(Int<0>());
+        else if (wave == 1) dir_loop(Int<1>());
+        else if (wave == 2) dir_loop(Int<2>());
+        else if (wave == 3) mail_loop();
+        else if (wave == 4) combine_loop(Int<0>());
+        else if (wave == 5) combine_loop(Int<1>());
+        else combine_loop(Int<2>());
     }
 }
 
