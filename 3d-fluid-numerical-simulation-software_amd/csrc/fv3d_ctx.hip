@@ -753,12 +753,12 @@ static int setup_sa(fv3d_ctx *c)
 
 // ------------------------------------------- scratch of fv3d_mlp_grad_noalloc
 // The partial gradients and losses of up to kNoAllocChunks 64-sample chunks
-// (8833 + 1 floats each) and the loss sum live in a file-scope device array,
+// (8833 + 1 floats each) live in a file-scope device array,
 // so fv3d_mlp_grad_noalloc allocates nothing.  Every GPU holds its own copy
 // (9 MB) until the process ends; host code uses only the per-device address
 // hipGetSymbolAddress returns, taken once per device at context creation.
 constexpr int kNoAllocChunks = 256;   // 16,384 samples
-constexpr long kNoAllocFloats = (long)kNoAllocChunks * (kMlpParams + 1) + 1;
+constexpr long kNoAllocFloats = (long)kNoAllocChunks * (kMlpParams + 1);
 static __device__ __align__(256) float scratch[kNoAllocFloats];
 constexpr int kNoAllocDevices = 64;
 static float *g_scratch_ptr[kNoAllocDevices];
@@ -775,11 +775,6 @@ static int noalloc_init(fv3d_ctx *c)
     if (e != hipSuccess || !p) return fail(c, FV3D_EHIP, "hipGetSymbolAddress(scratch): %s", hipGetErrorString(e));
     g_scratch_ptr[c->device] = (float *)p;
     return FV3D_OK;
-}
-
-__global__ void k_noalloc_loss(const float *__restrict__ sum, long n, float *__restrict__ loss)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) *loss = *sum / (float)n;
 }
 
 // ------------------------------------------------------------------ API
@@ -2698,14 +2693,19 @@ int fv3d_mlp_forward(fv3d_ctx *c, const float *x, long n, float *y)
 }
 
 // One gradient of the mean loss over samples [off, off + m) into d_mlp_g
-// (and the summed squared error into d_mlp_g[kMlpParams]).
-static void mlp_gradient(fv3d_ctx *c, const float *dx, const float *dt, long off, long m, float *dpart, float *dloss)
+// and the mean loss into loss_out; with adam the parameters' update too.
+static void mlp_gradient(fv3d_ctx *c, const float *dx, const float *dt, long off, long m, float *dpart, float *dloss,
+                         float *loss_out, const MlpAdam *adam)
 {
     const int nchunk = (int)((m + 63) / 64);
     hipLaunchKernelGGL(k_mlp_train_chunk, dim3((unsigned)nchunk), dim3(256), 0, c->stream, c->d_mlp, dx + off * kMlpIn,
                        dt + off, m, 1.0f / (float)m, dpart, dloss);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpParams + 1 + 255) / 256), dim3(256), 0, c->stream, dpart, dloss, nchunk,
-                       c->d_mlp_g, c->d_mlp_g + kMlpParams);
+    if (adam)
+        hipLaunchKernelGGL(k_mlp_reduce<true>, dim3(kMlpRedGroups), dim3(256), 0, c->stream, dpart, dloss, nchunk,
+                           c->d_mlp_g, loss_out, (float)m, *adam);
+    else
+        hipLaunchKernelGGL(k_mlp_reduce<false>, dim3(kMlpRedGroups), dim3(256), 0, c->stream, dpart, dloss, nchunk,
+                           c->d_mlp_g, loss_out, (float)m, MlpAdam{});
 }
 
 int fv3d_mlp_grad(fv3d_ctx *c, const float *x, const float *t, long n, float *grad, float *loss)
@@ -2719,7 +2719,7 @@ int fv3d_mlp_grad(fv3d_ctx *c, const float *x, const float *t, long n, float *gr
     if (!rc) rc = dalloc(c, &dpart, (size_t)nchunk * kMlpParams);
     if (!rc) rc = dalloc(c, &dloss, (size_t)nchunk);
     if (!rc) {
-        mlp_gradient(c, dx, dt, 0, n, dpart, dloss);
+        mlp_gradient(c, dx, dt, 0, n, dpart, dloss, c->d_mlp_g + kMlpParams, nullptr);
         std::vector<float> g(kMlpParams + 1);
         hipError_t e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -2727,7 +2727,7 @@ int fv3d_mlp_grad(fv3d_ctx *c, const float *x, const float *t, long n, float *gr
         if (e != hipSuccess) rc = fail(c, FV3D_EHIP, "mlp gradient: %s", hipGetErrorString(e));
         else {
             if (grad) std::copy(g.begin(), g.begin() + kMlpParams, grad);
-            if (loss) *loss = g[kMlpParams] / (float)n;
+            if (loss) *loss = g[kMlpParams];
         }
     }
     for (float *p : {dx, dt, dpart, dloss})
@@ -2747,13 +2747,12 @@ int fv3d_mlp_grad_noalloc(fv3d_ctx *c, const float *x_dev, const float *t_dev, l
     if (!s) return fail(c, FV3D_ESTATE, "scratch address of device %d not taken", c->device);
     // every chunk's partial gradient and loss is written before it is read, so
     // nothing in the scratch needs clearing between calls
-    float *part = s, *loss = s + (long)kNoAllocChunks * kMlpParams, *sum = s + kNoAllocFloats - 1;
+    float *part = s, *loss = s + (long)kNoAllocChunks * kMlpParams;
     const int nchunk = (int)((n + 63) / 64);
     hipLaunchKernelGGL(k_mlp_train_chunk, dim3((unsigned)nchunk), dim3(256), 0, c->stream, c->d_mlp, x_dev, t_dev, n,
                        1.0f / (float)n, part, loss);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((kMlpParams + 1 + 255) / 256), dim3(256), 0, c->stream, part, loss, nchunk,
-                       grad_dev, sum);
-    hipLaunchKernelGGL(k_noalloc_loss, dim3(1), dim3(64), 0, c->stream, sum, n, loss_dev);
+    hipLaunchKernelGGL(k_mlp_reduce<false>, dim3(kMlpRedGroups), dim3(256), 0, c->stream, part, loss, nchunk, grad_dev,
+                       loss_dev, (float)n, MlpAdam{});
     HIPCK(c, hipGetLastError());
     return FV3D_OK;
 }
@@ -2775,12 +2774,10 @@ int fv3d_mlp_train(fv3d_ctx *c, const float *x, const float *t, long n, int step
     for (int s = 0; s < steps && !rc; ++s) {
         // consecutive minibatches of the sample order, wrapping (the caller shuffles)
         const long off = (long)s * m % std::max<long>(1, n - m + 1);
-        mlp_gradient(c, dx, dt, off, m, dpart, dloss);
         ++c->mlp_step;
         const float c1 = 1.0f - powf(b1, (float)c->mlp_step), c2 = 1.0f - powf(b2, (float)c->mlp_step);
-        hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, c->stream, c->d_mlp, c->d_mlp_m,
-                           c->d_mlp_v, c->d_mlp_g, lr, b1, b2, eps, c1, c2);
-        HIPCK(c, hipMemcpyAsync(dhist + s, c->d_mlp_g + kMlpParams, sizeof(float), hipMemcpyDeviceToDevice, c->stream));
+        const MlpAdam adam{c->d_mlp, c->d_mlp_m, c->d_mlp_v, lr, b1, b2, eps, c1, c2};
+        mlp_gradient(c, dx, dt, off, m, dpart, dloss, dhist + s, &adam);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) rc = fail(c, FV3D_EHIP, "mlp training: %s", hipGetErrorString(e));
     }
@@ -2790,7 +2787,7 @@ int fv3d_mlp_train(fv3d_ctx *c, const float *x, const float *t, long n, int step
         if (e == hipSuccess) e = hipMemcpy(h.data(), dhist, steps * sizeof(float), hipMemcpyDeviceToHost);
         if (e != hipSuccess) rc = fail(c, FV3D_EHIP, "mlp training: %s", hipGetErrorString(e));
         else if (loss_hist)
-            for (int s = 0; s < steps; ++s) loss_hist[s] = h[s] / (float)m;
+            std::copy(h.begin(), h.end(), loss_hist);
     }
     for (float *p : {dx, dt, dpart, dloss, dhist})
         if (p) (void)hipFree(p);

@@ -31,8 +31,16 @@ __global__ void k_mlp_mut(const BlockDev *blocks, const long *cstart, int nblock
                           const float *xc, unsigned long long *tripped, double relax);
 __global__ void k_mlp_train_chunk(const float *P, const float *x, const float *tgt, long n, float inv_n, float *partial,
                                   float *loss);
-__global__ void k_mlp_reduce(const float *partial, const float *loss, int nchunk, float *grad, float *loss_sum);
-__global__ void k_mlp_adam(float *P, float *m, float *v, const float *grad, float lr, float b1, float b2, float eps,
-                           float c1, float c2);
+// the Adam update of a reduction that ends a training step: parameters, moments,
+// rate, decay rates, epsilon and the step's bias corrections
+struct MlpAdam {
+    float *P, *m, *v;
+    float lr, b1, b2, eps, c1, c2;
+};
+// launched with kMlpRedGroups workgroups
+constexpr int kMlpRedGroups = (kMlpParams + 1 + 63) / 64;
+template <bool ADAM>
+__global__ void k_mlp_reduce(const float *partial, const float *loss, int nchunk, float *grad, float *loss_out,
+                             float loss_div, MlpAdam A);
 
 }  // namespace fv3d
