@@ -82,8 +82,9 @@ __device__ inline void stream_face(BlockRef B, const Gas &g, int d, int i, int j
 
 template <int TJ, int TK, int MODE>
 __global__ void __launch_bounds__(TJ *TK) k_conv_stream(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles,
-                                                        int ntiles, int ci, Gas g)
+                                                        int ntiles, int ci, Gas g, int ndec)
 {
+    if (blockIdx.x == 0) flag_decrement(blocks, ndec);
     constexpr int NV = MODE == 2 ? 10 : 5;
     constexpr int NT = TJ * TK;
     __shared__ double ring[4][NV][TJ][TK];   // tile cells of planes p = i-1 .. i+2 (slot p & 3)
@@ -226,9 +227,9 @@ __global__ void __launch_bounds__(TJ *TK) k_conv_stream(const BlockDev *__restri
 }
 
 #define FV3D_STREAM(S, TJ, TK)                                                                            \
-    template __global__ void k_conv_stream<TJ, TK, 0>(const BlockDev *, const int4 *, int, int, Gas);     \
-    template __global__ void k_conv_stream<TJ, TK, 1>(const BlockDev *, const int4 *, int, int, Gas);     \
-    template __global__ void k_conv_stream<TJ, TK, 2>(const BlockDev *, const int4 *, int, int, Gas);
+    template __global__ void k_conv_stream<TJ, TK, 0>(const BlockDev *, const int4 *, int, int, Gas, int);     \
+    template __global__ void k_conv_stream<TJ, TK, 1>(const BlockDev *, const int4 *, int, int, Gas, int);     \
+    template __global__ void k_conv_stream<TJ, TK, 2>(const BlockDev *, const int4 *, int, int, Gas, int);
 FV3D_FOR_STREAM_TILES(FV3D_STREAM)
 #undef FV3D_STREAM
 

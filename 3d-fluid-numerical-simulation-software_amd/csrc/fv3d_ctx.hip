@@ -87,7 +87,7 @@ struct fv3d_ctx {
     int *d_pitch_sign = nullptr;
     std::vector<PatchDev> pd_host;   // the device patch list, host copy
     double *d_mbox = nullptr;         // sweep mailboxes of all blocks
-    long mbox_words = 0;
+    long mbox_fill = 0;               // their 16-byte words
     long *d_pack_start = nullptr;     // running pack (tile, chunk) item counts per block
     long pack_groups = 0;
     // Baldwin-Lomax: one launch per group size G (16, 32 or 64 cell groups per
@@ -125,16 +125,18 @@ struct fv3d_ctx {
     ScalarsDev *d_sc = nullptr;
     double *d_hist = nullptr;
     long hist_cap = 0;
-    double *d_stage_row = nullptr;   // history rows (one per instance) written by the captured graph
+    double **d_cursor = nullptr;     // where replayed iterations write their history (the finest level's)
+    int *d_arrived = nullptr;        // workgroups of k_finish done, per instance
     double *d_faces[3] = {nullptr, nullptr, nullptr};
     ViscDebug vdbg = {{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}, nullptr};
     int store_faces = 0;
     double total_vol = 0.0;
     // persistent wavefront sweep: tile lists (forward, backward) and the
-    // sync words [err, ticket_f, ticket_b, done_f[ntiles], done_b[ntiles]]
+    // words err, ticket_f, ticket_b, a cache line each
     KbaTile *d_kba[2] = {nullptr, nullptr};
     int nkba = 0;
     int *d_kba_sync = nullptr;
+    int *sweep_err = nullptr;    // the error word: the finest level's
     int sweep_mode = 4;   // 0 one launch per hyperplane (the reference's schedule, a cross-check),
                           // 4 the persistent wavefront on the tile-skewed row layout
     int kba_grid = 0;
@@ -842,7 +844,7 @@ int fv3d_ctx_destroy(fv3d_ctx *c)
     for (int q = 0; q < kNumStream; ++q)
         if (c->d_stiles[q]) (void)hipFree(c->d_stiles[q]);
     void *ps[] = {c->d_blocks, c->d_patches, c->d_pstart_bc, c->d_cstart, c->d_pstart_plane, c->d_secs,
-                  c->d_partial, c->d_sums, c->d_bad, c->d_flags, c->d_sc, c->d_hist, c->d_stage_row, c->d_kba[0], c->d_kba[1], c->d_kba_sync, c->d_faces[0], c->d_faces[1], c->d_faces[2]};
+                  c->d_partial, c->d_sums, c->d_bad, c->d_flags, c->d_sc, c->d_hist, c->parent ? nullptr : c->d_cursor, c->d_arrived, c->d_kba[0], c->d_kba[1], c->d_kba_sync, c->d_faces[0], c->d_faces[1], c->d_faces[2]};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     if (c->stream) {
@@ -1153,14 +1155,17 @@ int fv3d_setup(fv3d_ctx *c)
             words += 2 * b.sweep_rows * kMboxRow;
             gst.push_back(gst.back() + b.pack_groups);
         }
-        if ((rc = dalloc(c, &c->d_mbox, words))) return rc;
-        c->mbox_words = words;
+        // in doubles: a row of kMboxRow FP32 words takes half as many
+        static_assert(kMboxRow * 4 % 16 == 0, "rows of whole 16-byte words");
+        const long row = c->cfg.precision == FV3D_DEFECT_FP32 ? kMboxRow / 2 : kMboxRow;
+        if ((rc = dalloc(c, &c->d_mbox, words / kMboxRow * row))) return rc;
+        c->mbox_fill = words / kMboxRow * row / 2;
         long off = 0;
-        for (auto &b : c->blocks) {
-            b.dev.mbox[0] = c->d_mbox + off;
-            b.dev.mbox[1] = b.dev.mbox[0] + b.sweep_rows * kMboxRow;
-            off += 2 * b.sweep_rows * kMboxRow;
-        }
+        for (auto &b : c->blocks)
+            for (int dir = 0; dir < 2; ++dir) {
+                b.dev.mbox[dir] = c->d_mbox + off;
+                off += b.sweep_rows * row;
+            }
         c->pack_groups = gst.back();
         if ((rc = dalloc(c, &c->d_pack_start, gst.size()))) return rc;
         HIPCK(c, hipMemcpyAsync(c->d_pack_start, gst.data(), gst.size() * sizeof(long), hipMemcpyHostToDevice, c->stream));
@@ -1354,7 +1359,8 @@ int fv3d_setup(fv3d_ctx *c)
             HIPCK(c, hipMemcpyAsync(c->d_kba[dir], kt.data(), kt.size() * sizeof(KbaTile), hipMemcpyHostToDevice, c->stream));
         }
         c->nkba = (int)lst.size();
-        if ((rc = dalloc(c, &c->d_kba_sync, 64 + 2 * (size_t)c->nkba * kDonePad))) return rc;
+        if ((rc = dalloc(c, &c->d_kba_sync, 96))) return rc;
+        c->sweep_err = c->parent ? c->parent->sweep_err : c->d_kba_sync;
         c->kba_grid = std::min(c->nkba, 4096);
     }
     c->npart = (int)((c->ncell + 255) / 256);
@@ -1362,8 +1368,10 @@ int fv3d_setup(fv3d_ctx *c)
     if ((rc = dalloc(c, &c->d_parts, c->ninst))) return rc;
     HIPCK(c, hipMemcpyAsync(c->d_parts, c->parts_host.data(), c->ninst * sizeof(int2), hipMemcpyHostToDevice, c->stream));
     if (c->cfg.turbulence == 200 && (rc = setup_sa(c))) return rc;
-    if ((rc = dalloc(c, &c->d_sums, 2 * 3 * kSecParts * (size_t)c->ninst))) return rc;
-    if ((rc = dalloc(c, &c->d_stage_row, 7 * (size_t)c->ninst))) return rc;
+    if ((rc = dalloc(c, &c->d_sums, (2 * 3 * kSecParts + 6) * (size_t)c->ninst))) return rc;
+    if ((rc = dalloc(c, &c->d_arrived, c->ninst))) return rc;
+    if (c->parent) c->d_cursor = c->parent->d_cursor;
+    else if ((rc = dalloc(c, &c->d_cursor, 1))) return rc;
     // device scalars of each instance
     std::vector<ScalarsDev> scs(c->ninst);
     for (int w = 0; w < c->ninst; ++w) {
@@ -1626,19 +1634,19 @@ static int launch_spectral_dt(fv3d_ctx *c, bool decrement = true)
 // FP32 defect-correction form: lambda, dt and the LU-SGS diagonals it would form
 // are formed again by the level's next evaluation before anything reads them
 // (the restriction takes Q, R and the volumes), so only the Flag_low_dt
-// countdown at its end runs (source/TimeStep.cpp:89-92).  The plain FP64 path
-// forms them, as the reference's ResFlux does, so that they can be read after
-// an iteration.
+// countdown at its end runs (source/TimeStep.cpp:89-92), in the convective
+// launch.  The plain FP64 path forms them, as the reference's ResFlux does, so
+// that they can be read after an iteration.
 static int launch_restriction_timestep(fv3d_ctx *c)
 {
-    if (c->cfg.precision != FV3D_DEFECT_FP32) return launch_spectral_dt(c);
-    hipLaunchKernelGGL(k_dt_flag_decrement, dim3(1), dim3(256), 0, c->stream, c->d_blocks, (int)c->blocks.size());
-    HIPCK(c, hipGetLastError());
-    return FV3D_OK;
+    return c->cfg.precision == FV3D_DEFECT_FP32 ? FV3D_OK : launch_spectral_dt(c, false);
 }
 
-static int launch_convective(fv3d_ctx *c)
+// dec: the Flag_low_dt countdown of the time step before it (launch_spectral_dt
+// without decrement) runs in the same launch
+static int launch_convective(fv3d_ctx *c, bool dec = false)
 {
+    const int ndec = dec ? (int)c->blocks.size() : 0;
     // the reconstruction's variables (any code other than 100 and 200 is
     // characteristic, source/UserInput.cpp:117-130)
     const int mode = c->cfg.recon_var == 200 ? 0 : c->cfg.recon_var == 100 ? 1 : 2;
@@ -1650,7 +1658,7 @@ static int launch_convective(fv3d_ctx *c)
         else if (mode == 1) hipLaunchKernelGGL(k_conv_faces<1>, gf, dim3(256), 0, c->stream, c->d_blocks, c->d_fstart, 3 * nb, c->gas);
         else hipLaunchKernelGGL(k_conv_faces<2>, gf, dim3(256), 0, c->stream, c->d_blocks, c->d_fstart, 3 * nb, c->gas);
         hipLaunchKernelGGL(k_conv_sum, dim3((unsigned)((c->ncell + 255) / 256)), dim3(256), 0, c->stream, c->d_blocks,
-                           c->d_cstart, nb);
+                           c->d_cstart, nb, ndec);
         HIPCK(c, hipGetLastError());
         return FV3D_OK;
     }
@@ -1665,13 +1673,13 @@ static int launch_convective(fv3d_ctx *c)
     case S:                                                                                                         \
         if (mode == 0)                                                                                              \
             hipLaunchKernelGGL((k_conv_stream<TJ, TK, 0>), g, dim3(TJ * TK), 0, c->stream, c->d_blocks,             \
-                               c->d_stiles[q], nt, ci, c->gas);                                                     \
+                               c->d_stiles[q], nt, ci, c->gas, ndec);                                               \
         else if (mode == 1)                                                                                         \
             hipLaunchKernelGGL((k_conv_stream<TJ, TK, 1>), g, dim3(TJ * TK), 0, c->stream, c->d_blocks,             \
-                               c->d_stiles[q], nt, ci, c->gas);                                                     \
+                               c->d_stiles[q], nt, ci, c->gas, ndec);                                               \
         else                                                                                                        \
             hipLaunchKernelGGL((k_conv_stream<TJ, TK, 2>), g, dim3(TJ * TK), 0, c->stream, c->d_blocks,             \
-                               c->d_stiles[q], nt, ci, c->gas);                                                     \
+                               c->d_stiles[q], nt, ci, c->gas, ndec);                                               \
         break;
             FV3D_FOR_STREAM_TILES(FV3D_STREAM)
 #undef FV3D_STREAM
@@ -1686,7 +1694,7 @@ static int launch_convective(fv3d_ctx *c)
 #define FV3D_CONV_M(S, M, A, B, C)                                                                               \
     case 3 * S + M:                                                                                               \
         hipLaunchKernelGGL((k_convective<A, B, C, M>), g, b, 0, c->stream, c->d_blocks, c->d_tiles_s[q], c->gas,    \
-                           c->store_faces, c->d_faces[0], c->d_faces[1], c->d_faces[2]);                         \
+                           ndec, c->store_faces, c->d_faces[0], c->d_faces[1], c->d_faces[2]);                         \
         break;
 #define FV3D_CONV(S, A, B, C) FV3D_CONV_M(S, 0, A, B, C) FV3D_CONV_M(S, 1, A, B, C) FV3D_CONV_M(S, 2, A, B, C)
         FV3D_FOR_TILES(FV3D_CONV)
@@ -1834,10 +1842,8 @@ static void launch_sa_sweep(fv3d_ctx *c, bool fwd)
 
 static int launch_sweeps_kba(fv3d_ctx *c)
 {
-    // layout: err at 0, tickets at 32 and 48, padded counters from 64
-    long nsync = 64 + 2L * c->nkba * kDonePad - 32;
-    hipLaunchKernelGGL(k_fill_int, dim3((unsigned)((nsync + 255) / 256)), dim3(256), 0, c->stream, c->d_kba_sync + 32, nsync, 0);
-    int *err = c->d_kba_sync, *tf = c->d_kba_sync + 32, *tb = c->d_kba_sync + 48;
+    // layout: err at 0, tickets at 32 and 64
+    int *err = c->sweep_err, *tf = c->d_kba_sync + 32, *tb = c->d_kba_sync + 64;
     if (c->sweep_mode == 4) {
         const bool f32 = c->cfg.precision == FV3D_DEFECT_FP32;
         const bool visc = c->cfg.viscous;
@@ -1850,28 +1856,22 @@ static int launch_sweeps_kba(fv3d_ctx *c)
         const long per = c->pack_groups > 0 ? std::max(1L, (8192 + c->pack_groups - 1) / c->pack_groups) : 1;
         const int qs = (int)std::min<long>(nq, per), cs = (int)std::min<long>(ncomp, per);
         const unsigned pgq = (unsigned)(c->pack_groups * qs), pgc = (unsigned)(c->pack_groups * cs);
+        const unsigned pgf = (unsigned)((c->mbox_fill + kFillWords - 1) / kFillWords);
         if (f32) {
-            // FP32 words: fill every 32-bit word of the shared allocation
-            const long nw = 2 * c->mbox_words;
-            hipLaunchKernelGGL(k_fill_int, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, c->stream, (int *)c->d_mbox, nw,
-                               (int)kMboxEmpty32);
-            hipLaunchKernelGGL(k_sweep_pack<float>, dim3(pgq), dim3(256), 0, c->stream, c->d_blocks, c->d_pack_start, nb, nq,
-                               qs);
+            hipLaunchKernelGGL(k_sweep_pack<float>, dim3(pgq + pgf), dim3(256), 0, c->stream, c->d_blocks, c->d_pack_start,
+                               nb, nq, qs, pgq, (uint4 *)c->d_mbox, c->mbox_fill);
         } else {
-            const long nw = c->mbox_words;
-            hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((nw + 255) / 256)), dim3(256), 0, c->stream,
-                               (unsigned long long *)c->d_mbox, nw, kMboxEmpty);
-            hipLaunchKernelGGL(k_sweep_pack<double>, dim3(pgq), dim3(256), 0, c->stream, c->d_blocks, c->d_pack_start, nb, nq,
-                               qs);
+            hipLaunchKernelGGL(k_sweep_pack<double>, dim3(pgq + pgf), dim3(256), 0, c->stream, c->d_blocks, c->d_pack_start,
+                               nb, nq, qs, pgq, (uint4 *)c->d_mbox, c->mbox_fill);
         }
         // forward and backward sweeps in the operator's precision, with or
         // without the viscous terms
         auto sweep = [&](bool fwd) {
-            int *tk = fwd ? tf : tb;
+            int *tk = fwd ? tf : tb, *nt = fwd ? tb : tf;
             const KbaTile *tl = c->d_kba[fwd ? 0 : 1];
             dim3 g((unsigned)c->kba_grid), b(kSlThreads);
 #define FV3D_SL_LAUNCH(F, V, S, T) \
-    hipLaunchKernelGGL((k_lusgs_sl<F, kKbaTJ, kKbaTK, V, S, T>), g, b, 0, c->stream, c->d_blocks, tl, c->nkba, tk, err, \
+    hipLaunchKernelGGL((k_lusgs_sl<F, kKbaTJ, kKbaTK, V, S, T>), g, b, 0, c->stream, c->d_blocks, tl, c->nkba, tk, nt, err, \
                        c->gas.relax, c->gas)
 #define FV3D_SL_FORMS(F, T)                      \
     do {                                         \
@@ -1948,13 +1948,12 @@ static int launch_update(fv3d_ctx *c)
     return FV3D_OK;
 }
 
-static int launch_finalize(fv3d_ctx *c, double *hist_row)
+// hist_row null: the cursor's next row (replayed iterations)
+static int launch_finish(fv3d_ctx *c, double *hist_row)
 {
-    hipLaunchKernelGGL(k_sections, dim3(2 * kSecParts * c->ninst), dim3(256), 0, c->stream, c->d_blocks, c->d_secs, c->gas,
-                       c->d_sums);
-    HIPCK(c, hipGetLastError());
-    hipLaunchKernelGGL(k_finalize, dim3(c->ninst), dim3(256), 0, c->stream, c->d_partial, c->npart, c->d_parts, c->d_sums,
-                       c->d_sc, c->ramp_sc, c->gas, hist_row);
+    hipLaunchKernelGGL(k_finish, dim3((unsigned)(kFinParts * c->ninst)), dim3(256), 0, c->stream, c->d_blocks, c->d_secs,
+                       c->d_partial, c->npart, c->d_parts, c->d_sums, c->d_arrived, c->d_sc, c->ramp_sc, c->gas, hist_row,
+                       c->d_cursor, c->ninst);
     HIPCK(c, hipGetLastError());
     return FV3D_OK;
 }
@@ -1982,20 +1981,21 @@ int fv3d_resflux(fv3d_ctx *c)
     int rc;
     if ((rc = launch_bc(c))) return rc;
     if ((rc = launch_turbulence(c))) return rc;
-    if ((rc = launch_spectral_dt(c))) return rc;
-    if ((rc = launch_convective(c))) return rc;
+    if ((rc = launch_spectral_dt(c, false))) return rc;
+    if ((rc = launch_convective(c, true))) return rc;
     return launch_viscous(c);
 }
 
 // The wavefront sweep bounds every wait; a wait that ran out sets the error
 // word instead of hanging the device.
+// The error word of the sweeps, one for all grid levels.
 static int check_sweep_error(fv3d_ctx *c)
 {
     int e = 0;
-    HIPCK(c, hipMemcpy(&e, c->d_kba_sync, sizeof(int), hipMemcpyDeviceToHost));
+    HIPCK(c, hipMemcpy(&e, c->sweep_err, sizeof(int), hipMemcpyDeviceToHost));
     if (e) {
         int z = 0;
-        HIPCK(c, hipMemcpy(c->d_kba_sync, &z, sizeof(int), hipMemcpyHostToDevice));
+        HIPCK(c, hipMemcpy(c->sweep_err, &z, sizeof(int), hipMemcpyHostToDevice));
         return fail(c, FV3D_ESTATE, "wavefront sweep: a progress wait exceeded its bound");
     }
     return FV3D_OK;
@@ -2009,9 +2009,9 @@ static int lusgs_timed(fv3d_ctx *c)
     if (c->timing) HIPCK(c, hipEventRecord(c->ev[10], c->stream));
     if ((rc = launch_turbulence(c, 1))) return rc;
     if (c->timing) HIPCK(c, hipEventRecord(c->ev[11], c->stream));
-    if ((rc = launch_spectral_dt(c))) return rc;
+    if ((rc = launch_spectral_dt(c, false))) return rc;
     if (c->timing) HIPCK(c, hipEventRecord(c->ev[1], c->stream));
-    if ((rc = launch_convective(c))) return rc;
+    if ((rc = launch_convective(c, true))) return rc;
     if (c->timing) HIPCK(c, hipEventRecord(c->ev[12], c->stream));
     if ((rc = launch_viscous(c))) return rc;
     if (c->timing) HIPCK(c, hipEventRecord(c->ev[2], c->stream));
@@ -2142,8 +2142,8 @@ static int level_resflux(fv3d_ctx *c, bool restriction_only = false)
     int rc;
     if ((rc = launch_bc(c))) return rc;
     if ((rc = launch_turbulence(c))) return rc;
-    if ((rc = restriction_only ? launch_restriction_timestep(c) : launch_spectral_dt(c))) return rc;
-    if ((rc = launch_convective(c))) return rc;
+    if ((rc = restriction_only ? launch_restriction_timestep(c) : launch_spectral_dt(c, false))) return rc;
+    if ((rc = launch_convective(c, true))) return rc;
     return launch_viscous(c);
 }
 
@@ -2194,7 +2194,7 @@ static int mg_iteration(fv3d_ctx *c, int phase, double *row)
             HIPCK(c, hipGetLastError());
             if ((rc = launch_limiter(c))) return rc;
         }
-        return launch_finalize(m, row);
+        return launch_finish(m, row);
     }
     if ((rc = lusgs_timed(c))) return rc;
     // the fine residual at the new state, for the restriction (the coarse
@@ -2202,7 +2202,7 @@ static int mg_iteration(fv3d_ctx *c, int phase, double *row)
     if ((rc = launch_bc(c))) return rc;
     if ((rc = launch_turbulence(c, 0, true))) return rc;
     if ((rc = launch_restriction_timestep(c))) return rc;
-    if ((rc = launch_convective(c))) return rc;
+    if ((rc = launch_convective(c, true))) return rc;
     if ((rc = launch_viscous(c))) return rc;
     if (m->coarse) {
         // N-level V-cycle: the levels below take the full approximation storage form
@@ -2220,7 +2220,7 @@ static int mg_iteration(fv3d_ctx *c, int phase, double *row)
     HIPCK(c, hipGetLastError());
     if ((rc = launch_limiter(c))) return rc;
     if (c->timing) HIPCK(c, hipEventRecord(c->ev[9], c->stream));
-    return launch_finalize(c, row);
+    return launch_finish(c, row);
 }
 
 static int mg_phase(const fv3d_ctx *c, long it)
@@ -2302,12 +2302,11 @@ int fv3d_iteration_end(fv3d_ctx *c, double *row7)
     const long itn = c->iter_host + 1;
     // the coarse start-up iterations report the coarse level (source/Solver.cpp:71-87)
     fv3d_ctx *r = c->ng == 2 && mg_phase(c, itn) != kMgCycle ? c->coarse : c;
-    if ((rc = launch_finalize(r, c->d_hist))) return rc;
+    if ((rc = launch_finish(r, c->d_hist))) return rc;
     c->iter_host = itn;
     if (row7) HIPCK(c, hipMemcpyAsync(row7, c->d_hist, 7L * c->ninst * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCK(c, hipStreamSynchronize(c->stream));
     if ((rc = check_sweep_error(c))) return rc;
-    if (c->coarse && (rc = check_sweep_error(c->coarse))) return fail(c, rc, "coarse level: %s", c->coarse->err.c_str());
     return FV3D_OK;
 }
 
@@ -2381,7 +2380,7 @@ int fv3d_iterate(fv3d_ctx *c, int n, double *hist)
         } else {
             if ((rc = lusgs_timed(c))) return rc;
             if (c->timing) HIPCK(c, hipEventRecord(c->ev[9], c->stream));
-            if ((rc = launch_finalize(c, row))) return rc;
+            if ((rc = launch_finish(c, row))) return rc;
         }
         c->iter_host = itn;
         if (c->timing && timed) {
@@ -2393,7 +2392,6 @@ int fv3d_iterate(fv3d_ctx *c, int n, double *hist)
         HIPCK(c, hipMemcpyAsync(hist, c->d_hist, 7L * n * c->ninst * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCK(c, hipStreamSynchronize(c->stream));
     if ((rc = check_sweep_error(c))) return rc;
-    if (c->coarse && (rc = check_sweep_error(c->coarse))) return fail(c, rc, "coarse level: %s", c->coarse->err.c_str());
     if (hist && n > 0)
         for (int w = 0; w < c->ninst; ++w)
             if (!isfinite(hist[7L * (c->ninst * (n - 1L) + w) + 1]))
@@ -2413,11 +2411,11 @@ int fv3d_iterate_graph(fv3d_ctx *c, int n, double *hist)
                                     "file the reference's cycle divides by coarse time steps it never computed");
     if (c->cfg.turbulence == 200 && !c->ev_set)
         return fail(c, FV3D_ESTATE, "Spalart-Allmaras needs nu~: fv3d_nut_upload for every block, or fv3d_initial");
-    // each graph writes its history row into a fixed staging slot that is
-    // copied into the history buffer after each replay; with two levels the
+    // each replay writes the cursor's next history row; with two levels the
     // coarse start-up phase and the cycle have a graph each, and the one
     // iteration between them (Coarse_iter) runs eagerly
-    double *stage_row = c->d_stage_row;
+    hipLaunchKernelGGL(k_hist_begin, dim3(1), dim3(64), 0, c->stream, c->d_cursor, c->d_hist, c->ramp_sc, c->ninst);
+    HIPCK(c, hipGetLastError());
     auto capture = [&](hipGraphExec_t *exec, int phase) -> int {
         if (*exec) return FV3D_OK;
         hipGraph_t g;
@@ -2426,10 +2424,10 @@ int fv3d_iterate_graph(fv3d_ctx *c, int n, double *hist)
         HIPCK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
         int r;
         if (c->ng == 2) {
-            r = mg_iteration(c, phase, stage_row);
+            r = mg_iteration(c, phase, nullptr);
         } else {
             r = lusgs_timed(c);
-            if (!r) r = launch_finalize(c, stage_row);
+            if (!r) r = launch_finish(c, nullptr);
         }
         hipError_t e = hipStreamEndCapture(c->stream, &g);
         c->timing = saved;
@@ -2443,21 +2441,18 @@ int fv3d_iterate_graph(fv3d_ctx *c, int n, double *hist)
         const long itn = c->iter_host + 1;
         const int phase = c->ng == 2 ? mg_phase(c, itn) : kMgCycle;
         if (phase == kMgSwitch) {
-            if ((rc = mg_iteration(c, phase, stage_row))) return rc;
+            if ((rc = mg_iteration(c, phase, nullptr))) return rc;
         } else {
             hipGraphExec_t *exec = phase == kMgCoarse ? &c->graph_coarse : &c->graph_exec;
             if ((rc = capture(exec, phase))) return rc;
             HIPCK(c, hipGraphLaunch(*exec, c->stream));
         }
-        HIPCK(c, hipMemcpyAsync(c->d_hist + 7L * c->ninst * it, stage_row, 7L * c->ninst * sizeof(double),
-                                hipMemcpyDeviceToDevice, c->stream));
         c->iter_host = itn;
     }
     if (hist && n > 0)
         HIPCK(c, hipMemcpyAsync(hist, c->d_hist, 7L * n * c->ninst * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCK(c, hipStreamSynchronize(c->stream));
     if ((rc = check_sweep_error(c))) return rc;
-    if (c->coarse && (rc = check_sweep_error(c->coarse))) return fail(c, rc, "coarse level: %s", c->coarse->err.c_str());
     if (hist && n > 0)
         for (int w = 0; w < c->ninst; ++w)
             if (!isfinite(hist[7L * (c->ninst * (n - 1L) + w) + 1]))

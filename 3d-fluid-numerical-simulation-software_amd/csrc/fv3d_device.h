@@ -92,8 +92,9 @@ struct BlockDev {
     int nr;                   // rows per tile = ni + kKbaTJ + kKbaTK - 2
     // Edge mailboxes of the row-layout sweeps (forward, backward): per tile
     // row, the dQ of the lanes a downstream tile reads across the j edge
-    // (5 x kKbaTK) and across the k edge (5 x kKbaTJ).  Reset to a sentinel
-    // before each iteration; a consumer waits until its words are not it.
+    // (5 x kKbaTK) and across the k edge (5 x kKbaTJ), in the sweep's precision.
+    // Reset to a sentinel before each iteration; a consumer waits until its
+    // words are not it.
     double *mbox[2];
     // coarse level of the two-grid cycle (null elsewhere): the restricted state
     // cv_2h and the restricted residual Res_2h, 5*box each
@@ -570,6 +571,18 @@ __device__ inline void wall_face_core(double Gamma, const double wa[5], const do
     out[2] = c2 * (Vn_a - Vn_e) + fp * Sy;
     out[3] = c3 * (Vn_a - Vn_e) + fp * Sz;
     out[4] = (c4 + fp) * (Vn_a - Vn_e) + fp * Vn_e;
+}
+
+// Decrement of the time-step damping counters of blocks 0 .. nblock - 1 at the
+// end of CTimeDiscr::TimeStep (source/TimeStep.cpp:89-92), after every cell has
+// read them, by the threads of one workgroup.  The convective kernel that follows
+// the time step does it (ndec, else 0), which saves a launch.
+__device__ inline void flag_decrement(const BlockDev *blocks, int nblock)
+{
+    for (int n = threadIdx.x; n < nblock; n += blockDim.x) {
+        int *f = block_at(blocks, n).flag_low_dt;
+        if (*f > 0) *f = *f - 1;
+    }
 }
 
 }  // namespace fv3d

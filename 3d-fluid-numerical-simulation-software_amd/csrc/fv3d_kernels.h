@@ -66,6 +66,7 @@ struct ScalarsDev {
     double mass_in, mass_out, pr, eff;
     double p_out;
     double iter;
+    long hist_pos;      // history rows written since k_hist_begin
 };
 
 struct PeriodicDev;
@@ -105,12 +106,12 @@ __global__ void k_spectral_dt(const BlockDev *blocks, const long *cstart, int nb
 __global__ void k_dt_flag_decrement(const BlockDev *blocks, int nblock);
 // MODE: the reconstruction's variables, 0 primitive, 1 conservative, 2 characteristic
 template <int TI, int TJ, int TK, int MODE>
-__global__ void k_convective(const BlockDev *blocks, const int4 *tiles, Gas g, int store_faces, double *fI, double *fJ,
-                             double *fK);
+__global__ void k_convective(const BlockDev *blocks, const int4 *tiles, Gas g, int ndec, int store_faces, double *fI,
+                             double *fJ, double *fK);
 // fstart: running face counts per (block, direction), 3 * nblock entries + 1
 template <int MODE>
 __global__ void k_conv_faces(const BlockDev *blocks, const long *fstart, int nlist, Gas g);
-__global__ void k_conv_sum(const BlockDev *blocks, const long *cstart, int nblock);
+__global__ void k_conv_sum(const BlockDev *blocks, const long *cstart, int nblock, int ndec);
 template <bool FORWARD>
 __global__ void k_lusgs_plane(const BlockDev *blocks, const long *pstart, int nblock, int step, double relax, Gas g);
 // one tile of the persistent wavefront sweep; dep_*: ticket of the upstream
@@ -119,7 +120,6 @@ struct KbaTile {
     int block, j0, k0, dep_j, dep_k;
 };
 constexpr int kKbaTJ = 4, kKbaTK = 16;
-constexpr int kDonePad = 32;   // progress counters one per 128-byte line
 // quantities of a sweep-layout row (BlockDev::srow): Q (5), p, lamc (3),
 // swg (15), R (5), alpha, lamv (3, Navier-Stokes only), and with
 // Spalart-Allmaras nu~, its residual and its LU-SGS diagonal alpha2
@@ -135,8 +135,8 @@ constexpr int kSlThreads = 448;
 // T: double (plain FP64) or float (the FP32 operator of defect correction)
 // SA: the nu~ equation in the same sweep (Navier-Stokes only)
 template <bool FWD, int TJ, int TK, bool VISC, bool SA, class T>
-__global__ void k_lusgs_sl(const BlockDev *blocks, const KbaTile *tiles, int ntiles, int *ticket, int *err, double relax,
-                           Gas g);
+__global__ void k_lusgs_sl(const BlockDev *blocks, const KbaTile *tiles, int ntiles, int *ticket, int *next_ticket,
+                           int *err, double relax, Gas g);
 // mailbox words per tile row (kSweepD components of the j-edge lanes, then of
 // the k-edge lanes), and the bit pattern of an empty word (a NaN payload no
 // arithmetic produces)
@@ -153,8 +153,12 @@ __global__ void k_sweep_fill(const BlockDev *blocks, int block, long nrows, int 
 // serve block n, each split over qsplit workgroups (a grid of
 // gstart[nblock] * qsplit) that take equal shares of the nq quantities (15;
 // 18 with lamv; 21 with the nu~ rows, when nu~ is carried in the sweep)
+// Workgroups from npack on fill the nfill 16-byte words of mbox with the empty
+// pattern, kFillWords each.
+constexpr int kFillWords = 2048;
 template <class T>
-__global__ void k_sweep_pack(const BlockDev *blocks, const long *gstart, int nblock, int nq, int qsplit);
+__global__ void k_sweep_pack(const BlockDev *blocks, const long *gstart, int nblock, int nq, int qsplit, unsigned npack,
+                             uint4 *mbox, long nfill);
 // nc: components per cell (5, or 6 with the nu~ increment), split over csplit
 // workgroups per item
 template <class T>
@@ -165,17 +169,21 @@ __global__ void k_fill_int(int *p, long n, int v);
 __global__ void k_update(const BlockDev *blocks, const long *cstart, int nblock, Gas g, double *partial, int *bad_flag,
                          int *sa_hi, int sa);
 template <int TJ, int TK, int MODE>
-__global__ void k_conv_stream(const BlockDev *blocks, const int4 *tiles, int ntiles, int ci, Gas g);
+__global__ void k_conv_stream(const BlockDev *blocks, const int4 *tiles, int ntiles, int ci, Gas g, int ndec);
 __global__ void k_limiter_serial(const BlockDev *blocks, int nblock, Gas g, int *bad_flag, const long *cstart,
                                  double *partial, int npart);
 __global__ void k_sections(const BlockDev *blocks, const int2 *secs, Gas g, double *sums);
 // norms and section integrals of one level (lv) with the CFL ramp and the
 // iteration count kept in ramp (the fine level's scalars, shared by the
-// levels); one workgroup per instance w: its norm partials are
-// parts[w].x .. parts[w].x + parts[w].y - 1, its scalars lv[w] and ramp[w],
-// its history row hist_row + 7 w
-__global__ void k_finalize(const double *partial, int npart, const int2 *parts, const double *sums, ScalarsDev *lv,
-                           ScalarsDev *ramp, Gas g, double *hist_row);
+// levels); kFinParts workgroups per instance w: its norm partials are
+// parts[w].x .. parts[w].x + parts[w].y - 1, its scalars lv[w] and ramp[w], its
+// history row hist_row + 7 w, or the cursor's next one.  sums: the section
+// partials of every instance, then six norms each; arrived: zero between launches
+constexpr int kFinParts = 2 * kSecParts + 6;
+__global__ void k_finish(const BlockDev *blocks, const int2 *secs, const double *partial, int npart, const int2 *parts,
+                         double *sums, int *arrived, ScalarsDev *lv, ScalarsDev *ramp, Gas g, double *hist_row,
+                         double *const *cursor, int ninst);
+__global__ void k_hist_begin(double **cursor, double *hist, ScalarsDev *ramp, int ninst);
 // two-grid cycle (CSolver::Prolong / Interpolate, CMesh::CornerTreatment,
 // ComputeForceFunction / AddForceFunction)
 __global__ void k_mg_restrict(const BlockDev *fine, const BlockDev *coarse, const long *cstart, int nblock, Gas g,

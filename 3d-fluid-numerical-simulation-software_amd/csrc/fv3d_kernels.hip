@@ -364,15 +364,8 @@ __global__ void k_spectral_dt(const BlockDev *__restrict__ blocks, const long *_
     });
 }
 
-// Decrement of the time-step damping counter at the end of CTimeDiscr::TimeStep
-// (source/TimeStep.cpp:89-92), after every cell has read it.
-__global__ void k_dt_flag_decrement(const BlockDev *__restrict__ blocks, int nblock)
-{
-    for (int n = threadIdx.x; n < nblock; n += blockDim.x) {
-        int *f = blocks[n].flag_low_dt;
-        if (*f > 0) *f = *f - 1;
-    }
-}
+// As a launch of its own for a TimeStep that no convective residual follows.
+__global__ void k_dt_flag_decrement(const BlockDev *__restrict__ blocks, int nblock) { flag_decrement(blocks, nblock); }
 
 // =================================================== convective residual
 // Face flux of CSpaceDiscr::Upwind_Convective (source/Upwind_Convective.cpp:5-360)
@@ -449,9 +442,10 @@ __device__ static void face_flux(BlockRef B, const Gas &g, int d, int i, int j, 
 // keeps three).
 template <int TI, int TJ, int TK, int MODE>
 __global__ void __launch_bounds__(TI *TJ *TK) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 3 : 4)))
-k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles, Gas g, int store_faces, double *fI0,
-             double *fJ0, double *fK0)
+k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles, Gas g, int ndec, int store_faces,
+             double *fI0, double *fJ0, double *fK0)
 {
+    if (blockIdx.x == 0) flag_decrement(blocks, ndec);
     constexpr int NFI = (TI + 1) * TJ * TK, NFJ = TI * (TJ + 1) * TK, NFK = TI * TJ * (TK + 1);
     constexpr int GI = (NFI + 63) / 64, GJ = (NFJ + 63) / 64, GK = (NFK + 63) / 64;   // groups per direction
     __shared__ double sI[5][TI + 1][TJ][TK];
@@ -513,7 +507,8 @@ k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles
 }
 
 #define FV3D_CONV_M(M, A, B, C) \
-    template __global__ void k_convective<A, B, C, M>(const BlockDev *, const int4 *, Gas, int, double *, double *, double *);
+    template __global__ void k_convective<A, B, C, M>(const BlockDev *, const int4 *, Gas, int, int, double *, double *, \
+                                                      double *);
 #define FV3D_CONV(S, A, B, C) FV3D_CONV_M(0, A, B, C) FV3D_CONV_M(1, A, B, C) FV3D_CONV_M(2, A, B, C)
 FV3D_FOR_TILES(FV3D_CONV)
 #undef FV3D_CONV
@@ -546,8 +541,9 @@ template __global__ void k_conv_faces<1>(const BlockDev *, const long *, int, Ga
 template __global__ void k_conv_faces<2>(const BlockDev *, const long *, int, Gas);
 
 __global__ void __launch_bounds__(256) k_conv_sum(const BlockDev *__restrict__ blocks, const long *__restrict__ cstart,
-                                                  int nblock)
+                                                  int nblock, int ndec)
 {
+    if (blockIdx.x == 0) flag_decrement(blocks, ndec);
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     int n, i, j, k;
     if (!cell_item(blocks, cstart, nblock, t, n, i, j, k)) return;
@@ -702,13 +698,9 @@ __device__ inline float recip(float x) { return rcp_op(x); }
 // whether a mailbox word still holds the empty pattern
 __device__ inline bool mbox_empty(double x) { return __builtin_bit_cast(unsigned long long, x) == kMboxEmpty; }
 __device__ inline bool mbox_empty(float x) { return __builtin_bit_cast(unsigned int, x) == kMboxEmpty32; }
-// the mailbox set of a sweep direction, in words of T (both sets share one
-// allocation whose second half starts at mbox[1])
+// the mailbox set of a sweep direction
 template <class T>
-__device__ inline T *mbox_base(BlockRef B, bool fwd)
-{
-    return (T *)B.mbox[0] + (fwd ? 0 : (B.mbox[1] - B.mbox[0]));
-}
+__device__ inline T *mbox_base(BlockRef B, bool fwd) { return (T *)B.mbox[fwd ? 0 : 1]; }
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -779,15 +771,27 @@ __device__ inline void pack_item(BlockRef B, long wg, int nchunk, int &slot, int
 // spreads over the chip.  The chunk's cells are read plane by plane along k
 // (coalesced) into LDS, then written out row by row: the rows a chunk touches
 // are partly written (the lanes whose cell lies in the chunk), each as one
-// contiguous run.
+// contiguous run.  The workgroups after the first npack empty the sweeps'
+// mailboxes, kFillWords 16-byte words each (a launch of its own before; having
+// the sweeps' readers put the pattern back was tried: it cost the FP32 sweeps
+// 10 %, more than this).
 template <class T>
 __global__ void __launch_bounds__(256) k_sweep_pack(const BlockDev *__restrict__ blocks, const long *__restrict__ gstart,
-                                                    int nblock, int nq, int qsplit)
+                                                    int nblock, int nq, int qsplit, unsigned npack,
+                                                    uint4 *__restrict__ mbox, long nfill)
 {
     constexpr int TJ = kKbaTJ, TK = kKbaTK;
     __shared__ double buf[kPackChunk][64];
+    if (blockIdx.x >= npack) {
+        const unsigned lo = (unsigned)kMboxEmpty, hi = (unsigned)(kMboxEmpty >> 32);
+        const uint4 v = sizeof(T) == 4 ? make_uint4(kMboxEmpty32, kMboxEmpty32, kMboxEmpty32, kMboxEmpty32)
+                                       : make_uint4(lo, hi, lo, hi);
+        const long w0 = (long)(blockIdx.x - npack) * kFillWords, w1 = min(w0 + kFillWords, nfill);
+        for (long w = w0 + threadIdx.x; w < w1; w += 256) mbox[w] = v;
+        return;
+    }
     // the block of this workgroup: gstart holds the running (tile, chunk) counts
-    const long item = xcd_item(blockIdx.x, gridDim.x);
+    const long item = xcd_item(blockIdx.x, npack);
     const int qg = (int)(item % qsplit);
     const int block = find_range(gstart, nblock, item / qsplit);
     BlockRef B = block_at(blocks, block);
@@ -870,8 +874,8 @@ __global__ void __launch_bounds__(256) k_sweep_unpack(const BlockDev *__restrict
 
 template __global__ void k_sweep_fill<double>(const BlockDev *, int, long, int);
 template __global__ void k_sweep_fill<float>(const BlockDev *, int, long, int);
-template __global__ void k_sweep_pack<double>(const BlockDev *, const long *, int, int, int);
-template __global__ void k_sweep_pack<float>(const BlockDev *, const long *, int, int, int);
+template __global__ void k_sweep_pack<double>(const BlockDev *, const long *, int, int, int, unsigned, uint4 *, long);
+template __global__ void k_sweep_pack<float>(const BlockDev *, const long *, int, int, int, unsigned, uint4 *, long);
 template __global__ void k_sweep_unpack<double>(const BlockDev *, const long *, int, int, int);
 template __global__ void k_sweep_unpack<float>(const BlockDev *, const long *, int, int, int);
 
@@ -904,7 +908,8 @@ template __global__ void k_sweep_unpack<float>(const BlockDev *, const long *, i
 //
 // Across a tile edge dQ travels through the upstream tile's mailbox: its
 // combine waves store the dQ of its edge lanes there as soon as they have them;
-// a word that still holds the empty pattern has not been written.  Tiles
+// a word that still holds the empty pattern has not been written (k_sweep_pack
+// empties them).  Tiles
 // start in ticket order, so every upstream tile is already running.
 //
 // With SA the nu~ equation of Spalart-Allmaras rides along as a sixth
@@ -915,7 +920,8 @@ template __global__ void k_sweep_unpack<float>(const BlockDev *, const long *, i
 // order.
 template <bool FWD, int TJ, int TK, bool VISC, bool SA, class T>
 __global__ void __launch_bounds__(kSlThreads) k_lusgs_sl(const BlockDev *__restrict__ blocks, const KbaTile *__restrict__ tiles,
-                                                         int ntiles, int *__restrict__ ticket, int *__restrict__ err,
+                                                         int ntiles, int *__restrict__ ticket,
+                                                         int *__restrict__ next_ticket, int *__restrict__ err,
                                                          double relax, Gas g)
 {
     static_assert(TJ * TK == 64, "64 cells per tile");
@@ -945,6 +951,8 @@ __global__ void __launch_bounds__(kSlThreads) k_lusgs_sl(const BlockDev *__restr
     const int tj = lane / TK, tk = lane % TK;
     const T Gamma = (T)g.gamma;
     constexpr int RQ = kSweepQ * 64, RD = kSweepD * 64;   // words per row
+    // the other direction's tickets, whose sweep runs next
+    if (blockIdx.x == 0 && threadIdx.x == 0) *next_ticket = 0;
     for (;;) {
         if (threadIdx.x == 0) s_q = atomicAdd(ticket, 1);
         __syncthreads();
@@ -1291,7 +1299,7 @@ __global__ void __launch_bounds__(kSlThreads) k_lusgs_sl(const BlockDev *__restr
 }
 
 #define FV3D_SL(F, V, S, T) \
-    template __global__ void k_lusgs_sl<F, kKbaTJ, kKbaTK, V, S, T>(const BlockDev *, const KbaTile *, int, int *, int *, double, Gas);
+    template __global__ void k_lusgs_sl<F, kKbaTJ, kKbaTK, V, S, T>(const BlockDev *, const KbaTile *, int, int *, int *, int *, double, Gas);
 FV3D_SL(true, false, false, double)
 FV3D_SL(false, false, false, double)
 FV3D_SL(true, true, false, double)
@@ -1460,15 +1468,12 @@ __global__ void k_limiter_serial(const BlockDev *__restrict__ blocks, int nblock
 
 // ============================================= section integrals, norms
 // Mass flow, mass-averaged total pressure and total temperature over one K
-// plane (source/Ouput.cpp:9-95).  One workgroup per section, fixed-order tree
-// reduction; sums[sec*5 + {mass, ptm, ttm}].
-// grid: 2 x kSecParts workgroups; workgroup p of a section sums the cells
-// p*256 + t, (p + kSecParts)*256 + t, ... into sums[(sec*kSecParts + p)*3 + c]
-__global__ void __launch_bounds__(256) k_sections(const BlockDev *__restrict__ blocks, const int2 *__restrict__ secs, Gas g,
-                                                  double *__restrict__ sums)
+// plane (source/Ouput.cpp:9-95): workgroup `part` of section sec sums the cells
+// part*256 + t, (part + kSecParts)*256 + t, ... with a fixed-order tree into
+// sums[(sec*kSecParts + part)*3 + {mass, ptm, ttm}].
+__device__ static void section_part(const BlockDev *__restrict__ blocks, const int2 *__restrict__ secs, const Gas &g,
+                                    double *__restrict__ sums, int sec, int part, double (*red)[256])
 {
-    __shared__ double red[3][256];
-    const int sec = blockIdx.x / kSecParts, part = blockIdx.x % kSecParts;
     const int2 sc = secs[sec];
     BlockRef B = block_at(blocks, sc.x);
     const int K = sc.y;
@@ -1497,62 +1502,97 @@ __global__ void __launch_bounds__(256) k_sections(const BlockDev *__restrict__ b
         __syncthreads();
     }
     if (threadIdx.x == 0)
-        for (int c = 0; c < 3; ++c) sums[blockIdx.x * 3 + c] = red[c][0];
+        for (int c = 0; c < 3; ++c) sums[(sec * kSecParts + part) * 3 + c] = red[c][0];
 }
 
-// Residual norm (fixed-order sum of the per-workgroup partials), performance
-// parameters (source/Ouput.cpp:97-107,282-300), CFL ramp for the next iteration
-// (source/Solver.cpp:49-60) and the history row.  One workgroup.
-__global__ void __launch_bounds__(256) k_finalize(const double *__restrict__ partial, int npart, const int2 *__restrict__ parts,
-                                                  const double *__restrict__ secsum, ScalarsDev *lv, ScalarsDev *ramp, Gas g,
-                                                  double *__restrict__ hist_row)
+__global__ void __launch_bounds__(256) k_sections(const BlockDev *__restrict__ blocks, const int2 *__restrict__ secs, Gas g,
+                                                  double *__restrict__ sums)
 {
-    const int inst = blockIdx.x;
+    __shared__ double red[3][256];
+    section_part(blocks, secs, g, sums, blockIdx.x / kSecParts, blockIdx.x % kSecParts, red);
+}
+
+// The end of an iteration, kFinParts workgroups per instance: the section
+// integrals' parts, and one workgroup per component of the residual norm (the
+// fixed-order sum of the update's per-workgroup partials); the instance's last
+// workgroup to finish then forms the norms, the performance parameters
+// (source/Ouput.cpp:97-107,282-300), the CFL ramp for the next iteration
+// (source/Solver.cpp:49-60) and the history row, hist_row or, without it, the
+// cursor's next one.  As two launches, the second with one workgroup per
+// instance, this took 53 us on a 2.54M-cell passage and 12 on the smallest
+// grids, and a copy of the row 4.5 more.
+__global__ void __launch_bounds__(256) k_finish(const BlockDev *__restrict__ blocks, const int2 *__restrict__ secs,
+                                                const double *__restrict__ partial, int npart,
+                                                const int2 *__restrict__ parts, double *__restrict__ secsum,
+                                                int *__restrict__ arrived, ScalarsDev *lv, ScalarsDev *ramp, Gas g,
+                                                double *__restrict__ hist_row, double *const *__restrict__ cursor,
+                                                int ninst)
+{
+    __shared__ double red[3][256];
+    __shared__ int s_last;
+    const int inst = blockIdx.x / kFinParts, part = blockIdx.x % kFinParts;
+    const int t = threadIdx.x;
     ScalarsDev *sc = lv + inst;
     ramp += inst;
-    secsum += (long)inst * 2 * kSecParts * 3;
-    if (hist_row) hist_row += 7L * inst;
-    const int p0 = parts[inst].x, np = parts[inst].y;
+    double *norms = secsum + (long)ninst * 2 * kSecParts * 3 + 6 * inst;
     // component 5: Res_ev of Spalart-Allmaras (k_sa_res)
     const int nc = g.turbulence == 200 ? 6 : 5;
-    __shared__ double red[6][256];
-    double r[6] = {0, 0, 0, 0, 0, 0};
-    // each thread adds partials p = t, t + 256, ... in that order; eight of
-    // them are loaded before the first is added, so a thread waits on memory
-    // once per eight rather than once per partial (d_partial holds six
-    // components, so the sixth is always in bounds)
-    int p = threadIdx.x;
-    for (; p + 7 * 256 < np; p += 8 * 256) {
-        double v[8][6];
+    if (part < 2 * kSecParts) {
+        section_part(blocks, secs, g, secsum, inst * 2 + part / kSecParts, part % kSecParts, red);
+    } else {
+        const int c = part - 2 * kSecParts;
+        double r = 0.0;
+        if (c < nc) {
+            // each thread adds partials t, t + 256, ... in that order; sixteen
+            // loads are in flight before the first is added
+            const double *src = partial + (long)c * npart + parts[inst].x;
+            const int np = parts[inst].y;
+            int p = t;
+            for (; p + 15 * 256 < np; p += 16 * 256) {
+                double v[16];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+                for (int u = 0; u < 16; ++u) v[u] = src[p + u * 256];
 #pragma unroll
-            for (int c = 0; c < 6; ++c) v[u][c] = partial[(long)c * npart + p0 + p + u * 256];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-            for (int c = 0; c < 6; ++c)
-                if (c < nc) r[c] += v[u][c];
-    }
-    for (; p < np; p += 256)
-        for (int c = 0; c < nc; ++c) r[c] += partial[(long)c * npart + p0 + p];
-    for (int c = 0; c < 6; ++c) red[c][threadIdx.x] = r[c];
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int c = 0; c < 6; ++c) red[c][threadIdx.x] += red[c][threadIdx.x + w];
+                for (int u = 0; u < 16; ++u) r += v[u];
+            }
+            for (; p < np; p += 256) r += src[p];
+        }
+        red[0][t] = r;
         __syncthreads();
+        for (int w = 128; w > 0; w >>= 1) {
+            if (t < w) red[0][t] += red[0][t + w];
+            __syncthreads();
+        }
+        if (t == 0) norms[c] = red[0][0];
     }
-    if (threadIdx.x != 0) return;
-    for (int c = 0; c < 5; ++c) sc->res[c] = red[c][0] / sc->total_vol;
-    sc->res_ev = red[5][0] / sc->total_vol;
+    // what this workgroup wrote (thread 0) is visible before it counts itself in
+    if (t == 0) {
+        __threadfence();
+        s_last = atomicAdd(arrived + inst, 1) == kFinParts - 1;
+        if (s_last) __threadfence();
+    }
+    __syncthreads();
+    if (!s_last) return;
+    // section partials in a fixed order: section 0 inlet, 1 outlet; mass, ptm,
+    // ttm; then the norms
+    const double *own = secsum + (long)inst * 2 * kSecParts * 3;
+    if (t < 2 * kSecParts * 3)
+        red[0][t] = __hip_atomic_load(own + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else if (t < 2 * kSecParts * 3 + 6)
+        red[0][t] = __hip_atomic_load(norms + t - 2 * kSecParts * 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (t < 6) {
+        double s = 0.0;
+        for (int p = 0; p < kSecParts; ++p) s += red[0][((t / 3) * kSecParts + p) * 3 + t % 3];
+        red[1][t] = s;
+    }
+    __syncthreads();
+    if (t != 0) return;
+    arrived[inst] = 0;
+    const double *norm = &red[0][2 * kSecParts * 3], *sums = red[1];
+    for (int c = 0; c < 5; ++c) sc->res[c] = norm[c] / sc->total_vol;
+    sc->res_ev = norm[5] / sc->total_vol;
     const double Gamma = g.gamma, Rgas = g.rgas;
-    // section partials in a fixed order: section 0 inlet, 1 outlet; mass, ptm, ttm
-    double sums[6] = {0, 0, 0, 0, 0, 0};
-    for (int sec = 0; sec < 2; ++sec)
-        for (int p = 0; p < kSecParts; ++p)
-            for (int c = 0; c < 3; ++c) sums[sec * 3 + c] += secsum[(sec * kSecParts + p) * 3 + c];
-    // sums: section 0 inlet, section 1 outlet: mass, ptm, ttm
     double mi = sums[0] * sc->dens_ref * sc->vel_ref * sc->nblade_in;
     double mo = sums[3] * sc->dens_ref * sc->vel_ref * sc->nblade_out;
     double pti = pow(sums[1] / sums[0], Gamma / (Gamma - F32C(1.0))) * sc->dens_ref * sc->vel_ref * sc->vel_ref;
@@ -1562,6 +1602,12 @@ __global__ void __launch_bounds__(256) k_finalize(const double *__restrict__ par
     double L_adk = Gamma / (Gamma - F32C(1.0)) * Rgas * tti * (pow(PR, (Gamma - F32C(1.0)) / Gamma) - F32C(1.0));
     double L_k = Gamma / (Gamma - F32C(1.0)) * Rgas * tti * (tto / tti - F32C(1.0));
     ramp->iter += 1;
+    if (!hist_row) {
+        if (cursor) hist_row = *cursor + 7L * ((long)ramp->hist_pos * ninst + inst);
+        ramp->hist_pos += 1;
+    } else {
+        hist_row += 7L * inst;
+    }
     if (hist_row) {
         hist_row[0] = ramp->iter; hist_row[1] = sc->res[0]; hist_row[2] = mi; hist_row[3] = mo;
         hist_row[4] = PR; hist_row[5] = L_adk / L_k; hist_row[6] = ramp->cfl;
@@ -1574,6 +1620,13 @@ __global__ void __launch_bounds__(256) k_finalize(const double *__restrict__ par
         ramp->cfl_res = ramp->cfl_res / F32C(10.0);
     }
     if (ramp->cfl > F32C(10.0)) ramp->cfl = F32C(10.0);
+}
+
+// A run of replayed iterations starts: its history goes to hist from row 0.
+__global__ void k_hist_begin(double **cursor, double *hist, ScalarsDev *ramp, int ninst)
+{
+    if (threadIdx.x == 0) *cursor = hist;
+    for (int w = threadIdx.x; w < ninst; w += blockDim.x) ramp[w].hist_pos = 0;
 }
 
 // ============================================================ mixing plane
