@@ -131,6 +131,9 @@ struct fv3d_ctx {
     ViscDebug vdbg = {{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}, nullptr};
     int store_faces = 0;
     double total_vol = 0.0;
+    // fv3d_field_download's staging: the rows of a field, at most kFetchBytes at a time
+    double *d_fetch = nullptr;
+    long fetch_words = 0;
     // persistent wavefront sweep: tile lists (forward, backward) and the
     // words err, ticket_f, ticket_b, a cache line each
     KbaTile *d_kba[2] = {nullptr, nullptr};
@@ -185,6 +188,8 @@ struct fv3d_ctx {
     double t_ms[FV3D_TIMING_SLOTS] = {};
     long t_n[FV3D_TIMING_SLOTS] = {};
 };
+
+constexpr long kFetchBytes = 16L << 20;
 
 static int fail(fv3d_ctx *c, int code, const char *fmt, ...)
 {
@@ -844,7 +849,7 @@ int fv3d_ctx_destroy(fv3d_ctx *c)
     for (int q = 0; q < kNumStream; ++q)
         if (c->d_stiles[q]) (void)hipFree(c->d_stiles[q]);
     void *ps[] = {c->d_blocks, c->d_patches, c->d_pstart_bc, c->d_cstart, c->d_pstart_plane, c->d_secs,
-                  c->d_partial, c->d_sums, c->d_bad, c->d_flags, c->d_sc, c->d_hist, c->parent ? nullptr : c->d_cursor, c->d_arrived, c->d_kba[0], c->d_kba[1], c->d_kba_sync, c->d_faces[0], c->d_faces[1], c->d_faces[2]};
+                  c->d_partial, c->d_sums, c->d_bad, c->d_flags, c->d_sc, c->d_hist, c->parent ? nullptr : c->d_cursor, c->d_arrived, c->d_fetch, c->d_kba[0], c->d_kba[1], c->d_kba_sync, c->d_faces[0], c->d_faces[1], c->d_faces[2]};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     if (c->stream) {
@@ -1370,6 +1375,10 @@ int fv3d_setup(fv3d_ctx *c)
     if (c->cfg.turbulence == 200 && (rc = setup_sa(c))) return rc;
     if ((rc = dalloc(c, &c->d_sums, (2 * 3 * kSecParts + 6) * (size_t)c->ninst))) return rc;
     if ((rc = dalloc(c, &c->d_arrived, c->ninst))) return rc;
+    long box = 0;
+    for (const HostBlock &b : c->blocks) box = std::max(box, b.dev.box);
+    c->fetch_words = std::min(kFetchBytes / (long)sizeof(double), 12 * box);
+    if ((rc = dalloc(c, &c->d_fetch, c->fetch_words))) return rc;
     if (c->parent) c->d_cursor = c->parent->d_cursor;
     else if ((rc = dalloc(c, &c->d_cursor, 1))) return rc;
     // device scalars of each instance
@@ -2895,33 +2904,28 @@ long fv3d_field_download(fv3d_ctx *c, int block, const char *name, double *out)
     if (!name || !out) return FV3D_EINVAL;
     if (block < 1 || block > (int)c->blocks.size()) return fail(c, FV3D_EINVAL, "block %d", block);
     const BlockDev &B = c->blocks[block - 1].dev;
-    HIPCK(c, hipStreamSynchronize(c->stream));
-    auto fetch = [&](const double *src, long n, std::vector<double> &dst) -> int {
-        dst.resize(n);
-        HIPCK(c, hipMemcpy(dst.data(), src, n * sizeof(double), hipMemcpyDeviceToHost));
-        return 0;
-    };
-    std::vector<double> h;
-    long cnt = 0;
     std::string nm(name);
+    // cells lo .. lo + n - 1 along each direction of a box array of C components,
+    // interleaved on the device and copied straight to the caller's buffer
+    auto read = [&](const double *src, int C, int lo, int n1, int n2, int n3) -> long {
+        const long cells = (long)n1 * n2 * n3, chunk = c->fetch_words / C;
+        for (long t0 = 0; t0 < cells; t0 += chunk) {
+            const long n = std::min(chunk, cells - t0);
+            hipLaunchKernelGGL(k_field_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, src, B.box, C,
+                               B.si, B.sj, lo, n2, n3, t0, n, c->d_fetch);
+            HIPCK(c, hipGetLastError());
+            HIPCK(c, hipMemcpyAsync(out + t0 * C, c->d_fetch, (size_t)n * C * sizeof(double), hipMemcpyDeviceToHost,
+                                    c->stream));
+            HIPCK(c, hipStreamSynchronize(c->stream));
+        }
+        return cells * C;
+    };
     if (nm == "mut" || nm == "ev") {
         const double *p = nm == "mut" ? B.mut : B.ev;
         if (!p) return fail(c, FV3D_EINVAL, "%s exists with %s only", name, nm == "mut" ? "a turbulence model" : "Spalart-Allmaras");
-        if (fetch(p, B.box, h)) return FV3D_EHIP;
-        for (int i = 0; i <= B.IM; ++i)
-            for (int j = 0; j <= B.JM; ++j)
-                for (int k = 0; k <= B.KM; ++k) out[cnt++] = h[cidx(B, i, j, k)];
-        return cnt;
+        return read(p, 1, 0, B.IM + 1, B.JM + 1, B.KM + 1);
     }
-    if (nm == "cv" || nm == "pv") {
-        int C = nm == "cv" ? 5 : 6;
-        if (fetch(nm == "cv" ? B.Q : B.W, C * B.box, h)) return FV3D_EHIP;
-        for (int i = 0; i <= B.IM; ++i)
-            for (int j = 0; j <= B.JM; ++j)
-                for (int k = 0; k <= B.KM; ++k)
-                    for (int q = 0; q < C; ++q) out[cnt++] = h[q * B.box + cidx(B, i, j, k)];
-        return cnt;
-    }
+    if (nm == "cv" || nm == "pv") return read(nm == "cv" ? B.Q : B.W, nm == "cv" ? 5 : 6, 0, B.IM + 1, B.JM + 1, B.KM + 1);
     const double *src = nullptr;
     int C = 0, hiI = 0, hiJ = 0, hiK = 0;
     if (nm == "res") { src = B.R; C = 5; }
@@ -2952,20 +2956,16 @@ long fv3d_field_download(fv3d_ctx *c, int block, const char *name, double *out)
         if (!p) return fail(c, FV3D_ESTATE, "viscous fluxes were not captured (Navier-Stokes and fv3d_set_debug)");
         src = p; C = nm[0] == 'g' ? 12 : 5; hiI = d == 0; hiJ = d == 1; hiK = d == 2;
     }
-    if (src) {
-        if (fetch(src, (long)C * B.box, h)) return FV3D_EHIP;
-        for (int i = 1; i <= B.ni + hiI; ++i)
-            for (int j = 1; j <= B.nj + hiJ; ++j)
-                for (int k = 1; k <= B.nk + hiK; ++k)
-                    for (int q = 0; q < C; ++q) out[cnt++] = h[q * B.box + cidx(B, i, j, k)];
-        return cnt;
-    }
+    if (src) return read(src, C, 1, B.ni + hiI, B.nj + hiJ, B.nk + hiK);
     static const char *dn[6] = {"dIS", "dIP", "dJS", "dJP", "dKS", "dKP"};
     for (int s = 0; s < 6; ++s) {
         if (nm.compare(0, 3, dn[s]) != 0) continue;
         bool pvq = nm.size() > 3 && nm.substr(3) == "_pv";
         int C2 = pvq ? 6 : 5, c0 = pvq ? 5 : 0;
-        if (fetch(B.D[s], 22 * B.Dt[s], h)) return FV3D_EHIP;
+        std::vector<double> h(22 * B.Dt[s]);
+        long cnt = 0;
+        HIPCK(c, hipStreamSynchronize(c->stream));
+        HIPCK(c, hipMemcpy(h.data(), B.D[s], h.size() * sizeof(double), hipMemcpyDeviceToHost));
         int d = s / 2;
         int ra = d == 0 ? 2 : B.ni, rb = d == 0 ? B.nj : d == 1 ? 2 : B.nj, rc = d == 2 ? 2 : B.nk;
         for (int a = 1; a <= ra; ++a)

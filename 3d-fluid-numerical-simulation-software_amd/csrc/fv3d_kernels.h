@@ -166,6 +166,8 @@ __global__ void k_sweep_unpack(const BlockDev *blocks, const long *gstart, int n
 constexpr int kPackChunk = 16;   // i-planes per k_sweep_pack / k_sweep_unpack workgroup
 constexpr int kSecParts = 32;    // workgroups per section in k_sections
 __global__ void k_fill_int(int *p, long n, int v);
+__global__ void k_field_rows(const double *src, long box, int C, int si, int sj, int lo, int n2, int n3, long t0, long n,
+                             double *out);
 __global__ void k_update(const BlockDev *blocks, const long *cstart, int nblock, Gas g, double *partial, int *bad_flag,
                          int *sa_hi, int sa);
 template <int TJ, int TK, int MODE>
