@@ -129,6 +129,7 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
     const int t = threadIdx.x;
     const SaConst K;
     const double Re = g.re_ref;
+    const DivBy byRe(Re);
     for (int n = t; n < NH; n += NT) {
         const int hk = n % TL::HK, hj = (n / TL::HK) % TL::HJ, hi = n / (TL::HK * TL::HJ);
         const int ci = min(tl.y + hi, B.IM), cj = min(tl.z + hj, B.JM), ck = min(tl.w + hk, B.KM);
@@ -144,17 +145,10 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
         sw[6 * NH + n] = interior ? sa_clip(ev, T, rho, g) : ev;
     }
     __syncthreads();
-    for (int f = t; f < TL::NF; f += NT) {
-        int D, a, b, c;
-        if (f < TL::NFI) {
-            D = 0; c = f % TK; b = (f / TK) % TJ; a = f / (TK * TJ);
-        } else if (f < TL::NFI + TL::NFJ) {
-            const int r = f - TL::NFI;
-            D = 1; c = r % TK; b = (r / TK) % (TJ + 1); a = r / (TK * (TJ + 1));
-        } else {
-            const int r = f - TL::NFI - TL::NFJ;
-            D = 2; c = r % (TK + 1); b = (r / (TK + 1)) % TJ; a = r / ((TK + 1) * TJ);
-        }
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    for (int gq = wave; gq < TL::NG; gq += NT / 64) {
+        int D, a, b, c, f;
+        if (!TL::face(gq, t & 63, D, a, b, c, f)) continue;
         const int i = tl.y + a + 1, j = tl.z + b + 1, k = tl.w + c + 1;
         const bool ok = i <= B.ni + (D == 0) && j <= B.nj + (D == 1) && k <= B.nk + (D == 2);
         if (!ok) continue;
@@ -180,7 +174,8 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
         const double tz = (F32C(1.0) + K.Cb2) / K.sigma * (ev_lam + evf) * gz;
         const double *S = B.fS[D];
         const double Sx = S[x], Sy = S[box + x], Sz = S[2 * box + x], s = B.fs[D][x];
-        const double nx = Sx / s, ny = Sy / s, nz = Sz / s;
+        const DivBy bys(s);
+        const double nx = bys.of(Sx), ny = bys.of(Sy), nz = bys.of(Sz);
         const double Vn1 = sw[lm] * nx + sw[NH + lm] * ny + sw[2 * NH + lm] * nz;
         const double Vn2 = sw[l] * nx + sw[NH + l] * ny + sw[2 * NH + l] * nz;
         double fc = (F32C(0.5) * (Vn1 + fabs(Vn1)) * sw[6 * NH + lm] + F32C(0.5) * (Vn2 - fabs(Vn2)) * sw[6 * NH + l]) * s;
@@ -193,7 +188,7 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
             if (wm && wm[(long)ta * B.Db[side] + tb]) fc = 0;
         }
         sf[f] = fc;
-        sf[TL::NF + f] = (tx * Sx + ty * Sy + tz * Sz) / Re;
+        sf[TL::NF + f] = byRe.of(tx * Sx + ty * Sy + tz * Sz);
         sf[2 * TL::NF + f] = gx * Sx + gy * Sy + gz * Sz;
     }
     __syncthreads();

@@ -15,7 +15,22 @@ struct VTile {
     static constexpr int HI = TI + 2, HJ = TJ + 2, HK = TK + 2, NH = HI * HJ * HK;
     static constexpr int NFI = (TI + 1) * TJ * TK, NFJ = TI * (TJ + 1) * TK, NFK = TI * TJ * (TK + 1);
     static constexpr int NF = NFI + NFJ + NFK;
+    // groups of 64 faces of one direction, so that a wave evaluates one
+    // direction's faces at a time
+    static constexpr int GI = (NFI + 63) / 64, GJ = (NFJ + 63) / 64, NG = GI + GJ + (NFK + 63) / 64;
     __device__ static int h(int a, int b, int c) { return (a * HJ + b) * HK + c; }
+    // face `lane` of group q: its direction (wave-uniform), place in the tile and
+    // number among all faces (I faces, then J, then K); false past the last one
+    __device__ static bool face(int q, int lane, int &D, int &a, int &b, int &c, int &f)
+    {
+        D = q < GI ? 0 : q < GI + GJ ? 1 : 2;
+        const int r = (q - (D == 0 ? 0 : D == 1 ? GI : GI + GJ)) * 64 + lane;
+        if (D == 0) { c = r % TK; b = r / TK % TJ; a = r / (TK * TJ); }
+        else if (D == 1) { c = r % TK; b = r / TK % (TJ + 1); a = r / (TK * (TJ + 1)); }
+        else { c = r % (TK + 1); b = r / (TK + 1) % TJ; a = r / ((TK + 1) * TJ); }
+        f = r + (D == 0 ? 0 : D == 1 ? NFI : NFI + NFJ);
+        return a < TI + (D == 0);
+    }
 };
 
 // Gradients of u v w T at the face of direction D whose higher-index cell is
@@ -25,7 +40,11 @@ struct VTile {
 // lower and higher of D and t), summed in that order.  A cell outside the
 // block along both D and t (a never-filled ghost-box corner) is left out and
 // the other three averaged; at the J face j == JM, k == 1 the reference also
-// scales the lower three-cell sum by 0.25 (line 331).
+// scales the lower three-cell sum by 0.25 (line 331).  Such corners lie on the
+// block's edges only; a wave none of whose faces is at one takes the plain
+// four-cell averages: a third of the instructions of the general rule (with the
+// direction-uniform groups k_viscous 411 -> 329 us on a 2.54M-cell passage, 75 -> 58
+// on a 307k-cell one, the nu~ residual about 25 us less).
 template <int D, class TL, int NV = 4>
 __device__ inline void face_dv(const double *sw, int l, int i, int j, int k, BlockRef B, double dv[3][NV])
 {
@@ -36,13 +55,37 @@ __device__ inline void face_dv(const double *sw, int l, int i, int j, int k, Blo
     const int lD = l - st[D];
 #pragma unroll
     for (int q = 0; q < NV; ++q) dv[D][q] = sw[q * NH + l] - sw[q * NH + lD];
+    // offsets (along D, along t) of the four cells of each average
+    const int pD[4] = {0, 0, -1, -1}, pT[4] = {0, 1, 1, 0};
+    const int mf[4] = {0, -1, -1, 0}, ms[4] = {0, 0, -1, -1};
+    bool edge = false;
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+        if (t != D) edge = edge || pos[t] == 1 || pos[t] == lim[t];
+    const bool corner = edge && (pos[D] == 1 || pos[D] == lim[D] + 1);
+    if (__builtin_amdgcn_ballot_w64(corner) == 0) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            if (t == D) continue;
+            const bool lower = D < t;
+#pragma unroll
+            for (int q = 0; q < NV; ++q) {
+                const double *v = sw + q * NH + l;
+                double up = v[0], lo = v[0];
+#pragma unroll
+                for (int m = 1; m < 4; ++m) {
+                    up = up + v[pD[m] * st[D] + pT[m] * st[t]];
+                    lo = lo + v[(lower ? mf[m] : ms[m]) * st[D] + (lower ? ms[m] : mf[m]) * st[t]];
+                }
+                dv[t][q] = up / F32C(4.0) - lo / F32C(4.0);
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
         if (t == D) continue;
-        const int f = D < t ? D : t, s = D < t ? t : D;
-        // offsets (along D, along t) of the four cells of each average
-        const int pD[4] = {0, 0, -1, -1}, pT[4] = {0, 1, 1, 0};
-        const int mf[4] = {0, -1, -1, 0}, ms[4] = {0, 0, -1, -1};
+        const int f = D < t ? D : t;
         double avg[2][NV];
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {

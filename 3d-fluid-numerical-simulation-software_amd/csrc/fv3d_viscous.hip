@@ -132,12 +132,13 @@ __device__ static void face_fv(const double *sw, int l, int i, int j, int k, Blo
     const double wf = F32C(0.5) * (sw[2 * NH + l] + sw[2 * NH + l - st]);
     const double tf = F32C(0.5) * (sw[3 * NH + l] + sw[3 * NH + l - st]);
     const double mue_lam = sutherland(g, tf);
-    const double cond_lam = mue_lam * Gamma * Rgas / (Gamma - F32C(1.0)) / g.pr_lam;
+    const DivBy byg(Gamma - F32C(1.0));
+    const double cond_lam = DivBy(g.pr_lam).of(byg.of(mue_lam * Gamma * Rgas));
     double mue_tur = 0.0, cond_tur = 0.0;
     if (g.turbulence) {
         // face average of the eddy viscosity (source/ViscousFlux.cpp:59-62)
         mue_tur = (B.mut[x - (D == 0 ? B.si : D == 1 ? B.sj : 1)] + B.mut[x]) / F32C(2.0);
-        cond_tur = mue_tur * Gamma * Rgas / (Gamma - F32C(1.0)) / g.pr_tur;
+        cond_tur = DivBy(g.pr_tur).of(byg.of(mue_tur * Gamma * Rgas));
     }
     const double mue = mue_lam + mue_tur, cond = cond_lam + cond_tur;
     const double c43 = (double)(4.0f / 3.0f), c23 = (double)(2.0f / 3.0f);
@@ -189,17 +190,10 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_viscous(const BlockDev *__restri
     }
     __syncthreads();
     // every face of the tile once: I faces (TI+1)xTJxTK, then J, then K
-    for (int f = t; f < TL::NF; f += NT) {
-        int D, a, b, c;
-        if (f < TL::NFI) {
-            D = 0; c = f % TK; b = (f / TK) % TJ; a = f / (TK * TJ);
-        } else if (f < TL::NFI + TL::NFJ) {
-            const int r = f - TL::NFI;
-            D = 1; c = r % TK; b = (r / TK) % (TJ + 1); a = r / (TK * (TJ + 1));
-        } else {
-            const int r = f - TL::NFI - TL::NFJ;
-            D = 2; c = r % (TK + 1); b = (r / (TK + 1)) % TJ; a = r / ((TK + 1) * TJ);
-        }
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    for (int gq = wave; gq < TL::NG; gq += NT / 64) {
+        int D, a, b, c, f;
+        if (!TL::face(gq, t & 63, D, a, b, c, f)) continue;
         // higher-index cell of the face
         const int i = tl.y + a + 1, j = tl.z + b + 1, k = tl.w + c + 1;
         const bool ok = i <= B.ni + (D == 0) && j <= B.nj + (D == 1) && k <= B.nk + (D == 2);
