@@ -2702,7 +2702,7 @@ static void mlp_gradient(fv3d_ctx *c, const float *dx, const float *dt, long off
                          float *loss_out, const MlpAdam *adam)
 {
     const int nchunk = (int)((m + 63) / 64);
-    hipLaunchKernelGGL(k_mlp_train_chunk, dim3((unsigned)nchunk), dim3(256), 0, c->stream, c->d_mlp, dx + off * kMlpIn,
+    hipLaunchKernelGGL(k_mlp_train_chunk, dim3((unsigned)nchunk), dim3(1024), 0, c->stream, c->d_mlp, dx + off * kMlpIn,
                        dt + off, m, 1.0f / (float)m, dpart, dloss);
     if (adam)
         hipLaunchKernelGGL(k_mlp_reduce<true>, dim3(kMlpRedGroups), dim3(256), 0, c->stream, dpart, dloss, nchunk,
@@ -2753,7 +2753,7 @@ int fv3d_mlp_grad_noalloc(fv3d_ctx *c, const float *x_dev, const float *t_dev, l
     // nothing in the scratch needs clearing between calls
     float *part = s, *loss = s + (long)kNoAllocChunks * kMlpParams;
     const int nchunk = (int)((n + 63) / 64);
-    hipLaunchKernelGGL(k_mlp_train_chunk, dim3((unsigned)nchunk), dim3(256), 0, c->stream, c->d_mlp, x_dev, t_dev, n,
+    hipLaunchKernelGGL(k_mlp_train_chunk, dim3((unsigned)nchunk), dim3(1024), 0, c->stream, c->d_mlp, x_dev, t_dev, n,
                        1.0f / (float)n, part, loss);
     hipLaunchKernelGGL(k_mlp_reduce<false>, dim3(kMlpRedGroups), dim3(256), 0, c->stream, part, loss, nchunk, grad_dev,
                        loss_dev, (float)n, MlpAdam{});

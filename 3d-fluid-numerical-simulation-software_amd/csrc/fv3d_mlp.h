@@ -29,6 +29,7 @@ __global__ void k_mlp_cell_features(const BlockDev *blocks, const long *cstart, 
 __global__ void k_mlp_closure(const float *P, long ncell, float *xc);
 __global__ void k_mlp_mut(const BlockDev *blocks, const long *cstart, int nblock, Gas g, const float *bounds,
                           const float *xc, unsigned long long *tripped, double relax);
+// launched with 1024 threads per 64 samples
 __global__ void k_mlp_train_chunk(const float *P, const float *x, const float *tgt, long n, float inv_n, float *partial,
                                   float *loss);
 // the Adam update of a reduction that ends a training step: parameters, moments,

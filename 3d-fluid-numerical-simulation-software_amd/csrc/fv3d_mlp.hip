@@ -4,7 +4,7 @@
 // cores (v_mfma_f32_16x16x32_bf16) with FP32 accumulation, tanh hidden layers,
 // softplus output.  Inference runs per cell inside the residual evaluation in
 // place of the Spalart-Allmaras transport; training runs on the GPU with the
-// same forward code and a hand-written backward pass (per-chunk partial
+// same forward arithmetic and a hand-written backward pass (per-chunk partial
 // gradients, a fixed-order reduction, Adam).
 //
 // Matrix-core lane layout of v_mfma_f32_16x16x32_bf16 (one wave, D = A B + C,
@@ -19,6 +19,8 @@
 namespace fv3d {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kHS = kMlpH + 4;   // LDS row stride of an activation tile (floats)
@@ -442,116 +444,179 @@ __global__ void __launch_bounds__(256) k_mlp_mut(const BlockDev *__restrict__ bl
 
 // ------------------------------------------------------------ training
 // Loss = mean over the n samples of (softplus(z) - t)^2.  One workgroup per
-// chunk of 64 samples: forward (activations kept in LDS), then the backward
-// pass; the chunk's gradient goes to partial[chunk * kMlpParams + p] and its
-// sum of squared errors to loss[chunk].  Matrix products of the backward pass
-// run on the matrix cores with BF16 operands (deltas and activations
-// quantised as the forward pass quantises them), FP32 accumulation.
-__global__ void __launch_bounds__(256) k_mlp_train_chunk(const float *__restrict__ P, const float *__restrict__ x,
-                                                         const float *__restrict__ tgt, long n, float inv_n,
-                                                         float *__restrict__ partial, float *__restrict__ loss)
+// chunk of 64 samples: forward, then the backward pass; the chunk's gradient
+// goes to partial[chunk * kMlpParams + p] and its sum of squared errors to
+// loss[chunk].  Matrix products of the backward pass run on the matrix cores
+// with BF16 operands (deltas and activations quantised as the forward pass
+// quantises them), FP32 accumulation.
+//
+// A training step is a few chunks on a chip that holds hundreds, so the time
+// is one chunk's chain of products, tanh and sums.  Sixteen waves take one
+// 16 x 16 tile of every product each: wave (mt, nt) holds samples 16 mt.. and
+// units 16 nt.. of all three layers, so the activations that a delta needs
+// are in its own registers.  Both weight matrices come in with one round of
+// loads and every product's operands lie in LDS as BF16 with the summed index
+// contiguous (the array and its transpose where both are summed over), one
+// 16-byte read each.  The sums over samples keep the sample order, in waves of
+// their own once everything else is done.  Four waves that walked the tiles
+// and gathered each operand from FP32 arrays took 28 us for 64 chunks and 33 us
+// for 256; this takes 11 and 16 us, same bits.  What is left is a chunk's own
+// chain: one round of loads, 12 tanh a lane, eight barriers, the 64-term sums.
+constexpr int kBS = kMlpH + 8;   // LDS row stride of a BF16 tile: 16 rows' 16-byte reads cover all banks
+
+__device__ inline bf16x8 frag(const __bf16 *a, int r, int k) { return *(const bf16x8 *)(a + r * kBS + k); }
+
+// D = A B over 64 summed values: row r of a against row c of b
+__device__ inline f32x4 tile64(const __bf16 *a, int r, const __bf16 *b, int c, int kb)
 {
-    __shared__ float sx[64 * kMlpXS];
-    __shared__ float h[3][64 * kHS];   // activations, overwritten by the deltas
-    __shared__ float dz[64];
-    __shared__ float red[64];
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+        acc = mfma16(frag(a, r, 32 * ks + 8 * kb), frag(b, c, 32 * ks + 8 * kb), acc);
+    return acc;
+}
+
+// a lane's four values of column c, rows r..r+3, into a tile and its transpose
+__device__ inline void put4(__bf16 *a, __bf16 *at, int r, int c, const float v[4])
+{
+    bf16x4 q;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[(r + i) * kBS + c] = q[i] = (__bf16)v[i];
+    *(bf16x4 *)(at + c * kBS + r) = q;
+}
+
+__global__ void __launch_bounds__(1024) k_mlp_train_chunk(const float *__restrict__ P, const float *__restrict__ x,
+                                                          const float *__restrict__ tgt, long n, float inv_n,
+                                                          float *__restrict__ partial, float *__restrict__ loss)
+{
+    constexpr int kT = kMlpH * kBS, kF = 64 * kHS;
+    __shared__ __align__(16) __bf16 w1[kT], w2[kT], w1t[kT], w2t[kT];   // [unit][input], [input][unit]
+    __shared__ __align__(16) __bf16 a0[kT], a0t[kT], a1[kT], a1t[kT];   // [sample][unit], [unit][sample]
+    __shared__ __align__(16) float h2[kF], d2[kF], d1[kF], d0[kF];      // [sample][unit]
+    __shared__ __align__(16) float sx[64 * kMlpXS], sw3[kMlpH], dz[64], red[64];
+    // the deltas' BF16 tiles lie where the forward pass has read its last
+    __bf16 *const e2 = a0, *const e2t = w1, *const e1 = a1, *const e1t = w2;
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, row = lane & 15, kb = lane >> 4;
+    const int mt = wave >> 2, nt = wave & 3;
+    const int u = nt * 16 + row;          // unit of this lane's results
+    const int s = mt * 16 + 4 * kb;       // first of their four samples
+    const int ar = mt * 16 + row;         // row of an A operand
     const long s0 = (long)blockIdx.x * 64;
     float *G = partial + (long)blockIdx.x * kMlpParams;
-    for (int e = t; e < 64 * kMlpXS; e += 256) {
-        const int r = e / kMlpXS, q = e % kMlpXS;
-        sx[e] = (q < kMlpIn && s0 + r < n) ? x[(s0 + r) * kMlpIn + q] : 0.0f;
+
+    const float b0 = P[kMlpB0 + u], b1 = P[kMlpB1 + u], b2 = P[kMlpB2 + u], w3 = P[kMlpW3 + u];
+    if (t < kMlpH) sw3[t] = P[kMlpW3 + t];
+    float z = P[kMlpB3];
+    bf16x8 w0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w0[j] = (__bf16)((kb == 0 && j < kMlpIn) ? P[kMlpW0 + u * kMlpIn + j] : 0.0f);
+    const bool in = s0 + lane < n;
+    const float target = wave == 0 && in ? tgt[s0 + lane] : 0.0f;
+    if (t < 64 * kMlpXS) {
+        const int r = t / kMlpXS, q = t % kMlpXS;
+        sx[t] = (q < kMlpIn && s0 + r < n) ? x[(s0 + r) * kMlpIn + q] : 0.0f;
     }
-    __syncthreads();
-    const float z = mlp_forward16(P, sx, h[0], h[1], h[2], wave * 16, lane);
-    if (lane < 16) {
-        const int r = wave * 16 + lane;
-        const bool in = s0 + r < n;
-        const float e = in ? softplus(z) - tgt[s0 + r] : 0.0f;
-        dz[r] = in ? 2.0f * inv_n * e * sigmoid(z) : 0.0f;
-        red[r] = e * e;
-    }
-    __syncthreads();
-    if (t == 0) {
-        float s = 0.0f;
-        for (int r = 0; r < 64; ++r) s += red[r];
-        loss[blockIdx.x] = s;
-    }
-    // output layer: dW3, db3, then delta2 = dz W3 (1 - h2^2) in place
-    if (t < kMlpH) {
-        float s = 0.0f;
-        for (int r = 0; r < 64; ++r) s += dz[r] * h[2][r * kHS + t];
-        G[kMlpW3 + t] = s;
-    } else if (t == kMlpH) {
-        float s = 0.0f;
-        for (int r = 0; r < 64; ++r) s += dz[r];
-        G[kMlpB3] = s;
-    }
-    __syncthreads();
-    for (int e = t; e < 64 * kMlpH; e += 256) {
-        const int r = e / kMlpH, c = e % kMlpH;
-        const float a = h[2][r * kHS + c];
-        h[2][r * kHS + c] = dz[r] * P[kMlpW3 + c] * (1.0f - a * a);
-    }
-    __syncthreads();
-    // hidden layers L = 2, 1: delta in h[L], activations of the layer below in h[L-1]
-    for (int L = 2; L >= 1; --L) {
-        const float *Wl = P + (L == 2 ? kMlpW2 : kMlpW1);
-        const int oW = L == 2 ? kMlpW2 : kMlpW1, oB = L == 2 ? kMlpB2 : kMlpB1;
-        float *dl = h[L], *al = h[L - 1];
-        // dW[n][k] = sum_s delta[s][n] a[s][k]: output tiles (mt, nt), four per wave
-        for (int tile = wave * 4; tile < wave * 4 + 4; ++tile) {
-            const int mt = tile >> 2, nt = tile & 3;
-            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int ks = 0; ks < 2; ++ks) {
-                bf16x8 a, b;
-                for (int j = 0; j < 8; ++j) {
-                    const int s = 32 * ks + 8 * kb + j;
-                    a[j] = (__bf16)dl[s * kHS + mt * 16 + row];
-                    b[j] = (__bf16)al[s * kHS + nt * 16 + row];
-                }
-                acc = mfma16(a, b, acc);
-            }
-            for (int i = 0; i < 4; ++i) G[oW + (mt * 16 + 4 * kb + i) * kMlpH + nt * 16 + row] = acc[i];
+    {   // rows r, r + 1 and columns k..k+3 of one of the matrices
+        const bool second = t >= 512;
+        const int r = 2 * ((t >> 4) & 31), k = 4 * (t & 15);
+        const float *W = P + (second ? kMlpW2 : kMlpW1) + r * kMlpH + k;
+        const f32x4 v0 = *(const f32x4 *)W, v1 = *(const f32x4 *)(W + kMlpH);
+        __bf16 *w = second ? w2 : w1, *wt = second ? w2t : w1t;
+        bf16x4 q0, q1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            q0[j] = (__bf16)v0[j];
+            q1[j] = (__bf16)v1[j];
+            bf16x2 p;
+            p[0] = q0[j]; p[1] = q1[j];
+            *(bf16x2 *)(wt + (k + j) * kBS + r) = p;
         }
-        if (t < kMlpH) {
-            float s = 0.0f;
-            for (int r = 0; r < 64; ++r) s += dl[r * kHS + t];
-            G[oB + t] = s;
-        }
-        __syncthreads();
-        // delta below[s][k] = (sum_n delta[s][n] W[n][k]) (1 - a[s][k]^2), in place of a
-        for (int tile = wave * 4; tile < wave * 4 + 4; ++tile) {
-            const int mt = tile >> 2, nt = tile & 3;
-            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int ks = 0; ks < 2; ++ks) {
-                bf16x8 a, b;
-                for (int j = 0; j < 8; ++j) {
-                    const int nn = 32 * ks + 8 * kb + j;
-                    a[j] = (__bf16)dl[(mt * 16 + row) * kHS + nn];
-                    b[j] = (__bf16)Wl[nn * kMlpH + nt * 16 + row];
-                }
-                acc = mfma16(a, b, acc);
-            }
-            for (int i = 0; i < 4; ++i) {
-                const int s = mt * 16 + 4 * kb + i, c = nt * 16 + row;
-                const float av = al[s * kHS + c];
-                al[s * kHS + c] = acc[i] * (1.0f - av * av);
-            }
-        }
-        __syncthreads();
+        *(bf16x4 *)(w + r * kBS + k) = q0;
+        *(bf16x4 *)(w + (r + 1) * kBS + k) = q1;
     }
-    // input layer: dW0[n][f] = sum_s delta0[s][n] x[s][f], db0
-    for (int o = t; o < kMlpH * kMlpIn; o += 256) {
-        const int nn = o / kMlpIn, f = o % kMlpIn;
-        float s = 0.0f;
-        for (int r = 0; r < 64; ++r) s += h[0][r * kHS + nn] * (float)(__bf16)sx[r * kMlpXS + f];
-        G[kMlpW0 + o] = s;
+    __syncthreads();
+
+    float h[3][4];   // this lane's activations
+    {
+        bf16x8 a;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] = (__bf16)((kb == 0 && j < kMlpIn) ? sx[ar * kMlpXS + j] : 0.0f);
+        const f32x4 acc = mfma16(a, w0, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[0][i] = tanhf(acc[i] + b0);
+        put4(a0, a0t, s, u, h[0]);
     }
-    if (t < kMlpH) {
-        float s = 0.0f;
-        for (int r = 0; r < 64; ++r) s += h[0][r * kHS + t];
-        G[kMlpB0 + t] = s;
+    __syncthreads();
+    {
+        const f32x4 acc = tile64(a0, ar, w1, u, kb);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[1][i] = tanhf(acc[i] + b1);
+        put4(a1, a1t, s, u, h[1]);
+    }
+    __syncthreads();
+    {
+        const f32x4 acc = tile64(a1, ar, w2, u, kb);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h2[(s + i) * kHS + u] = h[2][i] = tanhf(acc[i] + b2);
+    }
+    __syncthreads();
+    if (wave == 0) {   // one sample per lane
+#pragma unroll
+        for (int k = 0; k < kMlpH; ++k) z += h2[lane * kHS + k] * sw3[k];
+        const float e = in ? softplus(z) - target : 0.0f;
+        dz[lane] = in ? 2.0f * inv_n * e * sigmoid(z) : 0.0f;
+        red[lane] = e * e;
+    }
+    __syncthreads();
+    float v[4];
+    // delta2 = dz W3 (1 - h2^2)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d2[(s + i) * kHS + u] = v[i] = dz[s + i] * w3 * (1.0f - h[2][i] * h[2][i]);
+    put4(e2, e2t, s, u, v);
+    __syncthreads();
+    // dW[m][k] = sum_s delta[s][m] a[s][k];
+    // delta below[s][k] = (sum_m delta[s][m] W[m][k]) (1 - a[s][k]^2)
+    const f32x4 g2 = tile64(e2t, ar, a1t, u, kb);
+    {
+        const f32x4 acc = tile64(e2, ar, w2t, u, kb);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d1[(s + i) * kHS + u] = v[i] = acc[i] * (1.0f - h[1][i] * h[1][i]);
+        put4(e1, e1t, s, u, v);
+    }
+    __syncthreads();
+    const f32x4 g1 = tile64(e1t, ar, a0t, u, kb);
+    {
+        const f32x4 acc = tile64(e1, ar, w1t, u, kb);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d0[(s + i) * kHS + u] = acc[i] * (1.0f - h[0][i] * h[0][i]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        G[kMlpW2 + (s + i) * kMlpH + u] = g2[i];
+        G[kMlpW1 + (s + i) * kMlpH + u] = g1[i];
+    }
+    // the sums over samples, each in sample order
+    float sum = 0.0f;
+    if (wave == 0) {
+#pragma unroll 32
+        for (int r = 0; r < 64; ++r) sum += dz[r] * h2[r * kHS + lane];
+        G[kMlpW3 + lane] = sum;
+    } else if (wave < 4) {
+        const float *d = wave == 1 ? d2 : wave == 2 ? d1 : d0;
+#pragma unroll 32
+        for (int r = 0; r < 64; ++r) sum += d[r * kHS + lane];
+        G[(wave == 1 ? kMlpB2 : wave == 2 ? kMlpB1 : kMlpB0) + lane] = sum;
+    } else if (wave < 4 + kMlpIn) {
+        const int o = t - 256, m = o / kMlpIn, f = o % kMlpIn;
+#pragma unroll 32
+        for (int r = 0; r < 64; ++r) sum += d0[r * kHS + m] * (float)(__bf16)sx[r * kMlpXS + f];
+        G[kMlpW0 + o] = sum;
+    } else if (wave == 4 + kMlpIn && lane < 2) {
+        const float *d = lane ? dz : red;
+#pragma unroll 32
+        for (int r = 0; r < 64; ++r) sum += d[r];
+        *(lane ? G + kMlpB3 : loss + blockIdx.x) = sum;
     }
 }
 
@@ -559,7 +624,7 @@ __global__ void __launch_bounds__(256) k_mlp_train_chunk(const float *__restrict
 // per 64 parameters: its four waves bring up to kRedChunks chunks into LDS with
 // every load in flight at once, then the first wave adds them in chunk order.
 // (One thread per parameter walking the chunks waits on memory once per chunk:
-// 60 us for 256 chunks, 16 us for 64; this takes 8 and 5 us, same bits.)
+// 60 us for 256 chunks, 16 us for 64; this takes 5.5 and 4 us, same bits.)
 // loss_out is the sum of the chunk losses over loss_div.  With ADAM the
 // gradient goes straight into the parameters' update (Kingma and Ba 2015) on
 // the FP32 master weights.
