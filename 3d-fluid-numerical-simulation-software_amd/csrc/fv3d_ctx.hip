@@ -594,7 +594,13 @@ static int build_exchange(fv3d_ctx *c)
                 double th_2 = atan(node(B, t.rng[1][0], t.rng[1][2], t.rng[1][4], 1) / node(B, t.rng[1][0], t.rng[1][2], t.rng[1][4], 0));
                 PeriodicDev q;
                 q.block = t.block[0] - 1;
-                q.flip = (th_2 - th_1) < 0.0;
+                q.odd = (th_2 - th_1) < 0.0;
+                q.last = 1;
+                for (PeriodicDev &o : per)
+                    if (o.block == q.block && o.last) {
+                        q.odd ^= o.odd;
+                        o.last = 0;
+                    }
                 // delta_th = 2*PI/NBlade in float (source/UserInput.cpp:443)
                 const double d = (double)(2.0f * 3.1415926535897932f / (float)A.nblade);
                 q.cs[0] = cos(d); q.cs[1] = sin(d);
@@ -618,9 +624,13 @@ static int build_exchange(fv3d_ctx *c)
                     return fail(c, FV3D_EINVAL, "connection sides do not match under orientation %d", t.orient);
                 const int da = (fa - 1) / 2, db = (fb - 1) / 2;
                 const int NA = da == 0 ? A.IM : da == 1 ? A.JM : A.KM, NB = db == 0 ? B.IM : db == 1 ? B.JM : B.KM;
-                for (int nd = 1; nd <= kND; ++nd)
+                // the layers of a K face lie side by side in memory: neighbouring
+                // items, so that a line is read once
+                const int nouter = da == 2 ? 1 : kND, ninner = kND / nouter;
+                for (int o1 = 1; o1 <= nouter; ++o1)
                     for (int l1 = 1; l1 <= L1; ++l1)
-                        for (int m1 = 1; m1 <= M1; ++m1) {
+                        for (int m1n = 0; m1n < M1 * ninner; ++m1n) {
+                            const int m1 = m1n / ninner + 1, nd = da == 2 ? m1n % ninner + 1 : o1;
                             int l2, m2;
                             switch (t.orient) {
                             case 1: l2 = l1; m2 = M1 + 1 - m1; break;
@@ -1597,9 +1607,9 @@ int fv3d_initial(fv3d_ctx *c)
 // ------------------------------------------------------------- stages
 static int launch_bc(fv3d_ctx *c)
 {
-    // the periodic signs are updated by k_bc's first thread when it runs
+    // the periodic signs are updated by k_bc's last workgroup when it runs
     if (c->nbc > 0)
-        hipLaunchKernelGGL(k_bc, dim3((unsigned)((c->nbc + 255) / 256)), dim3(256), 0, c->stream, c->d_blocks, c->d_patches,
+        hipLaunchKernelGGL(k_bc, dim3((unsigned)((c->nbc + 255) / 256) + (c->nper > 0)), dim3(256), 0, c->stream, c->d_blocks, c->d_patches,
                            c->npatch_dev, c->d_pstart_bc, c->gas, c->d_sc, c->d_per, c->nper, c->d_pitch_sign);
     else if (c->nper > 0)
         hipLaunchKernelGGL(k_periodic_flip, dim3(1), dim3(64), 0, c->stream, c->d_per, c->nper, c->d_pitch_sign);

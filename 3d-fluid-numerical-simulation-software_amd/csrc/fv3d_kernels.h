@@ -70,8 +70,8 @@ struct ScalarsDev {
 };
 
 struct PeriodicDev;
-// sc: the scalars of each instance (outlet pressure); with nper > 0 thread 0
-// first does the work of k_periodic_flip
+// sc: the scalars of each instance (outlet pressure); with nper > 0 the
+// launch has a workgroup more, which does the work of k_periodic_flip
 __global__ void k_bc(const BlockDev *blocks, const PatchDev *patches, int npatch, const long *pstart, Gas g,
                      const ScalarsDev *sc, PeriodicDev *per, int nper, int *pitch_sign);
 // radial-equilibrium outlet, one workgroup per patch (list: patch indices);
@@ -92,13 +92,16 @@ struct ExchDev {
     int src_block, dst_block, side, layer, rot, per;
     long src, slot, ghost;
 };
-// periodic patch: the block whose pitch angle it uses, whether applying it
-// flips that angle's sign (source/BndCondInteriorPeriodic.cpp:54-59), the sign
-// in force for this application, and cos/sin of +delta and -delta
+// periodic patch: the block whose pitch angle it uses, whether that angle's sign
+// has flipped an odd number of times in an application once this patch is
+// through (source/BndCondInteriorPeriodic.cpp:54-59), whether it is the block's
+// last patch, the sign in force for this application, and cos/sin of +delta
+// and -delta
 struct PeriodicDev {
-    int block, flip, sign;
+    int block, odd, last, sign;
     double cs[4];
 };
+// one workgroup
 __global__ void k_periodic_flip(PeriodicDev *per, int nper, int *pitch_sign);
 __global__ void k_exchange(const BlockDev *blocks, const ExchDev *el, long n, const PeriodicDev *per);
 // the CFL number of each block's instance: BlockDev::cfl

@@ -24,24 +24,33 @@ __device__ static void set_dummies(BlockRef B, int s, int a, int b, const double
 }
 
 // The pitch-angle sign of each periodic patch's block, updated in table order
-// (source/BndCondInteriorPeriodic.cpp:54-59); one thread, so patches that share
-// a block see each other's flips in order.
-__device__ static void periodic_flip(PeriodicDev *__restrict__ per, int nper, int *__restrict__ pitch_sign)
+// (source/BndCondInteriorPeriodic.cpp:54-59): patches that share a block see
+// each other's flips.  How often a patch's block has flipped by then is known
+// (PeriodicDev::odd), so one workgroup takes the patches side by side; one
+// thread walking them was 0.3 us each, the tail of the boundary kernel.
+__device__ static void periodic_flip(PeriodicDev *per, int nper, int *pitch_sign)
 {
-    for (int p = 0; p < nper; ++p) {
-        if (per[p].flip) pitch_sign[per[p].block] = -pitch_sign[per[p].block];
-        per[p].sign = pitch_sign[per[p].block];
+    for (int p = threadIdx.x; p < nper; p += blockDim.x) {
+        const int s = pitch_sign[per[p].block];
+        per[p].sign = per[p].odd ? -s : s;
     }
+    __syncthreads();
+    for (int p = threadIdx.x; p < nper; p += blockDim.x)
+        if (per[p].last) pitch_sign[per[p].block] = per[p].sign;
 }
 
-// Thread 0 also updates the periodic signs (nper > 0) for the exchange that
-// follows: no ghost fill here reads them, so this saves a launch.
+// With nper > 0 a workgroup past the patches' also updates the periodic signs
+// for the exchange that follows: no ghost fill here reads them, so this saves a
+// launch.
 __global__ void k_bc(const BlockDev *__restrict__ blocks, const PatchDev *__restrict__ patches, int npatch,
                      const long *__restrict__ pstart, Gas g, const ScalarsDev *__restrict__ sc,
-                     PeriodicDev *__restrict__ per, int nper, int *__restrict__ pitch_sign)
+                     PeriodicDev *per, int nper, int *pitch_sign)
 {
-    long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0 && nper > 0) periodic_flip(per, nper, pitch_sign);
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (nper > 0 && blockIdx.x == gridDim.x - 1) {
+        periodic_flip(per, nper, pitch_sign);
+        return;
+    }
     if (t >= pstart[npatch]) return;
     const int q = find_range(pstart, npatch, t);
     const PatchDev P = patches[q];
@@ -277,11 +286,7 @@ __global__ void __launch_bounds__(256) k_dt_global(const BlockDev *__restrict__ 
 }
 
 // ================================================== interior / periodic
-__global__ void k_periodic_flip(PeriodicDev *__restrict__ per, int nper, int *__restrict__ pitch_sign)
-{
-    if (threadIdx.x != 0) return;
-    periodic_flip(per, nper, pitch_sign);
-}
+__global__ void k_periodic_flip(PeriodicDev *per, int nper, int *pitch_sign) { periodic_flip(per, nper, pitch_sign); }
 
 // One transfer of source/ShadowOutIn.cpp: Trans rotates the momentum and the
 // velocity about z by dr when dr != 0 (lines 188-199).
@@ -291,27 +296,39 @@ __global__ void k_exchange(const BlockDev *__restrict__ blocks, const ExchDev *_
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     const ExchDev e = el[t];
-    BlockRef A = block_at(blocks, e.src_block), B = block_at(blocks, e.dst_block);
-    double q[5], w[6];
-    for (int c = 0; c < 5; ++c) q[c] = A.Q[c * A.box + e.src];
-    for (int c = 0; c < 6; ++c) w[c] = A.W[c * A.box + e.src];
-    if (e.rot) {
-        const PeriodicDev &P = per[e.per];
-        const bool pos = (e.rot == 1) == (P.sign > 0);   // dr = +delta or -delta
-        const double cr = pos ? P.cs[0] : P.cs[2], sr = pos ? P.cs[1] : P.cs[3];
-        const double qx = q[1], qy = q[2], ux = w[1], uy = w[2];
-        q[1] = qx * cr - qy * sr;
-        q[2] = qy * cr + qx * sr;
-        w[1] = ux * cr - uy * sr;
-        w[2] = uy * cr + ux * sr;
-    }
-    double *D = B.D[e.side] + (long)(e.layer - 1) * 11 * B.Dt[e.side] + e.slot;
-    for (int c = 0; c < 5; ++c) D[c * B.Dt[e.side]] = q[c];
-    for (int c = 0; c < 6; ++c) D[(5 + c) * B.Dt[e.side]] = w[c];
-    if (e.ghost >= 0) {
-        for (int c = 0; c < 5; ++c) B.Q[c * B.box + e.ghost] = q[c];
-        for (int c = 0; c < 6; ++c) B.W[c * B.box + e.ghost] = w[c];
-        if (B.ev) B.ev[e.ghost] = A.ev[e.src];   // nu~ of the ghost layer only (source/ShadowOutIn.cpp:339-345)
+    // One (source block, target block, side) of the wave's lanes after the other,
+    // nearly always one in all: what the block tables hold then comes through
+    // scalar loads.
+    for (unsigned long long left = __builtin_amdgcn_ballot_w64(true); left;) {
+        const int l = __builtin_ctzll(left);
+        const int sb = __builtin_amdgcn_readlane(e.src_block, l), db = __builtin_amdgcn_readlane(e.dst_block, l),
+                  side = __builtin_amdgcn_readlane(e.side, l);
+        const bool in = e.src_block == sb && e.dst_block == db && e.side == side;
+        left &= ~__builtin_amdgcn_ballot_w64(in);
+        if (!in) continue;
+        BlockRef A = block_at(blocks, sb), B = block_at(blocks, db);
+        double q[5], w[6];
+        for (int c = 0; c < 5; ++c) q[c] = A.Q[c * A.box + e.src];
+        for (int c = 0; c < 6; ++c) w[c] = A.W[c * A.box + e.src];
+        if (e.rot) {
+            const PeriodicDev &P = per[e.per];
+            const bool pos = (e.rot == 1) == (P.sign > 0);   // dr = +delta or -delta
+            const double cr = pos ? P.cs[0] : P.cs[2], sr = pos ? P.cs[1] : P.cs[3];
+            const double qx = q[1], qy = q[2], ux = w[1], uy = w[2];
+            q[1] = qx * cr - qy * sr;
+            q[2] = qy * cr + qx * sr;
+            w[1] = ux * cr - uy * sr;
+            w[2] = uy * cr + ux * sr;
+        }
+        const long Dt = B.Dt[side];
+        double *D = B.D[side] + (long)(e.layer - 1) * 11 * Dt + e.slot;
+        for (int c = 0; c < 5; ++c) D[c * Dt] = q[c];
+        for (int c = 0; c < 6; ++c) D[(5 + c) * Dt] = w[c];
+        if (e.ghost >= 0) {
+            for (int c = 0; c < 5; ++c) B.Q[c * B.box + e.ghost] = q[c];
+            for (int c = 0; c < 6; ++c) B.W[c * B.box + e.ghost] = w[c];
+            if (B.ev) B.ev[e.ghost] = A.ev[e.src];   // nu~ of the ghost layer only (source/ShadowOutIn.cpp:339-345)
+        }
     }
 }
 
