@@ -1954,8 +1954,7 @@ static int launch_update(fv3d_ctx *c)
     HIPCK(c, hipGetLastError());
     if (c->cfg.limiter) {
         hipLaunchKernelGGL(k_limiter_serial, dim3(1), dim3(64), 0, c->stream, c->d_blocks, nb, c->gas, c->d_bad,
-                           c->d_cstart, c->d_partial, c->npart);
-        if (sa) hipLaunchKernelGGL(k_sa_limit_serial, dim3(1), dim3(64), 0, c->stream, c->d_blocks, nb, c->d_sa_hi);
+                           c->d_cstart, c->d_partial, c->npart, sa_hi);
         HIPCK(c, hipGetLastError());
     }
     if (sa) {
@@ -2137,7 +2136,7 @@ static int launch_limiter(fv3d_ctx *c)
 {
     if (!c->cfg.limiter) return FV3D_OK;
     hipLaunchKernelGGL(k_limiter_serial, dim3(1), dim3(64), 0, c->stream, c->d_blocks, (int)c->blocks.size(), c->gas,
-                       c->d_bad, c->d_cstart, (double *)nullptr, 0);
+                       c->d_bad, c->d_cstart, (double *)nullptr, 0, (int *)nullptr);
     HIPCK(c, hipGetLastError());
     return FV3D_OK;
 }

@@ -175,8 +175,9 @@ __global__ void k_update(const BlockDev *blocks, const long *cstart, int nblock,
                          int *sa_hi, int sa);
 template <int TJ, int TK, int MODE>
 __global__ void k_conv_stream(const BlockDev *blocks, const int4 *tiles, int ntiles, int ci, Gas g, int ndec);
+// one wave; sa_hi: the nu~ flags, or null
 __global__ void k_limiter_serial(const BlockDev *blocks, int nblock, Gas g, int *bad_flag, const long *cstart,
-                                 double *partial, int npart);
+                                 double *partial, int npart, int *sa_hi);
 __global__ void k_sections(const BlockDev *blocks, const int2 *secs, Gas g, double *sums);
 // norms and section integrals of one level (lv) with the CFL ramp and the
 // iteration count kept in ramp (the fine level's scalars, shared by the
@@ -237,9 +238,8 @@ __global__ void k_sa_mut(const BlockDev *blocks, const long *cstart, int nblock,
 __global__ void k_sa_ghost(const BlockDev *blocks, const long *gstart, int nblock, Gas g);
 template <bool FORWARD>
 __global__ void k_sa_plane(const BlockDev *blocks, const long *pstart, int nblock, int step, double relax, Gas g);
-// Limit_SA: the blocks k_update flagged, serially; then the pointwise floor of
-// the others (clamp set) with the Res_ev partials in component 5
-__global__ void k_sa_limit_serial(const BlockDev *blocks, int nblock, int *hi_flag);
+// Limit_SA's pointwise floor (clamp set) of the blocks k_limiter_serial left
+// alone, and the Res_ev partials in component 5
 __global__ void k_sa_res(const BlockDev *blocks, const long *cstart, int nblock, double *partial, int clamp);
 
 __global__ void k_mixing_plane(const BlockDev *blocks, const MixDev *mix, int nmix, Gas g, int sa);

@@ -1414,9 +1414,7 @@ __global__ void __launch_bounds__(256) k_update(const BlockDev *__restrict__ blo
         for (int c = 0; c < 5; ++c) partial[(long)c * gridDim.x + blockIdx.x] = red[c][0];
 }
 
-// Limit_Vars (source/Limit_FlowVars.cpp:8-119) in the reference's serial order:
-// cells are repaired one after the other, so later repairs see earlier ones.
-// Runs as one thread and returns at once unless k_update flagged a bad cell.
+// the limiter's test of a cell (source/Limit_FlowVars.cpp:28-29)
 __device__ static bool bad_cell(BlockRef B, long x)
 {
     const long box = B.box;
@@ -1426,6 +1424,9 @@ __device__ static bool bad_cell(BlockRef B, long x)
            B.W[3 * box + x] > vmax;
 }
 
+// Limit_Vars (source/Limit_FlowVars.cpp:8-119) in the reference's serial order:
+// cells are repaired one after the other, so later repairs see earlier ones.
+//
 // Res_Calculate runs after Limit_Vars in the reference
 // (source/LU_SGS_Marching.cpp:287-290, source/Solver.cpp:92-93), but k_update
 // formed the norm partials from the state before the repair.  With partial
@@ -1433,10 +1434,9 @@ __device__ static bool bad_cell(BlockRef B, long x)
 // pre-repair value to the repaired one in its 256-cell group's partial
 // (q_old = the pre-repair value minus dQ).  Without it (the limiter after a
 // prolongation, which no norm follows) nothing is patched.
-__global__ void k_limiter_serial(const BlockDev *__restrict__ blocks, int nblock, Gas g, int *__restrict__ bad_flag,
-                                 const long *__restrict__ cstart, double *__restrict__ partial, int npart)
+__device__ static void limit_vars(const BlockDev *__restrict__ blocks, int nblock, const Gas &g, int *__restrict__ bad_flag,
+                                  const long *__restrict__ cstart, double *__restrict__ partial, int npart)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
     const double Gamma = g.gamma, Rgas = g.rgas;
     const double dmin = F32C(1.0E-6), dmax = F32C(1000.0), vmax = F32C(1000.0);
     for (int n = 0; n < nblock; ++n) {
@@ -1499,6 +1499,59 @@ __global__ void k_limiter_serial(const BlockDev *__restrict__ blocks, int nblock
     }
 }
 
+// CFluidProps::Limit_SA (source/Limit_FlowVars.cpp:122-168).  Raising values
+// below 1e-8 is pointwise; replacing a value above 1000 by the mean of its
+// admissible neighbours depends on the neighbours' already limited values, so
+// a block with such a value (k_update flags it) is limited by one thread in
+// the reference's order here, and the floor of the other blocks is applied in
+// k_sa_res.
+__device__ static void limit_sa(const BlockDev *__restrict__ blocks, int nblock, int *__restrict__ hi_flag)
+{
+    const double SAmin = F32C(1.0E-8), LSAmax = F32C(1000.0);
+    for (int n = 0; n < nblock; ++n) {
+        if (!hi_flag[n]) continue;
+        hi_flag[n] = 0;
+        BlockRef B = block_at(blocks, n);
+        const int IM = B.IM, JM = B.JM, KM = B.KM;
+        for (int i = 1; i <= B.ni; ++i)
+            for (int j = 1; j <= B.nj; ++j)
+                for (int k = 1; k <= B.nk; ++k) {
+                    double *e = B.ev + cidx(B, i, j, k);
+                    if (*e < SAmin) *e = SAmin;
+                    if (*e > LSAmax) {
+                        double s0 = 0.0;
+                        int kn = 0;
+                        for (int ka = -1; ka <= 1; ++ka)
+                            for (int ja = -1; ja <= 1; ++ja)
+                                for (int ia = -1; ia <= 1; ++ia) {
+                                    const int k1 = k + ka, j1 = j + ja, i1 = i + ia;
+                                    if (i1 > 0 && i1 < IM && j1 > 0 && j1 < JM && k1 > 0 && k1 < KM) {
+                                        const double v = B.ev[cidx(B, i1, j1, k1)];
+                                        if (v >= SAmin && v <= LSAmax) { s0 = s0 + v; kn = kn + 1; }
+                                    }
+                                }
+                        *e = kn == 0 ? LSAmax : s0 / kn;
+                    }
+                }
+    }
+}
+
+// The limiters, when k_update (or the multigrid transfers) flagged a bad cell:
+// one wave looks at all the flags at once and returns, its first thread
+// repairs.  One thread walking the flags of Limit_Vars, and a second launch for
+// those of Limit_SA, cost 4.5 us each; a launch that has nothing to do costs
+// that much whatever it looks at.
+__global__ void __launch_bounds__(64) k_limiter_serial(const BlockDev *__restrict__ blocks, int nblock, Gas g,
+                                                       int *__restrict__ bad_flag, const long *__restrict__ cstart,
+                                                       double *__restrict__ partial, int npart, int *__restrict__ sa_hi)
+{
+    int any = 0;
+    for (int n = threadIdx.x; n < nblock; n += 64) any |= bad_flag[n] | (sa_hi ? sa_hi[n] : 0);
+    if (__builtin_amdgcn_ballot_w64(any != 0) == 0 || threadIdx.x != 0) return;
+    limit_vars(blocks, nblock, g, bad_flag, cstart, partial, npart);
+    if (sa_hi) limit_sa(blocks, nblock, sa_hi);
+}
+
 // ============================================= section integrals, norms
 // Mass flow, mass-averaged total pressure and total temperature over one K
 // plane (source/Ouput.cpp:9-95): workgroup `part` of section sec sums the cells
@@ -1553,7 +1606,9 @@ __global__ void __launch_bounds__(256) k_sections(const BlockDev *__restrict__ b
 // (source/Solver.cpp:49-60) and the history row, hist_row or, without it, the
 // cursor's next one.  As two launches, the second with one workgroup per
 // instance, this took 53 us on a 2.54M-cell passage and 12 on the smallest
-// grids, and a copy of the row 4.5 more.
+// grids, and a copy of the row 4.5 more; now 20 and 8.  A workgroup without
+// cells leaves at once: with all kFinParts counting themselves in, eight
+// passages of one batch took 30 us, now 17.
 __global__ void __launch_bounds__(256) k_finish(const BlockDev *__restrict__ blocks, const int2 *__restrict__ secs,
                                                 const double *__restrict__ partial, int npart,
                                                 const int2 *__restrict__ parts, double *__restrict__ secsum,
@@ -1570,26 +1625,32 @@ __global__ void __launch_bounds__(256) k_finish(const BlockDev *__restrict__ blo
     double *norms = secsum + (long)ninst * 2 * kSecParts * 3 + 6 * inst;
     // component 5: Res_ev of Spalart-Allmaras (k_sa_res)
     const int nc = g.turbulence == 200 ? 6 : 5;
+    // section parts that hold cells; the other workgroups have nothing to do
+    // (each that counts itself in writes its XCD's L2 back first)
+    auto nonempty = [&](int sec) {
+        BlockRef B = block_at(blocks, secs[2 * inst + sec].x);
+        return min((B.ni * B.nj + 255) / 256, kSecParts);
+    };
+    const int np0 = nonempty(0), np1 = nonempty(1);
+    if (part < 2 * kSecParts ? part % kSecParts >= (part < kSecParts ? np0 : np1) : part - 2 * kSecParts >= nc) return;
     if (part < 2 * kSecParts) {
         section_part(blocks, secs, g, secsum, inst * 2 + part / kSecParts, part % kSecParts, red);
     } else {
         const int c = part - 2 * kSecParts;
         double r = 0.0;
-        if (c < nc) {
-            // each thread adds partials t, t + 256, ... in that order; sixteen
-            // loads are in flight before the first is added
-            const double *src = partial + (long)c * npart + parts[inst].x;
-            const int np = parts[inst].y;
-            int p = t;
-            for (; p + 15 * 256 < np; p += 16 * 256) {
-                double v[16];
+        // each thread adds partials t, t + 256, ... in that order; sixteen
+        // loads are in flight before the first is added
+        const double *src = partial + (long)c * npart + parts[inst].x;
+        const int np = parts[inst].y;
+        int p = t;
+        for (; p + 15 * 256 < np; p += 16 * 256) {
+            double v[16];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) v[u] = src[p + u * 256];
+            for (int u = 0; u < 16; ++u) v[u] = src[p + u * 256];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) r += v[u];
-            }
-            for (; p < np; p += 256) r += src[p];
+            for (int u = 0; u < 16; ++u) r += v[u];
         }
+        for (; p < np; p += 256) r += src[p];
         red[0][t] = r;
         __syncthreads();
         for (int w = 128; w > 0; w >>= 1) {
@@ -1601,36 +1662,45 @@ __global__ void __launch_bounds__(256) k_finish(const BlockDev *__restrict__ blo
     // what this workgroup wrote (thread 0) is visible before it counts itself in
     if (t == 0) {
         __threadfence();
-        s_last = atomicAdd(arrived + inst, 1) == kFinParts - 1;
+        s_last = atomicAdd(arrived + inst, 1) == np0 + np1 + nc - 1;
         if (s_last) __threadfence();
     }
     __syncthreads();
     if (!s_last) return;
+    const double total_vol = sc->total_vol, dens_ref = sc->dens_ref, vel_ref = sc->vel_ref, temp_ref = sc->temp_ref;
+    const double nblade_in = sc->nblade_in, nblade_out = sc->nblade_out;
     // section partials in a fixed order: section 0 inlet, 1 outlet; mass, ptm,
     // ttm; then the norms
     const double *own = secsum + (long)inst * 2 * kSecParts * 3;
-    if (t < 2 * kSecParts * 3)
-        red[0][t] = __hip_atomic_load(own + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else if (t < 2 * kSecParts * 3 + 6)
-        red[0][t] = __hip_atomic_load(norms + t - 2 * kSecParts * 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int e = t / 3;   // part of the partial this thread brings in
+    if (t < 2 * kSecParts * 3) {
+        if (e % kSecParts < (e < kSecParts ? np0 : np1))
+            red[0][t] = __hip_atomic_load(own + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if (t < 2 * kSecParts * 3 + 6) {
+        const int c = t - 2 * kSecParts * 3;
+        red[0][t] = c < nc ? __hip_atomic_load(norms + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+    }
     __syncthreads();
     if (t < 6) {
         double s = 0.0;
-        for (int p = 0; p < kSecParts; ++p) s += red[0][((t / 3) * kSecParts + p) * 3 + t % 3];
+        const int np = t < 3 ? np0 : np1;
+        for (int p = 0; p < np; ++p) s += red[0][((t / 3) * kSecParts + p) * 3 + t % 3];
         red[1][t] = s;
     }
     __syncthreads();
+    const double Gamma = g.gamma, Rgas = g.rgas;
+    const double *norm = &red[0][2 * kSecParts * 3], *sums = red[1];
+    if (t < 2)
+        red[2][t] = pow(sums[3 * t + 1] / sums[3 * t], Gamma / (Gamma - F32C(1.0))) * dens_ref * vel_ref * vel_ref;
+    __syncthreads();
     if (t != 0) return;
     arrived[inst] = 0;
-    const double *norm = &red[0][2 * kSecParts * 3], *sums = red[1];
-    for (int c = 0; c < 5; ++c) sc->res[c] = norm[c] / sc->total_vol;
-    sc->res_ev = norm[5] / sc->total_vol;
-    const double Gamma = g.gamma, Rgas = g.rgas;
-    double mi = sums[0] * sc->dens_ref * sc->vel_ref * sc->nblade_in;
-    double mo = sums[3] * sc->dens_ref * sc->vel_ref * sc->nblade_out;
-    double pti = pow(sums[1] / sums[0], Gamma / (Gamma - F32C(1.0))) * sc->dens_ref * sc->vel_ref * sc->vel_ref;
-    double pto = pow(sums[4] / sums[3], Gamma / (Gamma - F32C(1.0))) * sc->dens_ref * sc->vel_ref * sc->vel_ref;
-    double tti = sums[2] / sums[0] * sc->temp_ref, tto = sums[5] / sums[3] * sc->temp_ref;
+    for (int c = 0; c < 5; ++c) sc->res[c] = norm[c] / total_vol;
+    sc->res_ev = norm[5] / total_vol;
+    double mi = sums[0] * dens_ref * vel_ref * nblade_in;
+    double mo = sums[3] * dens_ref * vel_ref * nblade_out;
+    const double pti = red[2][0], pto = red[2][1];
+    double tti = sums[2] / sums[0] * temp_ref, tto = sums[5] / sums[3] * temp_ref;
     double PR = pto / pti;
     double L_adk = Gamma / (Gamma - F32C(1.0)) * Rgas * tti * (pow(PR, (Gamma - F32C(1.0)) / Gamma) - F32C(1.0));
     double L_k = Gamma / (Gamma - F32C(1.0)) * Rgas * tti * (tto / tti - F32C(1.0));

@@ -353,50 +353,11 @@ __global__ void k_sa_plane(const BlockDev *__restrict__ blocks, const long *__re
 template __global__ void k_sa_plane<true>(const BlockDev *, const long *, int, int, double, Gas);
 template __global__ void k_sa_plane<false>(const BlockDev *, const long *, int, int, double, Gas);
 
-// ------------------------------------------------------------- Limit_SA
-// CFluidProps::Limit_SA (source/Limit_FlowVars.cpp:122-168).  Raising values
-// below 1e-8 is pointwise; replacing a value above 1000 by the mean of its
-// admissible neighbours depends on the neighbours' already limited values, so
-// a block with such a value (k_update flags it) is limited by one thread in
-// the reference's order here, and the floor of the other blocks is applied in
-// k_sa_res.
-__global__ void k_sa_limit_serial(const BlockDev *__restrict__ blocks, int nblock, int *__restrict__ hi_flag)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const double SAmin = F32C(1.0E-8), LSAmax = F32C(1000.0);
-    for (int n = 0; n < nblock; ++n) {
-        if (!hi_flag[n]) continue;
-        hi_flag[n] = 0;
-        BlockRef B = block_at(blocks, n);
-        const int IM = B.IM, JM = B.JM, KM = B.KM;
-        for (int i = 1; i <= B.ni; ++i)
-            for (int j = 1; j <= B.nj; ++j)
-                for (int k = 1; k <= B.nk; ++k) {
-                    double *e = B.ev + cidx(B, i, j, k);
-                    if (*e < SAmin) *e = SAmin;
-                    if (*e > LSAmax) {
-                        double s0 = 0.0;
-                        int kn = 0;
-                        for (int ka = -1; ka <= 1; ++ka)
-                            for (int ja = -1; ja <= 1; ++ja)
-                                for (int ia = -1; ia <= 1; ++ia) {
-                                    const int k1 = k + ka, j1 = j + ja, i1 = i + ia;
-                                    if (i1 > 0 && i1 < IM && j1 > 0 && j1 < JM && k1 > 0 && k1 < KM) {
-                                        const double v = B.ev[cidx(B, i1, j1, k1)];
-                                        if (v >= SAmin && v <= LSAmax) { s0 = s0 + v; kn = kn + 1; }
-                                    }
-                                }
-                        *e = kn == 0 ? LSAmax : s0 / kn;
-                    }
-                }
-    }
-}
-
 // Res_ev of CMesh::Res_Calculate (source/ComputeAllBlockVars.cpp:352-357,
 // 368-371): partial sums of |(nu~_old - nu~)/nu~_old| Vol, after the limiter
 // as in the reference, into component 5 of the norm partials (same grid as
 // k_update).  With clamp set (limiter on) nu~ below 1e-8 is raised to it
-// first; blocks k_sa_limit_serial treated hold no such value any more.
+// first; blocks k_limiter_serial treated hold no such value any more.
 __global__ void __launch_bounds__(256) k_sa_res(const BlockDev *__restrict__ blocks, const long *__restrict__ cstart,
                                                 int nblock, double *__restrict__ partial, int clamp)
 {
