@@ -181,6 +181,7 @@ struct fv3d_ctx {
     ScalarsDev *ramp_sc = nullptr;
     // graph
     hipGraphExec_t graph_exec = nullptr;
+    hipGraphExec_t graph_many = nullptr;     // kGraphIters iterations
     hipGraphExec_t graph_coarse = nullptr;   // coarse start-up phase of the two-grid cycle
     // timing
     int timing = 0;
@@ -829,6 +830,7 @@ int fv3d_ctx_destroy(fv3d_ctx *c)
         c->coarse = nullptr;
     }
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
+    if (c->graph_many) (void)hipGraphExecDestroy(c->graph_many);
     if (c->graph_coarse) (void)hipGraphExecDestroy(c->graph_coarse);
     if (c->d_bl_walls) (void)hipFree(c->d_bl_walls);
     if (c->d_exch) (void)hipFree(c->d_exch);
@@ -2418,6 +2420,9 @@ int fv3d_iterate(fv3d_ctx *c, int n, double *hist)
     return FV3D_OK;
 }
 
+// iterations of graph_many
+static constexpr int kGraphIters = 4;
+
 int fv3d_iterate_graph(fv3d_ctx *c, int n, double *hist)
 {
     READY(c);
@@ -2434,18 +2439,20 @@ int fv3d_iterate_graph(fv3d_ctx *c, int n, double *hist)
     // iteration between them (Coarse_iter) runs eagerly
     hipLaunchKernelGGL(k_hist_begin, dim3(1), dim3(64), 0, c->stream, c->d_cursor, c->d_hist, c->ramp_sc, c->ninst);
     HIPCK(c, hipGetLastError());
-    auto capture = [&](hipGraphExec_t *exec, int phase) -> int {
+    auto capture = [&](hipGraphExec_t *exec, int phase, int count) -> int {
         if (*exec) return FV3D_OK;
         hipGraph_t g;
         int saved = c->timing;
         c->timing = 0;
         HIPCK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        int r;
-        if (c->ng == 2) {
-            r = mg_iteration(c, phase, nullptr);
-        } else {
-            r = lusgs_timed(c);
-            if (!r) r = launch_finish(c, nullptr);
+        int r = FV3D_OK;
+        for (int q = 0; q < count && !r; ++q) {
+            if (c->ng == 2) {
+                r = mg_iteration(c, phase, nullptr);
+            } else {
+                r = lusgs_timed(c);
+                if (!r) r = launch_finish(c, nullptr);
+            }
         }
         hipError_t e = hipStreamEndCapture(c->stream, &g);
         c->timing = saved;
@@ -2455,17 +2462,22 @@ int fv3d_iterate_graph(fv3d_ctx *c, int n, double *hist)
         HIPCK(c, hipGraphDestroy(g));
         return FV3D_OK;
     };
-    for (int it = 0; it < n; ++it) {
+    // Between two graph launches the device idles for some 8 us, between the
+    // kernels of one for none, so kGraphIters iterations go as one graph where
+    // that many are left (the cycle's phase is the last: it stays until the end).
+    for (int it = 0; it < n;) {
         const long itn = c->iter_host + 1;
         const int phase = c->ng == 2 ? mg_phase(c, itn) : kMgCycle;
+        const int count = phase == kMgCycle && n - it >= kGraphIters ? kGraphIters : 1;
         if (phase == kMgSwitch) {
             if ((rc = mg_iteration(c, phase, nullptr))) return rc;
         } else {
-            hipGraphExec_t *exec = phase == kMgCoarse ? &c->graph_coarse : &c->graph_exec;
-            if ((rc = capture(exec, phase))) return rc;
+            hipGraphExec_t *exec = phase == kMgCoarse ? &c->graph_coarse : count > 1 ? &c->graph_many : &c->graph_exec;
+            if ((rc = capture(exec, phase, count))) return rc;
             HIPCK(c, hipGraphLaunch(*exec, c->stream));
         }
-        c->iter_host = itn;
+        c->iter_host += count;
+        it += count;
     }
     if (hist && n > 0)
         HIPCK(c, hipMemcpyAsync(hist, c->d_hist, 7L * n * c->ninst * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -2510,6 +2522,7 @@ long fv3d_cell_count(const fv3d_ctx *c) { return c ? c->ncell_real : 0; }
 static void drop_graphs(fv3d_ctx *c)
 {
     if (c->graph_exec) { (void)hipGraphExecDestroy(c->graph_exec); c->graph_exec = nullptr; }
+    if (c->graph_many) { (void)hipGraphExecDestroy(c->graph_many); c->graph_many = nullptr; }
     if (c->graph_coarse) { (void)hipGraphExecDestroy(c->graph_coarse); c->graph_coarse = nullptr; }
 }
 
@@ -2858,7 +2871,7 @@ int fv3d_set_debug(fv3d_ctx *c, int flags)
         c->sweep_mode = 4;
         return fail(c, FV3D_EINVAL, "the FP32 operator runs with the default sweep form only");
     }
-    if (c->graph_exec) { (void)hipGraphExecDestroy(c->graph_exec); c->graph_exec = nullptr; }
+    drop_graphs(c);
     if (c->store_faces && !c->d_faces[0]) {
         long mx = 0;
         for (auto &b : c->blocks) mx = std::max(mx, b.dev.box);
