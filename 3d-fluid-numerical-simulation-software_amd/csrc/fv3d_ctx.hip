@@ -84,6 +84,7 @@ struct fv3d_ctx {
     long nexch = 0;
     PeriodicDev *d_per = nullptr;
     int nper = 0;
+    int nflip = 0;               // nper if any periodic patch flips its sign, else 0
     int *d_pitch_sign = nullptr;
     std::vector<PatchDev> pd_host;   // the device patch list, host copy
     double *d_mbox = nullptr;         // sweep mailboxes of all blocks
@@ -596,7 +597,7 @@ static int build_exchange(fv3d_ctx *c)
                 PeriodicDev q;
                 q.block = t.block[0] - 1;
                 q.odd = (th_2 - th_1) < 0.0;
-                q.last = 1;
+                q.last = q.sign = 1;   // pitch_sign's start
                 for (PeriodicDev &o : per)
                     if (o.block == q.block && o.last) {
                         q.odd ^= o.odd;
@@ -664,6 +665,9 @@ static int build_exchange(fv3d_ctx *c)
         }
     c->nexch = (long)el.size();
     c->nper = (int)per.size();
+    c->nflip = 0;
+    for (const PeriodicDev &p : per)
+        if (p.odd) c->nflip = c->nper;
     int rc;
     if (!c->mixes.empty()) {
         std::vector<MixDev> ml;
@@ -1609,18 +1613,25 @@ int fv3d_initial(fv3d_ctx *c)
 // ------------------------------------------------------------- stages
 static int launch_bc(fv3d_ctx *c)
 {
-    // the periodic signs are updated by k_bc's last workgroup when it runs
-    if (c->nbc > 0)
-        hipLaunchKernelGGL(k_bc, dim3((unsigned)((c->nbc + 255) / 256) + (c->nper > 0)), dim3(256), 0, c->stream, c->d_blocks, c->d_patches,
-                           c->npatch_dev, c->d_pstart_bc, c->gas, c->d_sc, c->d_per, c->nper, c->d_pitch_sign);
-    else if (c->nper > 0)
-        hipLaunchKernelGGL(k_periodic_flip, dim3(1), dim3(64), 0, c->stream, c->d_per, c->nper, c->d_pitch_sign);
-    if (c->n_axial > 0)
-        hipLaunchKernelGGL(k_bc_axial, dim3((unsigned)c->n_axial), dim3(256), 0, c->stream, c->d_blocks, c->d_patches,
-                           c->d_axial, c->gas, c->d_sc);
-    if (c->nexch > 0)
-        hipLaunchKernelGGL(k_exchange, dim3((unsigned)((c->nexch + 255) / 256)), dim3(256), 0, c->stream, c->d_blocks,
-                           c->d_exch, c->nexch, c->d_per);
+    const int bcg = (int)((c->nbc + 255) / 256), exg = (int)((c->nexch + 255) / 256);
+    auto boundary = [&](int nbcg, int nexg, int nflip) {
+        const int n = nbcg + nexg + (nflip > 0);
+        if (n > 0)
+            hipLaunchKernelGGL(k_boundary, dim3((unsigned)n), dim3(256), 0, c->stream, c->d_blocks, c->d_patches,
+                               c->npatch_dev, c->d_pstart_bc, nbcg, c->gas, c->d_sc, c->d_exch, c->nexch, c->d_per, nflip,
+                               c->d_pitch_sign);
+    };
+    // one launch, unless the exchange rotates by signs that this application
+    // flips, or follows a radial-equilibrium outlet that covers a whole face
+    if (c->nflip == 0 && c->n_axial == 0) {
+        boundary(bcg, exg, 0);
+    } else {
+        boundary(bcg, 0, c->nflip);
+        if (c->n_axial > 0)
+            hipLaunchKernelGGL(k_bc_axial, dim3((unsigned)c->n_axial), dim3(256), 0, c->stream, c->d_blocks, c->d_patches,
+                               c->d_axial, c->gas, c->d_sc);
+        boundary(0, exg, 0);
+    }
     if (c->nmix_lines > 0)   // after interior and periodic patches (source/BoundaryCondition.cpp:59-62)
         hipLaunchKernelGGL(k_mixing_plane, dim3((unsigned)c->nmix_lines), dim3(256), 0, c->stream, c->d_blocks, c->d_mix,
                            c->nmix, c->gas, c->cfg.turbulence == 200 ? 1 : 0);

@@ -42,7 +42,7 @@ struct PatchDev {
     int a0, b0;        // first tangential cell indices
     int na, nb;        // tangential extents
     int centrifugal;   // outlet variant
-    int axial;         // radial-equilibrium outlet: applied by k_bc_axial, skipped by k_bc
+    int axial;         // radial-equilibrium outlet: applied by k_bc_axial, skipped by k_boundary
     int inst;          // instance of the patch's block (its scalars hold the outlet pressure)
     double rot;        // wall rotation rate
 };
@@ -69,11 +69,6 @@ struct ScalarsDev {
     long hist_pos;      // history rows written since k_hist_begin
 };
 
-struct PeriodicDev;
-// sc: the scalars of each instance (outlet pressure); with nper > 0 the
-// launch has a workgroup more, which does the work of k_periodic_flip
-__global__ void k_bc(const BlockDev *blocks, const PatchDev *patches, int npatch, const long *pstart, Gas g,
-                     const ScalarsDev *sc, PeriodicDev *per, int nper, int *pitch_sign);
 // radial-equilibrium outlet, one workgroup per patch (list: patch indices);
 // the radial lines of a face are at most kAxialMaxI cells long
 constexpr int kAxialMaxI = 2048;
@@ -101,9 +96,11 @@ struct PeriodicDev {
     int block, odd, last, sign;
     double cs[4];
 };
-// one workgroup
-__global__ void k_periodic_flip(PeriodicDev *per, int nper, int *pitch_sign);
-__global__ void k_exchange(const BlockDev *blocks, const ExchDev *el, long n, const PeriodicDev *per);
+// sc: the scalars of each instance (outlet pressure); nbcg workgroups of boundary
+// items, one more when nflip > 0, then those of the exchange
+__global__ void k_boundary(const BlockDev *blocks, const PatchDev *patches, int npatch, const long *pstart, int nbcg,
+                           Gas g, const ScalarsDev *sc, const ExchDev *el, long nexch, PeriodicDev *per, int nflip,
+                           int *pitch_sign);
 // the CFL number of each block's instance: BlockDev::cfl
 __global__ void k_spectral_dt(const BlockDev *blocks, const long *cstart, int nblock, Gas g);
 __global__ void k_dt_flag_decrement(const BlockDev *blocks, int nblock);
