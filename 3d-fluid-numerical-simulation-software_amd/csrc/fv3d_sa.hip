@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(256) k_wall_distance(const BlockDev *__restric
 // sum of CMesh::ConvectiveFlux (source/ComputeAllBlockVars.cpp:109-114), the
 // WallFlux zero of the nu~ convection through walls (source/WallFlux.cpp:105,
 // 136, 167) and Res_ev = Fc_tur - Fv_tur (source/ComputeAllBlockVars.cpp:249).
-// A tile stages u v w T, nu~ (as it stands and clipped) and rho of its cells and
+// A tile stages nu~ (as it stands and clipped) and T of its cells and
 // a one-cell halo in LDS; every face of the tile is evaluated once: the face
 // gradient of nu~ (the shared 33-case rule), the upwind convection, the
 // diffusion (1 + c_b2)/sigma (nu + nu~) grad nu~ . S / Re and the plain
@@ -119,8 +119,8 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
 {
     using TL = VTile<TI, TJ, TK>;
     constexpr int NT = TI * TJ * TK, NH = TL::NH;
-    // planes: u v w T, nu~ as it stands, rho, nu~ clipped
-    __shared__ double sw[7 * NH];
+    // planes: nu~ as it stands, nu~ clipped, T
+    __shared__ double sw[3 * NH];
     __shared__ double sf[3 * TL::NF];   // convective, viscous, plain gradient flux
     const int4 tl = tiles[blockIdx.x];
     if (tl.x < 0) return;   // padding of the XCD-ordered tile list
@@ -135,14 +135,10 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
         const int ci = min(tl.y + hi, B.IM), cj = min(tl.z + hj, B.JM), ck = min(tl.w + hk, B.KM);
         const long x = cidx(B, ci, cj, ck);
         const double T = B.W[5 * box + x], rho = B.W[x], ev = B.ev[x];
-        sw[0 * NH + n] = B.W[1 * box + x];
-        sw[1 * NH + n] = B.W[2 * box + x];
-        sw[2 * NH + n] = B.W[3 * box + x];
-        sw[3 * NH + n] = T;
-        sw[4 * NH + n] = ev;
-        sw[5 * NH + n] = rho;
+        sw[0 * NH + n] = ev;
         const bool interior = ci >= 1 && ci <= B.ni && cj >= 1 && cj <= B.nj && ck >= 1 && ck <= B.nk;
-        sw[6 * NH + n] = interior ? sa_clip(ev, T, rho, g) : ev;
+        sw[1 * NH + n] = interior ? sa_clip(ev, T, rho, g) : ev;
+        sw[2 * NH + n] = T;
     }
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -155,19 +151,23 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
         const int l = TL::h(a + 1, b + 1, c + 1);
         const int st = D == 0 ? TL::HJ * TL::HK : D == 1 ? TL::HK : 1;
         const int lm = l - st;
+        const long x = cidx(B, i, j, k), xm = x - (D == 0 ? B.si : D == 1 ? B.sj : 1);
+        // rho u v w of the face's cells
+        double w1[4], w2[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) { w1[q] = B.W[q * box + xm]; w2[q] = B.W[q * box + x]; }
         double dv[3][1];
-        if (D == 0) face_dv<0, TL, 1>(sw + 4 * NH, l, i, j, k, B, dv);
-        else if (D == 1) face_dv<1, TL, 1>(sw + 4 * NH, l, i, j, k, B, dv);
-        else face_dv<2, TL, 1>(sw + 4 * NH, l, i, j, k, B, dv);
-        const long x = cidx(B, i, j, k);
+        if (D == 0) face_dv<0, TL, 1>(sw, l, i, j, k, B, dv);
+        else if (D == 1) face_dv<1, TL, 1>(sw, l, i, j, k, B, dv);
+        else face_dv<2, TL, 1>(sw, l, i, j, k, B, dv);
         const double *G = B.fg[D] + x;
         double gr[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) gr[q] = dv[0][0] * G[q * box] + dv[1][0] * G[(3 + q) * box] + dv[2][0] * G[(6 + q) * box];
         const double gx = gr[0], gy = D == 0 ? gr[0] : D == 1 ? gr[1] : gr[2], gz = D == 0 ? gr[0] : D == 1 ? gr[2] : gr[1];
-        const double densf = F32C(0.5) * (sw[5 * NH + l] + sw[5 * NH + lm]);
-        const double tempf = F32C(0.5) * (sw[3 * NH + l] + sw[3 * NH + lm]);
-        const double evf = F32C(0.5) * (sw[6 * NH + l] + sw[6 * NH + lm]);
+        const double densf = F32C(0.5) * (w2[0] + w1[0]);
+        const double tempf = F32C(0.5) * (sw[2 * NH + l] + sw[2 * NH + lm]);
+        const double evf = F32C(0.5) * (sw[NH + l] + sw[NH + lm]);
         const double ev_lam = Re * sutherland(g, tempf) / densf;
         const double tx = (F32C(1.0) + K.Cb2) / K.sigma * (ev_lam + evf) * gx;
         const double ty = (F32C(1.0) + K.Cb2) / K.sigma * (ev_lam + evf) * gy;
@@ -176,9 +176,9 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
         const double Sx = S[x], Sy = S[box + x], Sz = S[2 * box + x], s = B.fs[D][x];
         const DivBy bys(s);
         const double nx = bys.of(Sx), ny = bys.of(Sy), nz = bys.of(Sz);
-        const double Vn1 = sw[lm] * nx + sw[NH + lm] * ny + sw[2 * NH + lm] * nz;
-        const double Vn2 = sw[l] * nx + sw[NH + l] * ny + sw[2 * NH + l] * nz;
-        double fc = (F32C(0.5) * (Vn1 + fabs(Vn1)) * sw[6 * NH + lm] + F32C(0.5) * (Vn2 - fabs(Vn2)) * sw[6 * NH + l]) * s;
+        const double Vn1 = w1[1] * nx + w1[2] * ny + w1[3] * nz;
+        const double Vn2 = w2[1] * nx + w2[2] * ny + w2[3] * nz;
+        double fc = (F32C(0.5) * (Vn1 + fabs(Vn1)) * sw[NH + lm] + F32C(0.5) * (Vn2 - fabs(Vn2)) * sw[NH + l]) * s;
         // a wall face carries no nu~ convection
         const int p = D == 0 ? i : D == 1 ? j : k, N = D == 0 ? B.IM : D == 1 ? B.JM : B.KM;
         if (p == 1 || p == N) {
@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_sa_faces(const BlockDev *__restr
     const int fK0 = TL::NFI + TL::NFJ + (ti * TJ + tj) * (TK + 1) + tk, fK1 = fK0 + 1;
     const int l0 = TL::h(ti + 1, tj + 1, tk + 1);
     const long x = cidx(B, i, j, k);
-    const double ev = sw[6 * NH + l0], T = sw[3 * NH + l0], rho = sw[5 * NH + l0];
+    const double ev = sw[NH + l0], T = sw[2 * NH + l0], rho = B.W[x];
     const double ev_lam = Re * sutherland(g, T) / rho;
     const double X = ev / ev_lam;
     const double fv1 = sa_fv1(X, K.Cv1);
