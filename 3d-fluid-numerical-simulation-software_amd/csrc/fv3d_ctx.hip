@@ -98,7 +98,7 @@ struct fv3d_ctx {
     int2 *d_bl_walls = nullptr;
     std::vector<std::pair<int, long>> bl_launch;
     std::vector<int> bl_launch_n;
-    std::vector<int> bl_groups;
+    std::vector<int> bl_groups, bl_cells;   // form of k_bl_lines: groups per line, cells per thread
     long *d_pstart_bc = nullptr, *d_cstart = nullptr, *d_pstart_plane = nullptr;
     // residual tiles: one list per tile shape (built on first use), and the
     // shape each residual kernel uses (0 convective, 1 viscous, 2 nu~)
@@ -1281,7 +1281,7 @@ int fv3d_setup(fv3d_ctx *c)
         std::vector<int2> wl;
         for (int G = 16; G <= 64; G *= 2) {
             long lines = 0;
-            int n = 0, first = (int)wl.size();
+            int n = 0, first = (int)wl.size(), longest = 0;
             for (int q = 0; q < (int)pd.size(); ++q) {
                 if (c->patches[q].kind != 2) continue;
                 const PatchDev &P = pd[q];
@@ -1297,11 +1297,13 @@ int fv3d_setup(fv3d_ctx *c)
                 wl.push_back(make_int2(q, (int)nl));
                 lines += nl;
                 ++n;
+                longest = std::max(longest, len);
             }
             if (!n) continue;
             c->bl_launch.push_back({first, lines});
             c->bl_launch_n.push_back(n);
             c->bl_groups.push_back(G);
+            c->bl_cells.push_back(G == 16 && longest <= 32 ? 2 : G == 16 && longest <= 64 ? 4 : kBlCpt);
         }
         if (!wl.empty()) {
             if ((rc = dalloc(c, &c->d_bl_walls, wl.size()))) return rc;
@@ -1826,12 +1828,14 @@ static int launch_turbulence(fv3d_ctx *c, int save_old = 0, bool mut_only = fals
         const unsigned wgs = (unsigned)(c->bl_launch[r].second / kBlLines);
         const int2 *wl = c->d_bl_walls + c->bl_launch[r].first;
         const int G = c->bl_groups[r], n = c->bl_launch_n[r];
-        if (G == 16)
-            hipLaunchKernelGGL(k_bl_lines<16>, dim3(wgs), dim3(kBlLines * 16), 0, c->stream, c->d_blocks, c->d_patches, wl, n, c->gas);
-        else if (G == 32)
-            hipLaunchKernelGGL(k_bl_lines<32>, dim3(wgs), dim3(kBlLines * 32), 0, c->stream, c->d_blocks, c->d_patches, wl, n, c->gas);
-        else
-            hipLaunchKernelGGL(k_bl_lines<64>, dim3(wgs), dim3(kBlLines * 64), 0, c->stream, c->d_blocks, c->d_patches, wl, n, c->gas);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(wgs), dim3(kBlLines * G), 0, c->stream, c->d_blocks, c->d_patches, wl, n, c->gas);
+        };
+        if (G == 64) launch(k_bl_lines<64, 8>);
+        else if (G == 32) launch(k_bl_lines<32, 8>);
+        else if (c->bl_cells[r] == 8) launch(k_bl_lines<16, 8>);
+        else if (c->bl_cells[r] == 4) launch(k_bl_lines<16, 4>);
+        else launch(k_bl_lines<16, 2>);
     }
     if (!c->bl_launch.empty())
         hipLaunchKernelGGL(k_bl_merge, dim3((unsigned)((c->ncell + 255) / 256)), dim3(256), 0, c->stream, c->d_blocks,

@@ -214,13 +214,13 @@ __global__ void k_viscous(const BlockDev *blocks, const int4 *tiles, Gas g, int 
 // vorticity magnitude per cell
 __global__ void k_curl(const BlockDev *blocks, const long *cstart, int nblock);
 // Baldwin-Lomax along the grid lines normal to a set of wall patches:
-// kBlLines lines x G groups of kBlCpt cells per workgroup (so lines of up to
-// G*kBlCpt cells); walls[w] = (patch index, line count rounded up to a
+// kBlLines lines x G groups of C cells per workgroup (so lines of up to G*C
+// cells; C at most kBlCpt); walls[w] = (patch index, line count rounded up to a
 // multiple of kBlLines).  Each cell's value is folded into blmin with an
 // atomic minimum; k_bl_merge then moves the minima into mut.
 constexpr int kBlLines = 16, kBlCpt = 8;
 constexpr unsigned long long kBlUnvisited = ~0ull;
-template <int G>
+template <int G, int C>
 __global__ void k_bl_lines(const BlockDev *blocks, const PatchDev *patches, const int2 *walls, int nwalls, Gas g);
 __global__ void k_bl_merge(const BlockDev *blocks, const long *cstart, int nblock);
 

@@ -275,20 +275,23 @@ __global__ void k_curl(const BlockDev *__restrict__ blocks, const long *__restri
 // workgroup serves kBlLines grid lines normal to the wall that
 // are neighbours along their fastest tangential index (so a load of one cell
 // position is contiguous over the lines) and splits each line into G groups;
-// thread (group g, line l) holds the cells n0 = 1 + g + G c, c < kBlCpt, of its
-// line in registers.  The reference's sequential maxima become reductions
+// thread (group g, line l) holds the cells n0 = 1 + g + G c, c < C, of its
+// line in registers; C is the smallest form that holds the launch's longest
+// line, and the positions past a wall's lines are skipped: a position is three
+// powers and an exponential, and with all eight evaluated lines of 42 cells
+// took 62 us (307k-cell passage) at two waves per SIMD, now 35 at four.  The reference's sequential maxima become reductions
 // over the groups in LDS: tau_w and U_dif are plain maxima (NaN entries never
 // win, as with its strict comparisons; a NaN first entry is kept), and
 // (F_max, y_max) is the largest positive F with ties going to the smallest n0,
 // which is the first one its loop meets.  The first cell ends at zero; the
 // ghost cell gets zero and then the negated first-cell value, as WallFlux
 // writes it (source/WallFlux.cpp:106-110).
-template <int G>
+template <int G, int C>
 __global__ void __launch_bounds__(kBlLines *G) k_bl_lines(const BlockDev *__restrict__ blocks,
                                                           const PatchDev *__restrict__ patches,
                                                           const int2 *__restrict__ walls, int nwalls, Gas g)
 {
-    constexpr int L = kBlLines, C = kBlCpt;
+    constexpr int L = kBlLines;
     __shared__ double s_a[G][L], s_b[G][L];
     __shared__ int s_n[G][L];
     __shared__ double s_line[6][L];   // Tw, Udif, Ret, Fmax, y_max, Fwake
@@ -306,6 +309,7 @@ __global__ void __launch_bounds__(kBlLines *G) k_bl_lines(const BlockDev *__rest
     const int D = P.dir, hi = P.hi;
     const int N = D == 0 ? B.IM : D == 1 ? B.JM : B.KM;
     const int M = D == 0 ? B.IM : B.JM;   // line length of the reference's call (K walls need JM == KM)
+    const int nc = __builtin_amdgcn_readfirstlane((M - 2 + G) / G);   // cells of the line per thread
     const long box = B.box;
     auto cell = [&](int n0) -> long {
         const int n = hi ? N - n0 : n0;
@@ -321,6 +325,8 @@ __global__ void __launch_bounds__(kBlLines *G) k_bl_lines(const BlockDev *__rest
     double tw = -1.0, ud = 0.0, t1 = 0.0, d1 = 0.0, m1 = 0.0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
+        ok[c] = false;
+        if (c >= nc) continue;
         const int n0 = 1 + grp + G * c;
         ok[c] = active && n0 < M;
         const long x = cell(ok[c] ? n0 : 1);
@@ -361,6 +367,7 @@ __global__ void __launch_bounds__(kBlLines *G) k_bl_lines(const BlockDev *__rest
     int bN = 1 << 30;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
+        if (c >= nc) continue;
         const double y_plus = dis[c] * Ret;
         damp[c] = F32C(1.0) - exp(-y_plus / A_plus);
         const double F = dis[c] * fabs(om[c]) * damp[c];
@@ -427,8 +434,12 @@ __global__ void __launch_bounds__(256) k_bl_merge(const BlockDev *__restrict__ b
     }
 }
 
-template __global__ void k_bl_lines<16>(const BlockDev *, const PatchDev *, const int2 *, int, Gas);
-template __global__ void k_bl_lines<32>(const BlockDev *, const PatchDev *, const int2 *, int, Gas);
-template __global__ void k_bl_lines<64>(const BlockDev *, const PatchDev *, const int2 *, int, Gas);
+#define FV3D_BL(G, C) template __global__ void k_bl_lines<G, C>(const BlockDev *, const PatchDev *, const int2 *, int, Gas);
+FV3D_BL(16, 2)
+FV3D_BL(16, 4)
+FV3D_BL(16, 8)
+FV3D_BL(32, 8)
+FV3D_BL(64, 8)
+#undef FV3D_BL
 
 }  // namespace fv3d
