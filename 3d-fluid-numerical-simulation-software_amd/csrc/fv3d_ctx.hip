@@ -41,7 +41,7 @@ struct HostBlock {
     BlockDev dev;                // device pointers + dims
     std::vector<void *> allocs;
     long sweep_rows = 0;         // rows of the tile-skewed sweep layout
-    long pack_groups = 0;        // (tile, chunk) items of k_sweep_pack / k_sweep_unpack
+    long pack_groups = 0;        // (tile, chunk) items of k_sweep_pack
 };
 
 // An independent passage of a batched context: its blocks are
@@ -1888,10 +1888,10 @@ static int launch_sweeps_kba(fv3d_ctx *c)
         // rows packed per cell, increments per cell, and the split of each
         // (tile, chunk) item over workgroups: about 8192 workgroups per launch,
         // so that a coarse level's few tiles still spread over the chip
-        const int nq = sa ? 21 : visc ? 18 : 15, ncomp = sa ? 6 : 5;
+        const int nq = sa ? 21 : visc ? 18 : 15;
         const long per = c->pack_groups > 0 ? std::max(1L, (8192 + c->pack_groups - 1) / c->pack_groups) : 1;
-        const int qs = (int)std::min<long>(nq, per), cs = (int)std::min<long>(ncomp, per);
-        const unsigned pgq = (unsigned)(c->pack_groups * qs), pgc = (unsigned)(c->pack_groups * cs);
+        const int qs = (int)std::min<long>(nq, per);
+        const unsigned pgq = (unsigned)(c->pack_groups * qs);
         const unsigned pgf = (unsigned)((c->mbox_fill + kFillWords - 1) / kFillWords);
         if (f32) {
             hipLaunchKernelGGL(k_sweep_pack<float>, dim3(pgq + pgf), dim3(256), 0, c->stream, c->d_blocks, c->d_pack_start,
@@ -1905,7 +1905,7 @@ static int launch_sweeps_kba(fv3d_ctx *c)
         auto sweep = [&](bool fwd) {
             int *tk = fwd ? tf : tb, *nt = fwd ? tb : tf;
             const KbaTile *tl = c->d_kba[fwd ? 0 : 1];
-            dim3 g((unsigned)c->kba_grid), b(kSlThreads);
+            dim3 g((unsigned)c->kba_grid), b((unsigned)sl_threads(fwd));
 #define FV3D_SL_LAUNCH(F, V, S, T) \
     hipLaunchKernelGGL((k_lusgs_sl<F, kKbaTJ, kKbaTK, V, S, T>), g, b, 0, c->stream, c->d_blocks, tl, c->nkba, tk, nt, err, \
                        c->gas.relax, c->gas)
@@ -1925,20 +1925,11 @@ static int launch_sweeps_kba(fv3d_ctx *c)
 #undef FV3D_SL_FORMS
 #undef FV3D_SL_LAUNCH
         };
-        auto unpack = [&]() {
-            if (f32)
-                hipLaunchKernelGGL(k_sweep_unpack<float>, dim3(pgc), dim3(256), 0, c->stream, c->d_blocks, c->d_pack_start, nb,
-                                   ncomp, cs);
-            else
-                hipLaunchKernelGGL(k_sweep_unpack<double>, dim3(pgc), dim3(256), 0, c->stream, c->d_blocks, c->d_pack_start, nb,
-                                   ncomp, cs);
-        };
         if (c->timing) HIPCK(c, hipEventRecord(c->ev[6], c->stream));
         sweep(true);
         if (c->timing) HIPCK(c, hipEventRecord(c->ev[7], c->stream));
         sweep(false);
         if (c->timing) HIPCK(c, hipEventRecord(c->ev[8], c->stream));
-        unpack();
     }
     HIPCK(c, hipGetLastError());
     return FV3D_OK;
@@ -2368,8 +2359,8 @@ static int accumulate_timing(fv3d_ctx *c)
 {
     HIPCK(c, hipEventSynchronize(c->ev[5]));
     float ms;
-    // slots: 0 residual (convective + viscous), 1 LU-SGS operator (pack, sweeps,
-    // unpack), 2 update, 3 ghost fill + turbulence + spectral radii and dt,
+    // slots: 0 residual (convective + viscous), 1 LU-SGS operator (pack,
+    // sweeps), 2 update, 3 ghost fill + turbulence + spectral radii and dt,
     // 4 finalize, 5/6 forward/backward sweep kernels, 7 the cycle's coarse
     // correction (second fine residual, transfers, coarse levels), 8 convective
     // residual kernel, 9 viscous (and nu~) residual kernels, 10 ghost fill and

@@ -130,8 +130,8 @@ constexpr int kSweepD = 6;
 // what k_sweep_fill writes: the state quantities and/or the static metrics
 constexpr int kGatherState = 1, kGatherMetrics = 2;
 // threads per workgroup of k_lusgs_sl: three direction waves, the mailbox wave,
-// three combine waves
-constexpr int kSlThreads = 448;
+// three combine waves, backward the store wave
+__host__ __device__ constexpr int sl_threads(bool fwd) { return fwd ? 448 : 512; }
 // T: double (plain FP64) or float (the FP32 operator of defect correction)
 // SA: the nu~ equation in the same sweep (Navier-Stokes only)
 template <bool FWD, int TJ, int TK, bool VISC, bool SA, class T>
@@ -146,7 +146,7 @@ constexpr unsigned int kMboxEmpty32 = 0x7fa5eed1u;   // the same for FP32 words
 __global__ void k_fill_u64(unsigned long long *p, long n, unsigned long long v);
 __global__ void k_fill_i32(int *p, int n, int v);
 __global__ void k_prim_all(const BlockDev *blocks, const long *cstart, int nblock, Gas g, int *bad_flag);
-// row storage in T (double, or float for the FP32 operator); unpack widens dQ to double
+// row storage in T (double, or float for the FP32 operator); the backward sweep widens dQ to double
 template <class T>
 __global__ void k_sweep_fill(const BlockDev *blocks, int block, long nrows, int what);
 // one launch over all blocks: (tile, chunk) items gstart[n] .. gstart[n+1]-1
@@ -159,11 +159,7 @@ constexpr int kFillWords = 2048;
 template <class T>
 __global__ void k_sweep_pack(const BlockDev *blocks, const long *gstart, int nblock, int nq, int qsplit, unsigned npack,
                              uint4 *mbox, long nfill);
-// nc: components per cell (5, or 6 with the nu~ increment), split over csplit
-// workgroups per item
-template <class T>
-__global__ void k_sweep_unpack(const BlockDev *blocks, const long *gstart, int nblock, int nc, int csplit);
-constexpr int kPackChunk = 16;   // i-planes per k_sweep_pack / k_sweep_unpack workgroup
+constexpr int kPackChunk = 16;   // i-planes per k_sweep_pack workgroup
 constexpr int kSecParts = 32;    // workgroups per section in k_sections
 __global__ void k_fill_int(int *p, long n, int v);
 __global__ void k_field_rows(const double *src, long box, int C, int si, int sj, int lo, int n2, int n3, long t0, long n,

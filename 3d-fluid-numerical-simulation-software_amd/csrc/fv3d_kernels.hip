@@ -733,8 +733,8 @@ __device__ inline T *mbox_base(BlockRef B, bool fwd) { return (T *)B.mbox[fwd ? 
 // Lane (tj,tk) of row r of tile (J,K) is cell (r+1-tj-tk, J*TJ+tj+1, K*TK+tk+1).
 // k_sweep_fill writes whole rows, one wave per row, giving lanes outside the
 // block a harmless unit state; it runs at set-up (metrics and those lanes).
-// Each iteration k_sweep_pack copies the state of the cells in, and after the
-// sweeps k_sweep_unpack copies dQ back to the cell box.
+// Each iteration k_sweep_pack copies the state of the cells in; the backward
+// sweep leaves its dQ in the cell box.
 template <class T>
 __global__ void __launch_bounds__(256) k_sweep_fill(const BlockDev *__restrict__ blocks, int block, long nrows, int what)
 {
@@ -777,7 +777,7 @@ __device__ inline long xcd_item(long b, long n)
     for (long y = 0; y < x; ++y) start += (n - y + 7) / 8;   // items of the XCDs before x
     return start + b / 8;
 }
-// (tile, chunk) of pack/unpack work item wg of a block: k tiles fastest, then
+// (tile, chunk) of pack work item wg of a block: k tiles fastest, then
 // chunks of i, then j tiles, so consecutive items are neighbours along k (they
 // share the cell-box lines at their k edges) and items ntk apart neighbours
 // along i (they share the partly written rows at their chunk edges)
@@ -857,51 +857,10 @@ __global__ void __launch_bounds__(256) k_sweep_pack(const BlockDev *__restrict__
     }
 }
 
-// The reverse of k_sweep_pack for dQ (and dnu~), components split into
-// csplit groups the same way.
-template <class T>
-__global__ void __launch_bounds__(256) k_sweep_unpack(const BlockDev *__restrict__ blocks, const long *__restrict__ gstart,
-                                                      int nblock, int nc, int csplit)
-{
-    constexpr int TJ = kKbaTJ, TK = kKbaTK;
-    __shared__ double buf[kPackChunk][64];
-    // the block of this workgroup: gstart holds the running (tile, chunk) counts
-    const long item = xcd_item(blockIdx.x, gridDim.x);
-    const int cg = (int)(item % csplit);
-    const int block = find_range(gstart, nblock, item / csplit);
-    BlockRef B = block_at(blocks, block);
-    const long wg = item / csplit - gstart[block];
-    const int nchunk = (B.ni + kPackChunk - 1) / kPackChunk;
-    int slot, i0;
-    pack_item(B, wg, nchunk, slot, i0);
-    const int J = slot / B.ntk, K = slot % B.ntk;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int tj = lane / TK, tk = lane % TK, j = J * TJ + tj + 1, k = K * TK + tk + 1;
-    const bool col = j <= B.nj && k <= B.nk;
-    const long box = B.box;
-    const int NC = nc;   // 6: dnu~ too (the nu~ equation in the sweep)
-    for (int c = cg * NC / csplit; c < (cg + 1) * NC / csplit; ++c) {
-        for (int rr = w; rr < kPackChunk + TJ + TK - 2; rr += 4) {
-            const int r = i0 - 1 + rr, i = r + 1 - tj - tk;
-            if (col && i >= i0 && i < i0 + kPackChunk && i <= B.ni)
-                buf[i - i0][lane] = (double)((const T *)B.sdq)[((long)slot * B.nr + r) * (kSweepD * 64) + c * 64 + lane];
-        }
-        __syncthreads();
-        double *dst = c < 5 ? B.dQ + c * box : B.dev;
-        for (int ci = w; ci < kPackChunk; ci += 4) {
-            const int i = i0 + ci;
-            if (col && i <= B.ni) dst[cidx(B, i, j, k)] = buf[ci][lane];
-        }
-        __syncthreads();
-    }
-}
-
 template __global__ void k_sweep_fill<double>(const BlockDev *, int, long, int);
 template __global__ void k_sweep_fill<float>(const BlockDev *, int, long, int);
 template __global__ void k_sweep_pack<double>(const BlockDev *, const long *, int, int, int, unsigned, uint4 *, long);
 template __global__ void k_sweep_pack<float>(const BlockDev *, const long *, int, int, int, unsigned, uint4 *, long);
-template __global__ void k_sweep_unpack<double>(const BlockDev *, const long *, int, int, int);
-template __global__ void k_sweep_unpack<float>(const BlockDev *, const long *, int, int, int);
 
 // The persistent wavefront form of the sweeps, on the tile-skewed layout.  The
 // (j,k) cross-section is cut into 4 x 16 tiles, one workgroup per tile; tiles
@@ -919,8 +878,15 @@ template __global__ void k_sweep_unpack<float>(const BlockDev *, const long *, i
 //     ahead of its step, waits for it (bounded) and leaves it in LDS
 //     beside the in-tile dQ, so a direction wave reads both alike;
 //   waves 4, 5, 6 (combine): each sums two of the components into dQ, keeps dQ in
-//     LDS for the next step and stores it; the right-hand side, the diagonal
-//     and its reciprocal are ready before the terms are.
+//     LDS for the next step and stores it (backward: in a ring of the last
+//     steps); the right-hand side, the diagonal and its reciprocal are ready
+//     before the terms are;
+//   wave 7 (store, backward only): dQ back to the cell box.  A plane i of the tile
+//     is spread over nineteen steps; when the last of them is in the ring the plane
+//     goes out as runs of sixteen cells.  It takes the place of a launch that
+//     read the dQ rows back and wrote the box: backward sweep and that launch of the 1.05M-cell
+//     channel 320 -> 306 us (FP64), of 2.54M cells 325 -> 314 us (FP32).  The
+//     combine waves writing their 64 cells' lines themselves: 441 us.
 // Two barriers a step: the terms are in LDS, dQ is in LDS.  With three direction
 // waves and one combine wave, each doing its own loads and waits, a step took
 // 1.03 us (FP64) and 0.58 us (FP32); it takes 0.58 and 0.40 us.  Forward sweep: 96x32x32
@@ -943,7 +909,7 @@ template __global__ void k_sweep_unpack<float>(const BlockDev *, const long *, i
 // updates both per cell from the same neighbour increments, so this is its
 // order.
 template <bool FWD, int TJ, int TK, bool VISC, bool SA, class T>
-__global__ void __launch_bounds__(kSlThreads) k_lusgs_sl(const BlockDev *__restrict__ blocks, const KbaTile *__restrict__ tiles,
+__global__ void __launch_bounds__(sl_threads(FWD)) k_lusgs_sl(const BlockDev *__restrict__ blocks, const KbaTile *__restrict__ tiles,
                                                          int ntiles, int *__restrict__ ticket,
                                                          int *__restrict__ next_ticket, int *__restrict__ err,
                                                          double relax, Gas g)
@@ -970,6 +936,9 @@ __global__ void __launch_bounds__(kSlThreads) k_lusgs_sl(const BlockDev *__restr
     __shared__ Pair sA[kWide && VISC ? 1 : 3][3][64];
     __shared__ Pair sV[!kWide && VISC ? 3 : 1][3][64];
     __shared__ Quad sAV[kWide && VISC ? 3 : 1][3][64];
+    // the final dQ of the last steps, from which the store wave takes planes
+    constexpr int kStore = TJ + TK;   // a plane's cells spread over kStore - 1 steps
+    __shared__ T ring[FWD ? 1 : kStore][NC][64];
     __shared__ int s_q;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int tj = lane / TK, tk = lane % TK;
@@ -1260,6 +1229,7 @@ __global__ void __launch_bounds__(kSlThreads) k_lusgs_sl(const BlockDev *__restr
                 }
             };
             Rhs b[kRing] = {};
+            int slot_now = 0;   // of the step in the ring
             __builtin_amdgcn_s_waitcnt(0);
             for (int s0 = kRowS0; s0 < send; s0 += kRing) {
 #pragma unroll
@@ -1307,10 +1277,43 @@ __global__ void __launch_bounds__(kSlThreads) k_lusgs_sl(const BlockDev *__restr
                             for (int c = 0; c < N; ++c)
                                 __hip_atomic_store(mb + kMboxJ + tj + (C0 + c) * TJ, out[c], __ATOMIC_RELAXED,
                                                    __HIP_MEMORY_SCOPE_AGENT);
-                        for (int c = 0; c < N; ++c) drows[(long)ro * RD + (C0 + c) * 64 + lane] = out[c];
+                        for (int c = 0; c < N; ++c) {
+                            if constexpr (FWD) drows[(long)ro * RD + (C0 + c) * 64 + lane] = out[c];
+                            else ring[slot_now][C0 + c][lane] = out[c];
+                        }
                     }
+                    slot_now = slot_now == kStore - 1 ? 0 : slot_now + 1;
                 }
             }
+        };
+        // ---- store wave (backward): the cells of plane i, each from the step that
+        // formed it, into the cell box, once the last of them is in the ring
+        auto store_loop = [&]() {
+            double *const dst = B.dQ + cidx(B, 0, j, k);
+            int sl = lj + lk + 1;   // ring slot of this lane's cell of the plane
+            T v[NC];
+            auto fetch = [&]() {
+                for (int c = 0; c < NC; ++c) v[c] = ring[sl][c][lane];
+                sl = sl == kStore - 1 ? 0 : sl + 1;
+            };
+            auto put = [&](int s) {
+                const int i = ni + kStore - 1 - s;
+                if (col && i >= 1 && i <= ni) {
+                    const long x = (long)i * B.si;
+                    for (int c = 0; c < 5; ++c) dst[c * B.box + x] = (double)v[c];
+                    if constexpr (SA) B.dev[cidx(B, 0, j, k) + x] = (double)v[5];
+                }
+            };
+            // the stores go out beside the direction waves, the longer half of a step
+            for (int s = kRowS0; s < send; ++s) {
+                bar();
+                fetch();
+                bar();
+                put(s);
+            }
+            bar();
+            fetch();
+            put(send);
         };
         if (wave == 0) dir_loop(Int<0>());
         else if (wave == 1) dir_loop(Int<1>());
@@ -1318,7 +1321,10 @@ __global__ void __launch_bounds__(kSlThreads) k_lusgs_sl(const BlockDev *__restr
         else if (wave == 3) mail_loop();
         else if (wave == 4) combine_loop(Int<0>());
         else if (wave == 5) combine_loop(Int<1>());
-        else combine_loop(Int<2>());
+        else if (wave == 6) combine_loop(Int<2>());
+        else if constexpr (!FWD) store_loop();
+        if constexpr (!FWD)
+            if (wave < 7) bar();   // the store wave's last plane
     }
 }
 
