@@ -1723,15 +1723,19 @@ static int launch_convective(fv3d_ctx *c, bool dec = false)
     }
     const int q = c->tile_sel[0] < kNumTiles ? c->tile_sel[0] : 0;
     if (!c->d_tiles_s[q]) return fail(c, FV3D_ESTATE, "convective tiles of shape %d not built", q);
-    const dim3 g((unsigned)c->ntiles_s[q]), b(256);
-    switch (3 * q + mode) {
-#define FV3D_CONV_M(S, M, A, B, C)                                                                               \
+    const dim3 g((unsigned)c->ntiles_s[q]);
+    const bool wide = q == 0 && c->ntiles_s[q] <= kWideConv;
+    switch (wide ? kNumTiles * 3 + mode : 3 * q + mode) {
+#define FV3D_CONV_M(S, M, A, B, C, NT)                                                                           \
     case 3 * S + M:                                                                                               \
-        hipLaunchKernelGGL((k_convective<A, B, C, M>), g, b, 0, c->stream, c->d_blocks, c->d_tiles_s[q], c->gas,    \
-                           ndec, c->store_faces, c->d_faces[0], c->d_faces[1], c->d_faces[2]);                         \
+        hipLaunchKernelGGL((k_convective<A, B, C, M, NT>), g, dim3(NT), 0, c->stream, c->d_blocks, c->d_tiles_s[q],  \
+                           c->gas, ndec, c->store_faces, c->d_faces[0], c->d_faces[1], c->d_faces[2]);            \
         break;
-#define FV3D_CONV(S, A, B, C) FV3D_CONV_M(S, 0, A, B, C) FV3D_CONV_M(S, 1, A, B, C) FV3D_CONV_M(S, 2, A, B, C)
+#define FV3D_CONV(S, A, B, C) FV3D_CONV_M(S, 0, A, B, C, 256) FV3D_CONV_M(S, 1, A, B, C, 256) FV3D_CONV_M(S, 2, A, B, C, 256)
         FV3D_FOR_TILES(FV3D_CONV)
+        FV3D_CONV_M(kNumTiles, 0, 4, 4, 16, conv_wide(0))
+        FV3D_CONV_M(kNumTiles, 1, 4, 4, 16, conv_wide(1))
+        FV3D_CONV_M(kNumTiles, 2, 4, 4, 16, conv_wide(2))
 #undef FV3D_CONV
 #undef FV3D_CONV_M
     }
@@ -1745,7 +1749,7 @@ static int launch_viscous(fv3d_ctx *c)
 {
     if (!c->cfg.viscous) return FV3D_OK;
     const int q = c->tile_sel[1];
-    const dim3 g((unsigned)c->ntiles_s[q]), b(256);
+    const dim3 g((unsigned)c->ntiles_s[q]), b(c->ntiles_s[q] <= kWideVisc ? kViscThreads : 256);
     switch (q) {
 #define FV3D_VISC(S, A, B, C)                                                                                    \
     case S:                                                                                                       \

@@ -104,8 +104,16 @@ __global__ void k_boundary(const BlockDev *blocks, const PatchDev *patches, int 
 // the CFL number of each block's instance: BlockDev::cfl
 __global__ void k_spectral_dt(const BlockDev *blocks, const long *cstart, int nblock, Gas g);
 __global__ void k_dt_flag_decrement(const BlockDev *blocks, int nblock);
+// A residual tile is 256 cells and at most 16 groups of 64 faces.  A workgroup of
+// 256 threads takes the groups in four rounds; on a small grid more waves take
+// them in one or two, as many as the kernel's registers allow, which fill a CU.
+// k_convective (tiles of shape 0): up to two tiles a CU, 384 tiles 28.8 -> 26.3 us.
+// k_viscous: up to one, 56 tiles 23 -> 13 us, but 288 tiles 23 -> 26.
+constexpr int kWideConv = 512, kWideVisc = 256;
+__host__ __device__ constexpr int conv_wide(int mode) { return mode == 2 ? 768 : 1024; }
+constexpr int kViscThreads = 768;
 // MODE: the reconstruction's variables, 0 primitive, 1 conservative, 2 characteristic
-template <int TI, int TJ, int TK, int MODE>
+template <int TI, int TJ, int TK, int MODE, int NT>
 __global__ void k_convective(const BlockDev *blocks, const int4 *tiles, Gas g, int ndec, int store_faces, double *fI,
                              double *fJ, double *fK);
 // fstart: running face counts per (block, direction), 3 * nblock entries + 1

@@ -464,8 +464,13 @@ __device__ static void face_flux(BlockRef B, const Gas &g, int d, int i, int j, 
 // reconstruction per kernel the face code fits 128 registers and four waves per
 // SIMD: 494 -> 467 us, 201 -> 188 us (the characteristic one needs 166 and
 // keeps three).
-template <int TI, int TJ, int TK, int MODE>
-__global__ void __launch_bounds__(TI *TJ *TK) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 3 : 4)))
+// On a small grid the time is one workgroup's rounds of face code: with NT threads,
+// as many as the registers allow, the groups take one round (two for the
+// characteristic form) instead of four: 19 -> 12 us on 576 cells, 28.8 -> 26.3
+// on 98k (384 tiles).  The kernel of 256 threads stays for the others: built for up to 1024
+// it spills more and is 4 % slower on 1M cells.
+template <int TI, int TJ, int TK, int MODE, int NT>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(MODE == 2 ? 3 : 4)))
 k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles, Gas g, int ndec, int store_faces,
              double *fI0, double *fJ0, double *fK0)
 {
@@ -483,7 +488,7 @@ k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles
     // one copy of the face code in a rolled loop: a copy per direction (every
     // scheme and both fluxes) would crowd the instruction cache
 #pragma nounroll
-    for (int q = wave; q < GI + GJ + GK; q += TI * TJ * TK / 64) {
+    for (int q = wave; q < GI + GJ + GK; q += NT / 64) {
         const int d = q < GI ? 0 : q < GI + GJ ? 1 : 2;
         const int f = (q - (d == 0 ? 0 : d == 1 ? GI : GI + GJ)) * 64 + lane;   // face number within its direction
         // place in the tile; the divisors are constants in each branch
@@ -500,6 +505,7 @@ k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles
         for (int e = 0; e < 5; ++e) dst[e * n] = out[e];
     }
     __syncthreads();
+    if (t >= TI * TJ * TK) return;
     const int tk = t % TK, tj = (t / TK) % TJ, ti = t / (TK * TJ);
     const int i = tl.y + ti + 1, j = tl.z + tj + 1, k = tl.w + tk + 1;
     if (i > B.ni || j > B.nj || k > B.nk) return;
@@ -530,11 +536,14 @@ k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles
     }
 }
 
-#define FV3D_CONV_M(M, A, B, C) \
-    template __global__ void k_convective<A, B, C, M>(const BlockDev *, const int4 *, Gas, int, int, double *, double *, \
-                                                      double *);
-#define FV3D_CONV(S, A, B, C) FV3D_CONV_M(0, A, B, C) FV3D_CONV_M(1, A, B, C) FV3D_CONV_M(2, A, B, C)
+#define FV3D_CONV_M(M, A, B, C, NT) \
+    template __global__ void k_convective<A, B, C, M, NT>(const BlockDev *, const int4 *, Gas, int, int, double *, double *, \
+                                                          double *);
+#define FV3D_CONV(S, A, B, C) FV3D_CONV_M(0, A, B, C, 256) FV3D_CONV_M(1, A, B, C, 256) FV3D_CONV_M(2, A, B, C, 256)
 FV3D_FOR_TILES(FV3D_CONV)
+FV3D_CONV_M(0, 4, 4, 16, conv_wide(0))
+FV3D_CONV_M(1, 4, 4, 16, conv_wide(1))
+FV3D_CONV_M(2, 4, 4, 16, conv_wide(2))
 #undef FV3D_CONV
 #undef FV3D_CONV_M
 

@@ -162,11 +162,12 @@ __device__ static void face_fv(const double *sw, int l, int i, int j, int k, Blo
 }
 
 template <int TI, int TJ, int TK>
-__global__ void __launch_bounds__(TI *TJ *TK) k_viscous(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles,
-                                                        Gas g, int store, ViscDebug dbg)
+__global__ void __launch_bounds__(kViscThreads) k_viscous(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles,
+                                                          Gas g, int store, ViscDebug dbg)
 {
     using TL = VTile<TI, TJ, TK>;
-    constexpr int NT = TI * TJ * TK, NH = TL::NH;
+    constexpr int NH = TL::NH;
+    const int NT = blockDim.x;
     __shared__ double sw[4 * NH];
     // momentum and energy components of the face fluxes; the continuity
     // component of the viscous flux is zero on every face (F1 = 0,
@@ -211,6 +212,7 @@ __global__ void __launch_bounds__(TI *TJ *TK) k_viscous(const BlockDev *__restri
             for (int q = 0; q < 5; ++q) dbg.fv[D][q * box + x] = o[q];
     }
     __syncthreads();
+    if (t >= TI * TJ * TK) return;
     // cell sums (source/ViscousFlux.cpp:268-280) and Res = Fc - Fv - Fd with Fd = 0
     // (source/ComputeAllBlockVars.cpp:245)
     const int tk = t % TK, tj = (t / TK) % TJ, ti = t / (TK * TJ);
