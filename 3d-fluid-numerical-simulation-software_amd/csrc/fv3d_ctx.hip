@@ -2089,7 +2089,7 @@ static int instance_perf(fv3d_ctx *c, int w, double *out5)
     HIPCK(c, hipMemcpyAsync(part, c->d_sums + (size_t)w * 2 * 3 * kSecParts, sizeof part, hipMemcpyDeviceToHost,
                             c->stream));
     HIPCK(c, hipStreamSynchronize(c->stream));
-    // the partials in the order k_finalize adds them
+    // the partials in the order k_finish adds them
     double s[6] = {0, 0, 0, 0, 0, 0};
     for (int sec = 0; sec < 2; ++sec)
         for (int p = 0; p < kSecParts; ++p)

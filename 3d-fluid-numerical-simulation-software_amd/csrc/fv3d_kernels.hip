@@ -499,7 +499,13 @@ k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles
         const int i = tl.y + a + 1, j = tl.z + b + 1, k = tl.w + c + 1;   // the face's higher cell
         if (a >= TI + (d == 0) || i > B.ni + (d == 0) || j > B.nj + (d == 1) || k > B.nk + (d == 2)) continue;
         double out[5];
-        face_flux<MODE>(B, g, d, i, j, k, out);
+        // gamma anew each time round: what depends on it alone is a few
+        // instructions, but kept across the loop it takes the registers that the
+        // face code then spills (1.03 GB moved instead of 0.78 on 2.54M cells,
+        // 431 -> 393 us; 1.05M cells 159 -> 153)
+        Gas gl = g;
+        asm volatile("" : "+s"(gl.gamma));
+        face_flux<MODE>(B, gl, d, i, j, k, out);
         double *dst = (d == 0 ? &sI[0][0][0][0] : d == 1 ? &sJ[0][0][0][0] : &sK[0][0][0][0]) + f;
         const int n = d == 0 ? NFI : d == 1 ? NFJ : NFK;
         for (int e = 0; e < 5; ++e) dst[e * n] = out[e];
@@ -900,7 +906,7 @@ template __global__ void k_sweep_pack<float>(const BlockDev *, const long *, int
 // waves and one combine wave, each doing its own loads and waits, a step took
 // 1.03 us (FP64) and 0.58 us (FP32); it takes 0.58 and 0.40 us.  Forward sweep: 96x32x32
 // channel 188 -> 115 us (FP64), 127 -> 83 us (FP32); 1.05M-cell channel 511 -> 323 and
-// 348 -> 248 us; 2.54M-cell five-block passage with nu~ 735 -> 435 and 398 -> 275 us.
+// 348 -> 220 us; 2.54M-cell five-block passage with nu~ 735 -> 435 and 398 -> 275 us.
 // Every load is issued unconditionally with clamped indices, so the compiler's
 // memory-counter waits are exact.  The per-hyperplane kernel k_lusgs_plane above is the reference's own
 // schedule and gives the same bits.
@@ -1185,7 +1191,8 @@ __global__ void __launch_bounds__(sl_threads(FWD)) k_lusgs_sl(const BlockDev *__
             // reading later (between the barriers) holds up every step.
             // Measured, forward sweep, FP64 / FP32: 1.05M-cell channel 321 / 248 us
             // as here, 335 / 220 a step earlier, 410 / 305 later; 96x32x32 channel
-            // 111 / 82, 120 / 86, 112 / 87.
+            // 111 / 82, 120 / 86, 112 / 87.  (All with FP32 rows of FP64 length; at
+            // half of it, as now, the 1.05M cells take 220 us as here.)
             T x[2] = {};
             __builtin_amdgcn_s_waitcnt(0);
             for (int s = kRowS0; s < send; ++s) {
