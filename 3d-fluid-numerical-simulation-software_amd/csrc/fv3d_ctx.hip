@@ -83,8 +83,7 @@ struct fv3d_ctx {
     ExchDev *d_exch = nullptr;
     long nexch = 0;
     PeriodicDev *d_per = nullptr;
-    int nper = 0;
-    int nflip = 0;               // nper if any periodic patch flips its sign, else 0
+    int nflip = 0;               // the periodic patches if any flips its sign, else 0
     int *d_pitch_sign = nullptr;
     std::vector<PatchDev> pd_host;   // the device patch list, host copy
     double *d_mbox = nullptr;         // sweep mailboxes of all blocks
@@ -664,10 +663,9 @@ static int build_exchange(fv3d_ctx *c)
             }
         }
     c->nexch = (long)el.size();
-    c->nper = (int)per.size();
     c->nflip = 0;
     for (const PeriodicDev &p : per)
-        if (p.odd) c->nflip = c->nper;
+        if (p.odd) c->nflip = (int)per.size();
     int rc;
     if (!c->mixes.empty()) {
         std::vector<MixDev> ml;

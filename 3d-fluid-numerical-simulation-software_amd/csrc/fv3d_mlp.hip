@@ -33,69 +33,6 @@ __device__ inline f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c)
 __device__ inline float softplus(float z) { return z > 20.0f ? z : log1pf(expf(z)); }
 __device__ inline float sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
 
-// One wave: rows r0 .. r0+15 of the activation tile in (row stride kHS,
-// columns 0..63) times the weight matrix W (row n = output, 64 inputs, FP32
-// in global memory, quantised to BF16 here), plus bias, tanh, into out.
-__device__ inline void dense64(const float *in, int r0, const float *W, const float *b, float *out, int lane)
-{
-    const int row = lane & 15, kb = lane >> 4;
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        const int n = nt * 16 + row;
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            bf16x8 a, w;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int k = 32 * ks + 8 * kb + j;
-                a[j] = (__bf16)in[(r0 + row) * kHS + k];
-                w[j] = (__bf16)W[n * kMlpH + k];
-            }
-            acc = mfma16(a, w, acc);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) out[(r0 + 4 * kb + i) * kHS + n] = tanhf(acc[i] + b[n]);
-    }
-}
-
-// The forward pass of one wave's 16 samples (rows r0..r0+15): x (row stride
-// kMlpXS, features 0..5) -> h0, h1, h2 (tanh activations, FP32 in LDS) -> z
-// (pre-softplus output) for lanes 0..15.
-__device__ inline float mlp_forward16(const float *P, const float *x, float *h0, float *h1, float *h2, int r0,
-                                      int lane)
-{
-    const int row = lane & 15, kb = lane >> 4;
-    // layer 0: K = 6 features in the first 8-wide slice, zero elsewhere
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        const int n = nt * 16 + row;
-        bf16x8 a, w;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const bool in = kb == 0 && j < kMlpIn;
-            a[j] = (__bf16)(in ? x[(r0 + row) * kMlpXS + j] : 0.0f);
-            w[j] = (__bf16)(in ? P[kMlpW0 + n * kMlpIn + j] : 0.0f);
-        }
-        acc = mfma16(a, w, acc);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) h0[(r0 + 4 * kb + i) * kHS + n] = tanhf(acc[i] + P[kMlpB0 + n]);
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    dense64(h0, r0, P + kMlpW1, P + kMlpB1, h1, lane);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    dense64(h1, r0, P + kMlpW2, P + kMlpB2, h2, lane);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    float z = P[kMlpB3];
-    if (lane < 16)
-        for (int k = 0; k < kMlpH; ++k) z += h2[(r0 + lane) * kHS + k] * P[kMlpW3 + k];
-    return z;
-}
-
 // ------------------------------------------------- register-resident inference
 // Inference keeps the network in registers: each wave holds the BF16 weight
 // fragments of layers 0-2 and runs the transposed products h^T = W x^T (the
