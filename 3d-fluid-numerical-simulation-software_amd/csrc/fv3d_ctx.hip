@@ -84,6 +84,7 @@ struct fv3d_ctx {
     long nexch = 0;
     PeriodicDev *d_per = nullptr;
     int nflip = 0;               // the periodic patches if any flips its sign, else 0
+    bool bc_overlap = false;     // a patch cell is filled by a boundary condition and a transfer
     int *d_pitch_sign = nullptr;
     std::vector<PatchDev> pd_host;   // the device patch list, host copy
     double *d_mbox = nullptr;         // sweep mailboxes of all blocks
@@ -666,6 +667,25 @@ static int build_exchange(fv3d_ctx *c)
     c->nflip = 0;
     for (const PeriodicDev &p : per)
         if (p.odd) c->nflip = (int)per.size();
+    // whether a transfer ends on a cell that a boundary patch covers too: the
+    // transfer is the later one then
+    std::vector<std::vector<char>> bc(c->blocks.size() * 6);
+    for (const PatchDev &P : c->pd_host) {
+        const BlockDev &B = c->blocks[P.block].dev;
+        const int side = 2 * P.dir + P.hi;
+        std::vector<char> &m = bc[P.block * 6 + side];
+        m.resize(B.Dt[side]);
+        for (int a = 0; a < P.na; ++a)
+            for (int b = 0; b < P.nb; ++b) {
+                const size_t cell = (size_t)(P.a0 + a) * B.Db[side] + P.b0 + b;
+                if (cell < m.size()) m[cell] = 1;
+            }
+    }
+    c->bc_overlap = false;
+    for (const ExchDev &e : el) {
+        const std::vector<char> &m = bc[e.dst_block * 6 + e.side];
+        if ((size_t)e.slot < m.size() && m[e.slot]) c->bc_overlap = true;
+    }
     int rc;
     if (!c->mixes.empty()) {
         std::vector<MixDev> ml;
@@ -1622,8 +1642,9 @@ static int launch_bc(fv3d_ctx *c)
                                c->d_pitch_sign);
     };
     // one launch, unless the exchange rotates by signs that this application
-    // flips, or follows a radial-equilibrium outlet that covers a whole face
-    if (c->nflip == 0 && c->n_axial == 0) {
+    // flips, or overwrites cells that a boundary patch (or a radial-equilibrium
+    // outlet, which covers a whole face) fills too
+    if (c->nflip == 0 && c->n_axial == 0 && !c->bc_overlap) {
         boundary(bcg, exg, 0);
     } else {
         boundary(bcg, 0, c->nflip);
