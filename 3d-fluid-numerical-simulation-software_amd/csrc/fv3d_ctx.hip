@@ -84,6 +84,7 @@ struct fv3d_ctx {
     long nexch = 0;
     PeriodicDev *d_per = nullptr;
     int nflip = 0;               // the periodic patches if any flips its sign, else 0
+    bool many_exch = false;      // more than kManyExch transfers
     bool bc_overlap = false;     // a patch cell is filled by a boundary condition and a transfer
     int *d_pitch_sign = nullptr;
     std::vector<PatchDev> pd_host;   // the device patch list, host copy
@@ -577,9 +578,27 @@ static void shadow_axes(int fc, int *al, int *am)
     *am = M[fc - 1];
 }
 
+// Up to so many transfers the ghost fills and the exchange are one launch and
+// the layers of a K face neighbouring items: the time is launches and
+// latency then.  Beyond, both cost more than they give: the two kinds of scattered
+// lines compete for the caches, and the layers' writes alternate between two slabs.
+// us, one launch with the layers together / two with them apart: 8 small passages
+// (1.1e5 transfers) 37 / 52, a 2.54M-cell passage (1.9e5) 65 / 82, the 12.06M-cell stage
+// (9.9e5) 393 / 396, 16 passages (1.2e6) 455 / 453; 6 of 5M cells (1.7e6) 674 / 665,
+// 24 (1.8e6) 713 / 690, 200 small ones (2.0e6) 757 / 717, 32 (2.4e6) 985 / 916, 48 (3.5e6)
+// 1535 / 1369, 64 (4.7e6) 2222 / 1866.
+constexpr long kManyExch = 1500000;
+
 static int build_exchange(fv3d_ctx *c)
 {
     std::vector<ExchDev> el;
+    long total = 0;
+    for (const HostConn &t : c->conns) {
+        long cells = 2 * kND;   // both directions
+        for (int e = 0; e < 3; ++e) cells *= t.rng[0][2 * e + 1] - t.rng[0][2 * e] + 1;
+        total += cells;
+    }
+    c->many_exch = total > kManyExch;
     std::vector<PeriodicDev> per;
     // interiors first, then periodics (source/BoundaryCondition.cpp:46-58)
     for (int kind = 0; kind < 2; ++kind)
@@ -628,11 +647,12 @@ static int build_exchange(fv3d_ctx *c)
                 const int NA = da == 0 ? A.IM : da == 1 ? A.JM : A.KM, NB = db == 0 ? B.IM : db == 1 ? B.JM : B.KM;
                 // the layers of a K face lie side by side in memory: neighbouring
                 // items, so that a line is read once
-                const int nouter = da == 2 ? 1 : kND, ninner = kND / nouter;
+                const bool inner = da == 2 && !c->many_exch;
+                const int nouter = inner ? 1 : kND, ninner = kND / nouter;
                 for (int o1 = 1; o1 <= nouter; ++o1)
                     for (int l1 = 1; l1 <= L1; ++l1)
                         for (int m1n = 0; m1n < M1 * ninner; ++m1n) {
-                            const int m1 = m1n / ninner + 1, nd = da == 2 ? m1n % ninner + 1 : o1;
+                            const int m1 = m1n / ninner + 1, nd = inner ? m1n % ninner + 1 : o1;
                             int l2, m2;
                             switch (t.orient) {
                             case 1: l2 = l1; m2 = M1 + 1 - m1; break;
@@ -1643,8 +1663,8 @@ static int launch_bc(fv3d_ctx *c)
     };
     // one launch, unless the exchange rotates by signs that this application
     // flips, or overwrites cells that a boundary patch (or a radial-equilibrium
-    // outlet, which covers a whole face) fills too
-    if (c->nflip == 0 && c->n_axial == 0 && !c->bc_overlap) {
+    // outlet, which covers a whole face) fills too, or is a long one (kManyExch)
+    if (c->nflip == 0 && c->n_axial == 0 && !c->bc_overlap && !c->many_exch) {
         boundary(bcg, exg, 0);
     } else {
         boundary(bcg, 0, c->nflip);
