@@ -2020,9 +2020,10 @@ static int launch_update(fv3d_ctx *c)
 // hist_row null: the cursor's next row (replayed iterations)
 static int launch_finish(fv3d_ctx *c, double *hist_row)
 {
-    hipLaunchKernelGGL(k_finish, dim3((unsigned)(kFinParts * c->ninst)), dim3(256), 0, c->stream, c->d_blocks, c->d_secs,
+    const int nsw = fin_section_groups(c->ninst);
+    hipLaunchKernelGGL(k_finish, dim3((unsigned)((2 * nsw + 6) * c->ninst)), dim3(256), 0, c->stream, c->d_blocks, c->d_secs,
                        c->d_partial, c->npart, c->d_parts, c->d_sums, c->d_arrived, c->d_sc, c->ramp_sc, c->gas, hist_row,
-                       c->d_cursor, c->ninst);
+                       c->d_cursor, c->ninst, nsw);
     HIPCK(c, hipGetLastError());
     return FV3D_OK;
 }

@@ -182,14 +182,18 @@ __global__ void k_limiter_serial(const BlockDev *blocks, int nblock, Gas g, int 
 __global__ void k_sections(const BlockDev *blocks, const int2 *secs, Gas g, double *sums);
 // norms and section integrals of one level (lv) with the CFL ramp and the
 // iteration count kept in ramp (the fine level's scalars, shared by the
-// levels); kFinParts workgroups per instance w: its norm partials are
+// levels); 2 nsw + 6 workgroups per instance w: its norm partials are
 // parts[w].x .. parts[w].x + parts[w].y - 1, its scalars lv[w] and ramp[w], its
 // history row hist_row + 7 w, or the cursor's next one.  sums: the section
 // partials of every instance, then six norms each; arrived: zero between launches
-constexpr int kFinParts = 2 * kSecParts + 6;
+// nsw: workgroups per section.  A workgroup that counts itself in writes its XCD's L2
+// back first, all in turn: with one per section part, 64 passages of a batch took
+// 181 us (156 as the two launches this replaced).  Eight per section: 159 us, 32 passages
+// 100 -> 95, 16 60 -> 57; four: 153, 99 and 77; eight passages 18.6 either way.
+inline int fin_section_groups(int ninst) { return ninst >= 48 ? 4 : ninst > 8 ? 8 : kSecParts; }
 __global__ void k_finish(const BlockDev *blocks, const int2 *secs, const double *partial, int npart, const int2 *parts,
                          double *sums, int *arrived, ScalarsDev *lv, ScalarsDev *ramp, Gas g, double *hist_row,
-                         double *const *cursor, int ninst);
+                         double *const *cursor, int ninst, int nsw);
 __global__ void k_hist_begin(double **cursor, double *hist, ScalarsDev *ramp, int ninst);
 // two-grid cycle (CSolver::Prolong / Interpolate, CMesh::CornerTreatment,
 // ComputeForceFunction / AddForceFunction)

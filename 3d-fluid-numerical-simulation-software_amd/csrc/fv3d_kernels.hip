@@ -1627,8 +1627,8 @@ __global__ void __launch_bounds__(256) k_sections(const BlockDev *__restrict__ b
     section_part(blocks, secs, g, sums, blockIdx.x / kSecParts, blockIdx.x % kSecParts, red);
 }
 
-// The end of an iteration, kFinParts workgroups per instance: the section
-// integrals' parts, and one workgroup per component of the residual norm (the
+// The end of an iteration, 2 nsw + 6 workgroups per instance: nsw per section for
+// the integrals' parts, and one per component of the residual norm (the
 // fixed-order sum of the update's per-workgroup partials); the instance's last
 // workgroup to finish then forms the norms, the performance parameters
 // (source/Ouput.cpp:97-107,282-300), the CFL ramp for the next iteration
@@ -1636,18 +1636,18 @@ __global__ void __launch_bounds__(256) k_sections(const BlockDev *__restrict__ b
 // cursor's next one.  As two launches, the second with one workgroup per
 // instance, this took 53 us on a 2.54M-cell passage and 12 on the smallest
 // grids, and a copy of the row 4.5 more; now 20 and 8.  A workgroup without
-// cells leaves at once: with all kFinParts counting themselves in, eight
-// passages of one batch took 30 us, now 17.
+// cells leaves at once: with all 70 counting themselves in, eight passages of one
+// batch took 30 us, now 17.
 __global__ void __launch_bounds__(256) k_finish(const BlockDev *__restrict__ blocks, const int2 *__restrict__ secs,
                                                 const double *__restrict__ partial, int npart,
                                                 const int2 *__restrict__ parts, double *__restrict__ secsum,
                                                 int *__restrict__ arrived, ScalarsDev *lv, ScalarsDev *ramp, Gas g,
                                                 double *__restrict__ hist_row, double *const *__restrict__ cursor,
-                                                int ninst)
+                                                int ninst, int nsw)
 {
     __shared__ double red[3][256];
     __shared__ int s_last;
-    const int inst = blockIdx.x / kFinParts, part = blockIdx.x % kFinParts;
+    const int inst = blockIdx.x / (2 * nsw + 6), part = blockIdx.x % (2 * nsw + 6);
     const int t = threadIdx.x;
     ScalarsDev *sc = lv + inst;
     ramp += inst;
@@ -1661,25 +1661,26 @@ __global__ void __launch_bounds__(256) k_finish(const BlockDev *__restrict__ blo
         return min((B.ni * B.nj + 255) / 256, kSecParts);
     };
     const int np0 = nonempty(0), np1 = nonempty(1);
-    if (part < 2 * kSecParts ? part % kSecParts >= (part < kSecParts ? np0 : np1) : part - 2 * kSecParts >= nc) return;
-    if (part < 2 * kSecParts) {
-        section_part(blocks, secs, g, secsum, inst * 2 + part / kSecParts, part % kSecParts, red);
+    const int sec = part / nsw, np = sec == 0 ? np0 : np1;
+    if (sec < 2 ? part % nsw >= np : part - 2 * nsw >= nc) return;
+    if (sec < 2) {
+        for (int p = part % nsw; p < np; p += nsw) section_part(blocks, secs, g, secsum, inst * 2 + sec, p, red);
     } else {
-        const int c = part - 2 * kSecParts;
+        const int c = part - 2 * nsw;
         double r = 0.0;
         // each thread adds partials t, t + 256, ... in that order; sixteen
         // loads are in flight before the first is added
         const double *src = partial + (long)c * npart + parts[inst].x;
-        const int np = parts[inst].y;
+        const int n = parts[inst].y;
         int p = t;
-        for (; p + 15 * 256 < np; p += 16 * 256) {
+        for (; p + 15 * 256 < n; p += 16 * 256) {
             double v[16];
 #pragma unroll
             for (int u = 0; u < 16; ++u) v[u] = src[p + u * 256];
 #pragma unroll
             for (int u = 0; u < 16; ++u) r += v[u];
         }
-        for (; p < np; p += 256) r += src[p];
+        for (; p < n; p += 256) r += src[p];
         red[0][t] = r;
         __syncthreads();
         for (int w = 128; w > 0; w >>= 1) {
@@ -1691,7 +1692,7 @@ __global__ void __launch_bounds__(256) k_finish(const BlockDev *__restrict__ blo
     // what this workgroup wrote (thread 0) is visible before it counts itself in
     if (t == 0) {
         __threadfence();
-        s_last = atomicAdd(arrived + inst, 1) == np0 + np1 + nc - 1;
+        s_last = atomicAdd(arrived + inst, 1) == min(np0, nsw) + min(np1, nsw) + nc - 1;
         if (s_last) __threadfence();
     }
     __syncthreads();
@@ -1712,8 +1713,8 @@ __global__ void __launch_bounds__(256) k_finish(const BlockDev *__restrict__ blo
     __syncthreads();
     if (t < 6) {
         double s = 0.0;
-        const int np = t < 3 ? np0 : np1;
-        for (int p = 0; p < np; ++p) s += red[0][((t / 3) * kSecParts + p) * 3 + t % 3];
+        const int m = t < 3 ? np0 : np1;
+        for (int p = 0; p < m; ++p) s += red[0][((t / 3) * kSecParts + p) * 3 + t % 3];
         red[1][t] = s;
     }
     __syncthreads();
