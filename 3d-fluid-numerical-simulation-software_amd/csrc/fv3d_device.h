@@ -221,13 +221,21 @@ struct Gas {
 // on it, the quotient, its remainder and the corrected quotient, about eleven
 // instructions of which six depend on the denominator only.  Here those six are
 // done once: of(a) is the remaining product, remainder, correction and
-// special-case fix-up (zeros, infinities, NaN).  The operations and their order
-// are the compiler's, so of(a) has the bits of a / b; only its rescaling is left
-// out, which acts when b or a / b is subnormal or their exponents are some 2^768
-// apart (1e+/-231 in non-dimensional flow quantities of order one).  A face of the
-// Roe flux has 48 divisions by 21 different denominators; sharing them took
-// k_convective from 467 to 412 us on a 2.54M-cell passage, 188 to 168 us on a
-// 1.05M-cell channel.
+// special-case fix-up (operands that are zero, infinite or NaN).  The operations
+// and their order are the compiler's; only its rescaling is left out.  So of(a)
+// has the bits of a / b for normal b below 2^1021 and a of 2^-969 or more, while a / b is
+// normal too.  Outside that: a smaller a loses bits of the remainder (at most the
+// last one of the quotient is off), a subnormal b or one above 2^1021 those of the
+// reciprocal, and a quotient that overflows, or any quotient by a b below 2^-1024,
+// is NaN where a / b is infinite or large.  The denominators
+// here are densities, areas, sound speeds and sums with a floor of 1e-6 or 1e-8, in
+// non-dimensional units: a quotient overflows only where the squares that are formed
+// of the same values have done so.  Clamping the quotient before its
+// remainder is taken would give the infinity: one instruction more per division, 1 %
+// of k_convective and 1 to 2.5 % of the FP64 sweeps (218 -> 223 us on 293k cells).
+// A face of the Roe flux has 48 divisions by 21 different denominators; sharing
+// them took k_convective from 467 to 412 us on a 2.54M-cell passage, 188 to 168 us on
+// a 1.05M-cell channel.
 struct DivBy {
     double b, r;
     __device__ explicit DivBy(double den) : b(den)
