@@ -133,7 +133,9 @@ struct fv3d_ctx {
     ViscDebug vdbg = {{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}, nullptr};
     int store_faces = 0;
     double total_vol = 0.0;
-    // fv3d_field_download's staging: the rows of a field, at most kFetchBytes at a time
+    // fv3d_field_download's staging: the rows of a field, at most kFetchBytes at a
+    // time; the finest level's, whose blocks are the largest (the calls of a context
+    // come one at a time, whatever the level they read)
     double *d_fetch = nullptr;
     long fetch_words = 0;
     // persistent wavefront sweep: tile lists (forward, backward) and the
@@ -903,7 +905,7 @@ int fv3d_ctx_destroy(fv3d_ctx *c)
     for (int q = 0; q < kNumStream; ++q)
         if (c->d_stiles[q]) (void)hipFree(c->d_stiles[q]);
     void *ps[] = {c->d_blocks, c->d_patches, c->d_pstart_bc, c->d_cstart, c->d_pstart_plane, c->d_secs,
-                  c->d_partial, c->d_sums, c->d_bad, c->d_flags, c->d_sc, c->d_hist, c->parent ? nullptr : c->d_cursor, c->d_arrived, c->d_fetch, c->d_kba[0], c->d_kba[1], c->d_kba_sync, c->d_faces[0], c->d_faces[1], c->d_faces[2]};
+                  c->d_partial, c->d_sums, c->d_bad, c->d_flags, c->d_sc, c->d_hist, c->parent ? nullptr : c->d_cursor, c->parent ? nullptr : c->d_fetch, c->d_arrived, c->d_kba[0], c->d_kba[1], c->d_kba_sync, c->d_faces[0], c->d_faces[1], c->d_faces[2]};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     if (c->stream) {
@@ -1431,12 +1433,17 @@ int fv3d_setup(fv3d_ctx *c)
     if (c->cfg.turbulence == 200 && (rc = setup_sa(c))) return rc;
     if ((rc = dalloc(c, &c->d_sums, (2 * 3 * kSecParts + 6) * (size_t)c->ninst))) return rc;
     if ((rc = dalloc(c, &c->d_arrived, c->ninst))) return rc;
-    long box = 0;
-    for (const HostBlock &b : c->blocks) box = std::max(box, b.dev.box);
-    c->fetch_words = std::min(kFetchBytes / (long)sizeof(double), 12 * box);
-    if ((rc = dalloc(c, &c->d_fetch, c->fetch_words))) return rc;
-    if (c->parent) c->d_cursor = c->parent->d_cursor;
-    else if ((rc = dalloc(c, &c->d_cursor, 1))) return rc;
+    if (c->parent) {
+        c->d_cursor = c->parent->d_cursor;
+        c->d_fetch = c->parent->d_fetch;
+        c->fetch_words = c->parent->fetch_words;
+    } else {
+        if ((rc = dalloc(c, &c->d_cursor, 1))) return rc;
+        long box = 0;
+        for (const HostBlock &b : c->blocks) box = std::max(box, b.dev.box);
+        c->fetch_words = std::min(kFetchBytes / (long)sizeof(double), 12 * box);
+        if ((rc = dalloc(c, &c->d_fetch, c->fetch_words))) return rc;
+    }
     // device scalars of each instance
     std::vector<ScalarsDev> scs(c->ninst);
     for (int w = 0; w < c->ninst; ++w) {
