@@ -203,12 +203,16 @@ __device__ static void exchange_item(const BlockDev *__restrict__ blocks, const 
 
 // Boundary conditions: nbcg workgroups fill the ghost cells of inlets, outlets
 // and walls, one updates the periodic signs where nflip patches need it, the
-// others run the exchange.  The ghost fills and the exchange read interior cells
-// only and write ghost cells of their own patches, so they run side by side,
-// unless the exchange waits for new signs.  Both are look-ups and one round of
-// loads, bound by latency (on large K faces by the exchange's scattered lines):
-// as two launches 25 us on a rotor-stator stage, 42 us on a batch of eight
-// passages, 69 us on 2.54M cells; as one 18, 33 and 58 us.
+// others run the exchange.  Nothing here orders these against each other.  All three
+// may come in one launch only if no transfer ends on a cell that a boundary
+// patch fills too (or a radial-equilibrium outlet, which comes between the two)
+// and no sign flips: launch_bc sees to that (bc_overlap, n_axial, nflip) and
+// otherwise launches the fills with the signs first, then the exchange.  Both
+// read interior cells only.  They are look-ups and one round of loads, bound by
+// latency (on large K faces by the exchange's scattered lines): as two launches
+// 25 us on a rotor-stator stage, 42 us on a batch of eight passages, 69 us on
+// 2.54M cells; as one 18, 33 and 58 us.  A long exchange goes by itself again
+// (kManyExch).
 __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(8)))
 k_boundary(const BlockDev *__restrict__ blocks, const PatchDev *__restrict__ patches, int npatch,
            const long *__restrict__ pstart, int nbcg, Gas g, const ScalarsDev *__restrict__ sc,
@@ -502,7 +506,11 @@ k_convective(const BlockDev *__restrict__ blocks, const int4 *__restrict__ tiles
         // gamma anew each time round: what depends on it alone is a few
         // instructions, but kept across the loop it takes the registers that the
         // face code then spills (1.03 GB moved instead of 0.78 on 2.54M cells,
-        // 431 -> 393 us; 1.05M cells 159 -> 153)
+        // 431 -> 393 us; 1.05M cells 159 -> 153).  On conservative variables it
+        // gains 8 % with the Roe flux on 1.05M cells (166 -> 154) and 2 % on
+        // 292k (64.5 -> 63.4), but costs 2 % with Steger-Warming there (61.3 -> 62.4):
+        // the flux is a run-time choice of one kernel, so both get it.  The
+        // characteristic form takes 156 registers instead of 168, the same time.
         Gas gl = g;
         asm volatile("" : "+s"(gl.gamma));
         face_flux<MODE>(B, gl, d, i, j, k, out);

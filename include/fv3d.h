@@ -4,8 +4,9 @@
  * Every entry point returns 0 on success and a negative fv3d_status code on
  * failure; fv3d_last_error() then holds a message.  The library never exits
  * the process.  Calls on one context are stream-ordered on that context's HIP
- * stream; only the functions that return host data synchronise.  One context
- * per host thread.  Host pointers are borrowed for the duration of the call.
+ * stream; only the functions that return host data synchronise, and fv3d_lusgs,
+ * which waits to report a sweep whose bounded wait ran out.  One context per host
+ * thread.  Host pointers are borrowed for the duration of the call.
  *
  * Reference interfaces replaced (paths relative to the reference tree):
  *   the CMesh / CSpaceDiscr / CTimeDiscr / CSolver method surface of
@@ -263,7 +264,9 @@ int fv3d_perf(fv3d_ctx *ctx, double *out5);
  * Synchronises once at the end. */
 int fv3d_iterate(fv3d_ctx *ctx, int n, double *hist);
 
-/* Same as fv3d_iterate, but replays one captured HIP graph per iteration. */
+/* Same as fv3d_iterate, but replays captured HIP graphs, each captured on first
+ * use: four iterations per launch while that many are left, then single ones
+ * (with two levels, single ones up to Coarse_iter, which itself runs eagerly). */
 int fv3d_iterate_graph(fv3d_ctx *ctx, int n, double *hist);
 
 int fv3d_sync(fv3d_ctx *ctx);
