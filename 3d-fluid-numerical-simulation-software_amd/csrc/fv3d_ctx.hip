@@ -585,10 +585,9 @@ static void shadow_axes(int fc, int *al, int *am)
 // latency then.  Beyond, both cost more than they give: the two kinds of scattered
 // lines compete for the caches, and the layers' writes alternate between two slabs.
 // us, one launch with the layers together / two with them apart: 8 small passages
-// (1.1e5 transfers) 37 / 52, a 2.54M-cell passage (1.9e5) 65 / 82, the 12.06M-cell stage
-// (9.9e5) 393 / 396, 16 passages (1.2e6) 455 / 453; 6 of 5M cells (1.7e6) 674 / 665,
-// 24 (1.8e6) 713 / 690, 200 small ones (2.0e6) 757 / 717, 32 (2.4e6) 985 / 916, 48 (3.5e6)
-// 1535 / 1369, 64 (4.7e6) 2222 / 1866.
+// (1.1e5 transfers) 39 / 51, a 2.54M-cell passage (1.9e5) 63 / 83, 16 passages (1.2e6)
+// 447 / 453; 6 of 5M cells (1.7e6) 667 / 666, 24 (1.8e6) 699 / 686, 200 small ones (2.0e6)
+// 740 / 704, 32 (2.4e6) 978 / 906, 64 (4.7e6) 2245 / 1830.
 constexpr long kManyExch = 1500000;
 
 static int build_exchange(fv3d_ctx *c)

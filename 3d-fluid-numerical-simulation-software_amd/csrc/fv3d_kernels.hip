@@ -212,8 +212,10 @@ __device__ static void exchange_item(const BlockDev *__restrict__ blocks, const 
 // latency (on large K faces by the exchange's scattered lines): as two launches
 // 25 us on a rotor-stator stage, 42 us on a batch of eight passages, 69 us on
 // 2.54M cells; as one 18, 33 and 58 us.  A long exchange goes by itself again
-// (kManyExch).
-__global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(8)))
+// (kManyExch).  84 registers, five waves per SIMD: held to 64 for eight waves, the
+// fills of a 16x512x512 channel took 62 us instead of 58, of 192x192x512 71 instead
+// of 67, and the passages' exchanges 2 % more.
+__global__ void __launch_bounds__(256)
 k_boundary(const BlockDev *__restrict__ blocks, const PatchDev *__restrict__ patches, int npatch,
            const long *__restrict__ pstart, int nbcg, Gas g, const ScalarsDev *__restrict__ sc,
            const ExchDev *__restrict__ el, long nexch, PeriodicDev *per, int nflip, int *pitch_sign)
