@@ -195,6 +195,25 @@ struct fv3d_ctx {
 };
 
 constexpr long kFetchBytes = 16L << 20;
+// A field of at most kFetchBox bytes per component and kFetchSmall in all comes as
+// one copy of its cell box, interleaved on the host: a kernel and its wait cost
+// more than that loop.  vol of 8^3 / 20^3 / 24^3 cells 16 / 15 / 18 us this way, 25 / 26 / 28
+// by k_field_rows; cv 27 / 35 / 54 and 41 / 41 / 53.
+constexpr long kFetchBox = 160L << 10, kFetchSmall = 512L << 10;
+
+// Cells lo .. along each direction (n1 x n2 x n3) of a box array on the host, the
+// components of a cell together; N: their number, or 0 if it is none of the usual.
+template <int N>
+static void interleave(const double *h, const BlockDev &B, int comps, int lo, int n1, int n2, int n3, double *o)
+{
+    const int C = N ? N : comps;
+    for (int i = lo; i < lo + n1; ++i)
+        for (int j = lo; j < lo + n2; ++j) {
+            const double *p = h + cidx(B, i, j, lo);
+            for (int k = 0; k < n3; ++k)
+                for (int q = 0; q < C; ++q) *o++ = p[q * B.box + k];
+        }
+}
 
 static int fail(fv3d_ctx *c, int code, const char *fmt, ...)
 {
@@ -2987,6 +3006,15 @@ long fv3d_field_download(fv3d_ctx *c, int block, const char *name, double *out)
     // interleaved on the device and copied straight to the caller's buffer
     auto read = [&](const double *src, int C, int lo, int n1, int n2, int n3) -> long {
         const long cells = (long)n1 * n2 * n3, chunk = c->fetch_words / C;
+        const long bytes = B.box * (long)sizeof(double);
+        if (bytes <= kFetchBox && C * bytes <= kFetchSmall) {
+            std::vector<double> h(C * B.box);
+            HIPCK(c, hipStreamSynchronize(c->stream));
+            HIPCK(c, hipMemcpy(h.data(), src, C * bytes, hipMemcpyDeviceToHost));
+            auto *f = C == 1 ? interleave<1> : C == 5 ? interleave<5> : C == 6 ? interleave<6> : interleave<0>;
+            f(h.data(), B, C, lo, n1, n2, n3, out);
+            return cells * C;
+        }
         for (long t0 = 0; t0 < cells; t0 += chunk) {
             const long n = std::min(chunk, cells - t0);
             hipLaunchKernelGGL(k_field_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, src, B.box, C,
