@@ -232,7 +232,7 @@ struct Gas {
 // non-dimensional units: a quotient overflows only where the squares that are formed
 // of the same values have done so.  Clamping the quotient before its
 // remainder is taken would give the infinity: one instruction more per division, 1 %
-// of k_convective and 1 to 2.5 % of the FP64 sweeps (218 -> 223 us on 293k cells).
+// of k_convective and 1 to 2.5 % of the FP64 sweeps (218 -> 223 us on 292k cells).
 // A face of the Roe flux has 48 divisions by 21 different denominators; sharing
 // them took k_convective from 467 to 412 us on a 2.54M-cell passage, 188 to 168 us on
 // a 1.05M-cell channel.
